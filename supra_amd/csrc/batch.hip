@@ -51,7 +51,9 @@ using namespace supra_amd;
 
 namespace {
 
-constexpr uint32_t kMaxQueues = 9;         // DAS + MV x {L<=32, L<=64} x {int16, float} x {means}
+// DAS + refined MV x {L<=32, L<=64} x {int16, float} x {means} + well-loaded
+// MV x {L<=16, L<=32, L<=64} x {int16, float}
+constexpr uint32_t kMaxQueues = 15;
 constexpr uint32_t kMaxFramesPerQueue = 256;
 constexpr uint32_t kMaxItemsPerFrame = 1u << 24;
 
@@ -74,9 +76,10 @@ struct FrameDesc {
 
 struct Queue {
     bool mv = false;
-    uint32_t lmax = 0;         // MV: 32 or 64
+    uint32_t lmax = 0;         // MV: 16 (block), 32 or 64
     int32_t rf_dtype = 0;      // MV
-    int32_t means = 0;         // MV
+    int32_t means = 0;         // MV (not block)
+    int32_t block = 0;         // MV: well-loaded systems (mv_block.hip)
     void* frames = nullptr;    // DasBatchFrame[] or MvBatchFrame[] (device)
     uint32_t* items = nullptr;
     uint32_t n_items = 0, n_frames = 0;
@@ -275,8 +278,9 @@ int build_mv_queue(supra_batch* b, uint32_t qi, size_t budget) {
         size_t frame_lds = 0;
         int st = mv_prepare(fr.a, it.ctx->n_rx, it.num_channels, it.ctx->n_depths, it.sub_array_size,
                             it.temporal_smoothing, it.sub_array_scaling_power, it.compute_means, it.loading_factor,
-                            budget, &frame_lds);
+                            false, budget, &frame_lds);
         if (st != SUPRA_OK) return st;
+        if (fr.a.block != q.block) return fail(SUPRA_ERR_TOO_LARGE, "batch: item %u does not fit the LDS budget", f);
         lds = std::max(lds, frame_lds);
         fr.rf_dtype = it.rf_dtype;
         fr.n_items = fr.a.n_rx * fr.a.n_tiles;
@@ -341,6 +345,7 @@ hipError_t launch_queue(const supra_batch* b, uint32_t qi, hipStream_t s) {
     a.items = q.items;
     a.n_items = q.n_items;
     a.sync = make_sync(b, qi);
+    if (q.block) return launch_mv_block_batch(a, q.lmax, q.rf_dtype, wg, q.lds, s);
     return launch_mv_batch(a, q.lmax, q.rf_dtype, q.means, wg, q.lds, s);
 }
 
@@ -560,13 +565,15 @@ extern "C" int supra_batch_create(const supra_batch_item* items, uint32_t num_it
         if (items[i].mode == SUPRA_BATCH_MV) {
             const uint32_t L = items[i].sub_array_size ? items[i].sub_array_size : items[i].num_channels / 2;
             key.mv = true;
-            key.lmax = L <= 32 ? 32 : 64;
             key.rf_dtype = items[i].rf_dtype;
-            key.means = items[i].compute_means ? 1 : 0;
+            key.block = mv_well_loaded(L, items[i].loading_factor) ? 1 : 0;
+            key.lmax = key.block ? mv_block_lmax(L) : (L <= 32 ? 32 : 64);
+            key.means = !key.block && items[i].compute_means ? 1 : 0;
         }
         uint32_t qi = 0;
         while (qi < b->queues.size() && !(b->queues[qi].mv == key.mv && b->queues[qi].lmax == key.lmax &&
-                                          b->queues[qi].rf_dtype == key.rf_dtype && b->queues[qi].means == key.means))
+                                          b->queues[qi].rf_dtype == key.rf_dtype && b->queues[qi].means == key.means &&
+                                          b->queues[qi].block == key.block))
             qi++;
         if (qi == b->queues.size()) {
             if (qi == kMaxQueues) return fail(SUPRA_ERR_TOO_LARGE, "batch: too many kernel classes");

@@ -1,0 +1,599 @@
+// Minimum variance for well-loaded systems: the per-sample covariances are
+// accumulated on the FP64 matrix cores and every system is factorised by 16
+// lanes.
+//
+// Same per-sample mathematics as mv_kernels.hip (which keeps the forms this
+// one does not have: FP64 refinement of weakly loaded systems and conjugate
+// gradients); the references are the same: RxBeamformerMV.cu:44-113 apertures
+// and sub-arrays, :115-195 covariance, :197-228 temporal sum, :239-305
+// loading, :558-586 solve, :307-378 output.
+//
+// One workgroup takes nb consecutive output depths of one scanline:
+//
+//   1. stage x[channel][tau] of the nb depths and their +-T halo in LDS, find
+//      the apertures (mv_stage.hpp);
+//   2. the window sums R~(t) = sum_{|tau-t| <= T} sum_k x_k x_k^T of the nb
+//      outputs, as 16 x 16 blocks of the lower triangle with
+//      v_mfma_f64_16x16x4 (products of floats are exact in FP64).  The
+//      outputs go in sub-blocks of at most 2T + 1: their windows share a core
+//      of samples, so the accumulator is filled with the core, then extended
+//      downwards (one sample per output, stored as it grows) and a second one
+//      upwards (added to what was stored).  No sum is ever subtracted from,
+//      so a weak window next to a strong echo keeps its precision, and about
+//      2 evaluations per output replace the 2T + 1 additions of stored
+//      covariances.  Along a block diagonal, block (r+1, c+1) differs from
+//      (r, c) by 16 entering and 16 leaving products, so with LMAX = 64 the first
+//      block column (and one more block, to even out the waves) is summed in
+//      full and the rest by differences (125 instead of 170 matrix
+//      instructions per sample with 65 sub-arrays);
+//   3. sixteen lanes per system, row 16 r + q in slot r of lane q: diagonal
+//      loading, then a right-looking Cholesky factorisation whose column is
+//      broadcast inside the FMAs (DPP row_newbcast), FP64 pivots and
+//      diagonal, with the two right-hand sides 1 and the sub-array sums xs as
+//      extra columns.  With z = G^-1 1 and u = G^-1 xs the output is
+//      xs^T R~^-1 1 / 1^T R~^-1 1 = u.z / z.z: no backward substitution and
+//      no factor kept.
+//
+// Bound by vector instructions (56 % busy) and the matrix cores (24 % busy) at
+// L = 32; by the latency of one wave per SIMD at L = 64, whose matrices fill
+// the LDS.  128 x 2080 samples, L = 32, T = 5: 0.80 ms against 2.02 ms of
+// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 2.93 ms against
+// 9.54 ms; relative error of the image against FP64 1.1e-6 against 1.6e-6.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
+#include <cstdint>
+
+#include "bf_internal.hpp"
+#include "das_device.hpp"
+#include "mv_launch.hpp"
+#include "mv_stage.hpp"
+
+namespace supra_amd {
+namespace {
+
+typedef double double4v __attribute__((ext_vector_type(4)));
+
+// Waves per workgroup: the matrix blocks are dealt to the waves (3 blocks for
+// 32 rows, 10 for 64), for 16 rows the sub-blocks of outputs are.
+template <int LMAX> struct Cfg {
+    static constexpr int kBlocks = LMAX / 16;
+    static constexpr int kWaves = LMAX == 32 ? 3 : 4;
+    static constexpr int kThreads = 64 * kWaves;
+    // floats of one stored lower triangle: full 16 x 16 blocks below the
+    // diagonal, 160 floats per diagonal block (its 4-column chunks without
+    // the rows above them)
+    static constexpr int kMatrix = kBlocks * 160 + kBlocks * (kBlocks - 1) / 2 * 256;
+};
+
+// First float of block (r, c), c <= r.  Blocks are stored by chunks of 4
+// columns, [chunk][row][4], so that 16 rows of a chunk are 256 contiguous
+// bytes for the solver's 16-byte reads.
+__device__ constexpr int block_at(int r, int c) { return r * 160 + r * (r - 1) / 2 * 256 + c * 256; }
+// First float of a diagonal block's chunk (rows 4 chunk .. 15).
+__device__ constexpr int diag_chunk(int chunk) { return chunk == 0 ? 0 : (chunk == 1 ? 64 : (chunk == 2 ? 112 : 144)); }
+
+struct Gram {
+    const float* xs;
+    const SampleMeta* meta;
+    const float* mean;     // [h][16 kBlocks], nullptr without mean removal
+    float* mats;
+    int rs, mean_stride, matrix;
+    int T, n_d, h_lo;
+};
+
+// The block diagonal chain (R0, C0), (R0+1, C0+1), ... of LEN blocks.
+template <int R0, int C0, int LEN>
+struct Chain {
+    double4v acc[LEN];     // block (R0, C0), then the differences to the previous block
+    __device__ inline void clear() {
+#pragma unroll
+        for (int d = 0; d < LEN; d++) acc[d] = double4v{0.0, 0.0, 0.0, 0.0};
+    }
+    // acc += covariance of sample tau.  Matrix-core operands: lane = (row or
+    // column i = lane % 16, term k = lane / 16); D[j][i] holds row i of the
+    // block in lane % 16 and column j = lane / 16 + 4 v in register v.
+    __device__ inline void add(const Gram& g, int tau) {
+        const int h = tau - g.h_lo;
+        const SampleMeta m = g.meta[h];
+        if (__builtin_amdgcn_readfirstlane(m.bad)) return;
+        const int kact = __builtin_amdgcn_readfirstlane(m.kact);
+        const int lane = static_cast<int>(threadIdx.x % 64), i = lane % 16, kq = lane / 16;
+        const float* row = g.xs + h * g.rs + __builtin_amdgcn_readfirstlane(m.first) + i + kq;
+        const int steps = (kact + 3) / 4;
+#pragma unroll 4
+        for (int s = 0; s < steps; s++) {
+            const float vc = row[4 * s + 16 * C0];
+            const float vr = R0 == C0 ? vc : row[4 * s + 16 * R0];
+            const float va = 4 * s + kq < kact ? vc : 0.0f;
+            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(va), static_cast<double>(vr), acc[0], 0, 0, 0);
+        }
+        if constexpr (LEN > 1) {
+            // R[16+i][16+j] - R[i][j] = sum over the entering minus the leaving terms
+            const int n = min(kact, 16), p0 = max(kact, 16);
+#pragma unroll 4
+            for (int s = 0; s < (n + 3) / 4; s++) {
+                const bool in = 4 * s + kq < n;
+                const float* lo = row + 4 * s;
+                const float* hi = lo + p0;
+#pragma unroll
+                for (int d = 1; d < LEN; d++) {
+                    const float hc = hi[16 * (C0 + d - 1)], hr = R0 == C0 ? hc : hi[16 * (R0 + d - 1)];
+                    const float lc = lo[16 * (C0 + d - 1)], lr = R0 == C0 ? lc : lo[16 * (R0 + d - 1)];
+                    acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(in ? hc : 0.0f),
+                                                                  static_cast<double>(hr), acc[d], 0, 0, 0);
+                    acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(-static_cast<double>(in ? lc : 0.0f),
+                                                                  static_cast<double>(lr), acc[d], 0, 0, 0);
+                }
+            }
+        }
+        if (g.mean) {   // - K m m^T
+            const float* mu = g.mean + h * g.mean_stride + i;
+            const double k = static_cast<double>(kact);
+            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(kq == 0 ? -k * static_cast<double>(mu[16 * C0]) : 0.0,
+                                                          static_cast<double>(mu[16 * R0]), acc[0], 0, 0, 0);
+#pragma unroll
+            for (int d = 1; d < LEN; d++) {
+                const int e = kq == 0 ? d : d - 1;
+                const double f = kq == 0 ? -k : (kq == 1 ? k : 0.0);
+                acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(f * static_cast<double>(mu[16 * (C0 + e)]),
+                                                              static_cast<double>(mu[16 * (R0 + e)]), acc[d], 0, 0, 0);
+            }
+        }
+    }
+    // Stores (ADD: adds) the blocks to output matrix o.
+    template <bool ADD>
+    __device__ inline void store(const Gram& g, int o) const {
+        const int lane = static_cast<int>(threadIdx.x % 64), i = lane % 16, e = lane / 16;
+        double4v sum = acc[0];
+#pragma unroll
+        for (int d = 0; d < LEN; d++) {
+            if (d > 0) sum += acc[d];
+            float* blk = g.mats + o * g.matrix + block_at(R0 + d, C0 + d);
+#pragma unroll
+            for (int v = 0; v < 4; v++) {
+                float* p = R0 == C0 ? blk + diag_chunk(v) + (i - 4 * v) * 4 + e : blk + v * 64 + i * 4 + e;
+                if (R0 != C0 || i >= 4 * v) *p = ADD ? static_cast<float>(static_cast<double>(*p) + sum[v]) : static_cast<float>(sum[v]);
+            }
+        }
+    }
+};
+
+// Window sums of the outputs [ta, ta + n) into matrices o, o + 1, ...; n <= 2T + 1.
+template <int R0, int C0, int LEN>
+__device__ inline void window_sums(const Gram& g, int ta, int n, int o) {
+    Chain<R0, C0, LEN> c;
+    c.clear();
+    for (int tau = max(0, ta + n - 1 - g.T); tau <= min(g.n_d - 1, ta + g.T); tau++) c.add(g, tau);
+    c.template store<false>(g, o + n - 1);
+    for (int j = n - 2; j >= 0; j--) {
+        if (ta + j - g.T >= 0) c.add(g, ta + j - g.T);
+        c.template store<false>(g, o + j);
+    }
+    c.clear();
+    for (int j = 1; j < n; j++) {
+        if (ta + j + g.T < g.n_d) c.add(g, ta + j + g.T);   // else the window ends with the last sample
+        c.template store<true>(g, o + j);
+    }
+}
+
+template <int LMAX>
+__device__ inline void all_window_sums(const Gram& g, int t0, int n_out, int sub, int wave) {
+    if constexpr (LMAX == 16) {
+        for (int b = wave * sub; b < n_out; b += Cfg<LMAX>::kWaves * sub)
+            window_sums<0, 0, 1>(g, t0 + b, min(sub, n_out - b), b);
+    } else {
+        for (int b = 0; b < n_out; b += sub) {
+            const int ta = t0 + b, n = min(sub, n_out - b);
+            if constexpr (LMAX == 32) {
+                if (wave == 0) window_sums<0, 0, 1>(g, ta, n, b);
+                else if (wave == 1) window_sums<1, 0, 1>(g, ta, n, b);
+                else window_sums<1, 1, 1>(g, ta, n, b);
+            } else {
+                if (wave == 0) {
+                    window_sums<0, 0, 3>(g, ta, n, b);
+                } else if (wave == 1) {
+                    window_sums<1, 0, 3>(g, ta, n, b);
+                } else if (wave == 2) {
+                    window_sums<2, 0, 2>(g, ta, n, b);
+                } else {
+                    window_sums<3, 0, 1>(g, ta, n, b);
+                    window_sums<3, 3, 1>(g, ta, n, b);
+                }
+            }
+        }
+    }
+}
+
+// ---- the solver: 16 lanes per system -------------------------------------------
+
+// a[k] += (lane k's l of this row of 16 lanes) * nl for k = START .. 15, one
+// v_fmac_f32_dpp row_newbcast each.  The leading s_nop covers the two wait
+// states between a VALU write of l and its DPP read.
+#define SUPRA_FM(K) "v_fmac_f32_dpp %" #K ", %16, %17 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"
+#define SUPRA_FM_15 SUPRA_FM(15)
+#define SUPRA_FM_14 SUPRA_FM(14) SUPRA_FM_15
+#define SUPRA_FM_13 SUPRA_FM(13) SUPRA_FM_14
+#define SUPRA_FM_12 SUPRA_FM(12) SUPRA_FM_13
+#define SUPRA_FM_11 SUPRA_FM(11) SUPRA_FM_12
+#define SUPRA_FM_10 SUPRA_FM(10) SUPRA_FM_11
+#define SUPRA_FM_9 SUPRA_FM(9) SUPRA_FM_10
+#define SUPRA_FM_8 SUPRA_FM(8) SUPRA_FM_9
+#define SUPRA_FM_7 SUPRA_FM(7) SUPRA_FM_8
+#define SUPRA_FM_6 SUPRA_FM(6) SUPRA_FM_7
+#define SUPRA_FM_5 SUPRA_FM(5) SUPRA_FM_6
+#define SUPRA_FM_4 SUPRA_FM(4) SUPRA_FM_5
+#define SUPRA_FM_3 SUPRA_FM(3) SUPRA_FM_4
+#define SUPRA_FM_2 SUPRA_FM(2) SUPRA_FM_3
+#define SUPRA_FM_1 SUPRA_FM(1) SUPRA_FM_2
+#define SUPRA_FM_0 SUPRA_FM(0) SUPRA_FM_1
+
+template <int START>
+__device__ __attribute__((always_inline)) inline void fmac16(float* a, float l, float nl) {
+#define SUPRA_FM_CASE(S)                                                                                               \
+    if constexpr (START == S)                                                                                         \
+        asm("s_nop 1\n\t" SUPRA_FM_##S                                                                                \
+            : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),         \
+              "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15])    \
+            : "v"(l), "v"(nl))
+    SUPRA_FM_CASE(0);
+    SUPRA_FM_CASE(1);
+    SUPRA_FM_CASE(2);
+    SUPRA_FM_CASE(3);
+    SUPRA_FM_CASE(4);
+    SUPRA_FM_CASE(5);
+    SUPRA_FM_CASE(6);
+    SUPRA_FM_CASE(7);
+    SUPRA_FM_CASE(8);
+    SUPRA_FM_CASE(9);
+    SUPRA_FM_CASE(10);
+    SUPRA_FM_CASE(11);
+    SUPRA_FM_CASE(12);
+    SUPRA_FM_CASE(13);
+    SUPRA_FM_CASE(14);
+    SUPRA_FM_CASE(15);
+#undef SUPRA_FM_CASE
+}
+
+// Lane N's value in each row of 16 lanes.
+template <int N> __device__ inline float row_bcast(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
+}
+
+template <typename T> __device__ inline T row_sum(T v) {
+#pragma unroll
+    for (int m = 8; m > 0; m >>= 1) v += __shfl_xor(v, m, 16);
+    return v;
+}
+
+// 1/sqrt in FP64: hardware estimate and one Newton step (NaN for v <= 0)
+__device__ inline double rsqrt64(double v) {
+    const double r = __builtin_amdgcn_rsq(v);
+    return r * (1.5 - (0.5 * v) * (r * r));
+}
+
+template <int LMAX> struct System {
+    static constexpr int kB = LMAX / 16;
+    float a[kB][LMAX];       // row 16 r + q in slot r; entries beyond column 16 r + 15 unused
+    double dd[kB];           // running diagonal of the slot's row
+    float b1[kB], b2[kB];    // right-hand sides
+};
+
+// Elimination step J: column J scaled by 1/pivot, then subtracted from the
+// rows below.  Rows at or above the pivot take a zero multiplier; entries
+// right of a row's own column are its unused upper part.
+template <int LMAX, int J>
+__device__ __attribute__((always_inline)) inline void eliminate(System<LMAX>& s, int q) {
+    constexpr int rj = J / 16, qj = J % 16, kB = LMAX / 16;
+    const float invg = row_bcast<qj>(static_cast<float>(rsqrt64(s.dd[rj])));
+    const float z1 = row_bcast<qj>(s.b1[rj]) * invg;
+    const float z2 = row_bcast<qj>(s.b2[rj]) * invg;
+    float l[kB], nl[kB];
+#pragma unroll
+    for (int r = rj; r < kB; r++) {
+        l[r] = s.a[r][J] * invg;
+        if (r == rj) l[r] = q > qj ? l[r] : 0.0f;
+        nl[r] = -l[r];
+        s.dd[r] = fma(-static_cast<double>(l[r]), static_cast<double>(l[r]), s.dd[r]);
+        s.b1[r] = fmaf(nl[r], z1, s.b1[r]);
+        s.b2[r] = fmaf(nl[r], z2, s.b2[r]);
+    }
+#pragma unroll
+    for (int r = rj; r < kB; r++) {
+        if constexpr (qj < 15) fmac16<(qj + 1) % 16>(&s.a[r][16 * rj], l[rj], nl[r]);
+#pragma unroll
+        for (int c = rj + 1; c <= r; c++) fmac16<0>(&s.a[r][16 * c], l[c], nl[r]);
+    }
+}
+
+template <int LMAX, int J>
+__device__ __attribute__((always_inline)) inline void eliminate_from(System<LMAX>& s, int q, int nmax) {
+    if constexpr (J < LMAX) {
+        if (J < nmax) eliminate<LMAX, J>(s, q);   // uniform
+        eliminate_from<LMAX, J + 1>(s, q, nmax);
+    }
+}
+
+// The samples of outputs [t0, t0 + n_out) of scanline s.
+template <int LMAX>
+__device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int n_out, int h_lo, const float* xs,
+                                     const SampleMeta* meta, const float* mats, int wave) {
+    constexpr int kB = LMAX / 16;
+    const int lane = static_cast<int>(threadIdx.x % 64), q = lane % 16;
+    const int rs = static_cast<int>(a.rs);
+    for (int o0 = wave * 4; o0 < n_out; o0 += 4 * Cfg<LMAX>::kWaves) {
+        const int o = min(o0 + lane / 16, n_out - 1);    // a spare row of lanes repeats the last sample
+        const int t = t0 + o, ht = t - h_lo;
+        const SampleMeta m = meta[ht];
+        const int n = m.lt;
+        const float* mat = mats + o * Cfg<LMAX>::kMatrix;
+        System<LMAX> s;
+        float diag[kB], tr = 0.0f;
+#pragma unroll
+        for (int r = 0; r < kB; r++) {
+#pragma unroll
+            for (int c = 0; c < r; c++)
+#pragma unroll
+                for (int v = 0; v < 4; v++) {
+                    const float4 x = *reinterpret_cast<const float4*>(mat + block_at(r, c) + v * 64 + q * 4);
+                    float* p = &s.a[r][16 * c + 4 * v];
+                    p[0] = x.x, p[1] = x.y, p[2] = x.z, p[3] = x.w;
+                }
+#pragma unroll
+            for (int v = 0; v < 4; v++) {   // (rows above the chunk read its first row: unused entries)
+                const float4 x = *reinterpret_cast<const float4*>(mat + block_at(r, r) + diag_chunk(v) + max(q - 4 * v, 0) * 4);
+                float* p = &s.a[r][16 * r + 4 * v];
+                p[0] = x.x, p[1] = x.y, p[2] = x.z, p[3] = x.w;
+            }
+            const int dc = q / 4;
+            diag[r] = mat[block_at(r, r) + dc * 64 - (dc * (dc - 1) / 2) * 16 + (q % 4) * 4 + q % 4];
+            tr += 16 * r + q < n ? diag[r] : 0.0f;
+        }
+        const float trace = row_sum(tr);
+        const float delta = ((1.0f / static_cast<float>(n)) * trace) * a.alpha;
+        int bad = 0;
+        for (int h = max(0, ht - static_cast<int>(a.T)); h <= min(static_cast<int>(a.n_d) - 1 - h_lo, ht + static_cast<int>(a.T)); h++)
+            bad |= meta[h].bad;
+#pragma unroll
+        for (int r = 0; r < kB; r++) {
+            s.dd[r] = static_cast<double>(diag[r] + delta);
+            s.b1[r] = 1.0f;
+            // sub-array sums x_i = sum_k x[f+k+i] (applyWeights, RxBeamformerMV.cu:342-376)
+            float acc = 0.0f;
+            const float* x = xs + ht * rs + m.first + 16 * r + q;
+            for (int k = 0; k < m.kact; k++) acc += x[k];
+            s.b2[r] = acc;
+        }
+        int nmax = n;
+#pragma unroll
+        for (int p = 16; p < 64; p += 16) nmax = max(nmax, __shfl_xor(nmax, p, 64));
+        eliminate_from<LMAX, 0>(s, q, __builtin_amdgcn_readfirstlane(nmax));
+        double zz = 0.0, uz = 0.0;
+#pragma unroll
+        for (int r = 0; r < kB; r++) {
+            // row 16 r + q's right-hand sides and diagonal are final
+            const float ginv = static_cast<float>(rsqrt64(s.dd[r]));
+            const float z = s.b1[r] * ginv, u = s.b2[r] * ginv;
+            if (16 * r + q < n) {
+                zz += static_cast<double>(z) * static_cast<double>(z);
+                uz += static_cast<double>(u) * static_cast<double>(z);
+            }
+        }
+        zz = row_sum(zz);
+        uz = row_sum(uz);
+        float y = static_cast<float>(uz) / (static_cast<float>(zz) * powf(static_cast<float>(m.kact), a.p));
+        if (fabsf(y) > 1e7f || isnan(y) || bad) y = 0.0f;
+        if (q == 0 && o0 + lane / 16 < n_out) {
+            const uint64_t at = static_cast<uint64_t>(t) * a.n_rx + scan;
+            y *= static_cast<float>(a.n_ch);
+            if (a.out_i16) static_cast<int16_t*>(a.out)[at] = clamp_out<int16_t>(y);
+            else static_cast<float*>(a.out)[at] = clamp_out<float>(y);
+        }
+    }
+}
+
+// Marks the samples whose covariance is not finite in single precision (e.g.
+// from a -FLT_MAX pre-delayed value): by Cauchy-Schwarz those with a
+// non-finite diagonal entry, which is at most the sample's energy.
+template <int LMAX>
+__device__ inline void find_bad(const MvArgs& a, const float* xs, const float* mean, int H, SampleMeta* meta) {
+    constexpr int kWaves = Cfg<LMAX>::kWaves;
+    const int wave = static_cast<int>(threadIdx.x / 64), lane = static_cast<int>(threadIdx.x % 64);
+    const int n_ch = static_cast<int>(a.n_ch), rs = static_cast<int>(a.rs);
+    for (int h = wave; h < H; h += kWaves) {
+        float e = 0.0f;
+        for (int c = lane; c < n_ch; c += 64) e += xs[h * rs + c] * xs[h * rs + c];
+#pragma unroll
+        for (int m = 32; m > 0; m >>= 1) e += __shfl_xor(e, m, 64);
+        if (e <= 1e38f) continue;      // uniform
+        const SampleMeta m = meta[h];
+        double r = 0.0;
+        if (lane < m.lt) {
+            for (int k = 0; k < m.kact; k++) {
+                const double x = static_cast<double>(xs[h * rs + m.first + k + lane]);
+                r = fma(x, x, r);
+            }
+            if (mean) {
+                const double mu = static_cast<double>(mean[h * LMAX + lane]);
+                r -= static_cast<double>(m.kact) * mu * mu;
+            }
+        }
+        if (__ballot(!(fabsf(static_cast<float>(r)) <= FLT_MAX)) != 0 && lane == 0) meta[h].bad = 1;
+    }
+}
+
+template <typename InT, int LMAX, bool FUSED>
+__device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t scan, uint32_t tile, unsigned char* lds) {
+    constexpr int kThreads = Cfg<LMAX>::kThreads;
+    float* xs = reinterpret_cast<float*>(lds);
+    SampleMeta* meta = reinterpret_cast<SampleMeta*>(lds + a.off_meta);
+    float* mean = a.means ? reinterpret_cast<float*>(lds + a.off_mean) : nullptr;
+    float* mats = reinterpret_cast<float*>(lds + a.off_r);
+    const uint32_t t0 = tile * a.tile, t1 = min(t0 + a.tile, a.n_d);
+    const uint32_t h_lo = t0 >= a.T ? t0 - a.T : 0;
+    const int H = static_cast<int>(min(a.n_d - 1, t1 - 1 + a.T) - h_lo + 1);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64));
+
+    if (FUSED) stage_delayed<InT, kThreads>(a, lut, scan, h_lo, H, xs, lds);
+    else stage_read<InT, kThreads>(a, scan, h_lo, H, xs);
+    find_apertures<kThreads>(a, xs, H, meta);
+    __syncthreads();
+    if (mean) {
+        for (int idx = threadIdx.x; idx < H * LMAX; idx += kThreads) {
+            const int h = idx / LMAX, i = idx % LMAX;
+            const SampleMeta m = meta[h];
+            float acc = 0.0f;
+            if (i < m.lt) {
+                for (int k = 0; k < m.kact; k++) acc += xs[h * a.rs + m.first + k + i];
+                acc = acc / static_cast<float>(m.kact);
+            }
+            mean[idx] = acc;
+        }
+        __syncthreads();
+    }
+    find_bad<LMAX>(a, xs, mean, H, meta);
+    __syncthreads();
+    Gram g;
+    g.xs = xs;
+    g.meta = meta;
+    g.mean = mean;
+    g.mats = mats;
+    g.rs = static_cast<int>(a.rs);
+    g.mean_stride = LMAX;
+    g.matrix = Cfg<LMAX>::kMatrix;
+    g.T = static_cast<int>(a.T);
+    g.n_d = static_cast<int>(a.n_d);
+    g.h_lo = static_cast<int>(h_lo);
+    const int n_out = static_cast<int>(t1 - t0);
+    all_window_sums<LMAX>(g, static_cast<int>(t0), n_out, static_cast<int>(a.sub), wave);
+    __syncthreads();
+    solve_outputs<LMAX>(a, scan, static_cast<int>(t0), n_out, g.h_lo, xs, meta, mats, wave);
+}
+
+// Renumbers the workgroups as mv_logical_wg in mv_kernels.hip does: 32
+// consecutive tiles (which share halos) on one XCD, XCDs rotated per round.
+constexpr uint32_t kXcdTile = 32;
+
+template <typename InT, int LMAX, bool FUSED>
+__global__ __launch_bounds__(Cfg<LMAX>::kThreads) void mv_block_kernel(const MvArgs a) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    const uint32_t b = blockIdx.x, xcd = b % 8u, local = b / 8u;
+    const uint32_t round = local / kXcdTile, k = local % kXcdTile;
+    const uint32_t wg = (round * 8u + (xcd + round) % 8u) * kXcdTile + k;
+    if (wg >= a.n_rx * a.n_tiles) return;   // whole workgroup: the padded grid
+    mv_block_tile<InT, LMAX, FUSED>(a, a.g.lut, wg / a.n_tiles, wg % a.n_tiles, lds);
+}
+
+// Persistent work queue over many frames (fused pre-delay), as mv_batch_kernel.
+template <typename InT, int LMAX>
+__global__ __launch_bounds__(Cfg<LMAX>::kThreads) void mv_block_batch_kernel(const MvBatchArgs b) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ uint32_t s_item;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) s_item = atomicAdd(b.sync.head, 1u);
+        __syncthreads();
+        const uint32_t item = s_item;
+        if (item >= b.n_items) break;
+        const uint32_t code = b.items[item];
+        const MvBatchFrame& fr = b.frames[code >> 24];
+        const MvArgs a = fr.a;     // scalars of the frame (the LUT is read from fr)
+        const uint32_t local = code & 0xffffffu;
+        mv_block_tile<InT, LMAX, true>(a, fr.a.g.lut, local / a.n_tiles, local % a.n_tiles, lds);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            __threadfence();
+            if (atomicAdd(&b.sync.done[fr.frame], 1u) + 1u == fr.n_items) b.sync.stamp[fr.frame] = wall_clock64();
+        }
+    }
+}
+
+size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
+    const uint32_t H = tile + 2 * a.T, blocks = lmax / 16;
+    a.tile = tile;
+    size_t off = (static_cast<size_t>(H) * a.rs * 4 + 15) & ~static_cast<size_t>(15);
+    a.off_meta = static_cast<uint32_t>(off);
+    off += static_cast<size_t>(H) * sizeof(SampleMeta);
+    a.off_mean = static_cast<uint32_t>(off);
+    off += a.means ? static_cast<size_t>(H) * lmax * 4 : 0;
+    a.off_r = static_cast<uint32_t>(off);
+    // the pre-delay tables are only read before the matrices are written
+    const size_t mats = static_cast<size_t>(tile) * (blocks * 160 + blocks * (blocks - 1) / 2 * 256) * 4;
+    a.off_fused = static_cast<uint32_t>(off);
+    const size_t fused = a.g.rf ? (kWindowEntries + 4 * static_cast<size_t>(a.n_ch) + 6 * static_cast<size_t>(H)) * 4 : 0;
+    return off + std::max(mats, fused);
+}
+
+}  // namespace
+
+uint32_t mv_block_lmax(uint32_t L) { return L <= 16 ? 16 : (L <= 32 ? 32 : 64); }
+
+bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds) {
+    const uint32_t lmax = mv_block_lmax(a.L), w = 2 * a.T + 1;
+    // zero padding: the last 4-term step and the unused rows read past the aperture
+    a.rs = a.n_ch + lmax + 4;
+    // Of the tiles that fit, the one with the least modelled time per output:
+    // subs (w - 1) + tile covariance evaluations on the busiest wave (9 or 41
+    // matrix instructions of 64 cycles; the waves share them with 16 rows) and
+    // one round of 4 systems per wave.
+    const uint32_t waves = lmax == 32 ? 3 : 4;
+    const double eval = lmax == 64 ? 2600.0 : (lmax == 32 ? 580.0 : 320.0);
+    const double solve = lmax == 64 ? 23000.0 : (lmax == 32 ? 6000.0 : 2000.0);
+    double best = 0;
+    uint32_t pick = 0;
+    for (uint32_t tile = 1; tile <= 4 * waves; tile++) {
+        if (plan_lds(a, lmax, tile) > budget) break;
+        const uint32_t per_wave = lmax == 16 ? (tile + waves - 1) / waves : tile;
+        const uint32_t subs = (per_wave + w - 1) / w;
+        const double cost = ((subs * (w - 1) + per_wave) * eval + solve) / tile;
+        if (pick && cost >= best) continue;
+        best = cost;
+        pick = tile;
+        a.sub = (per_wave + subs - 1) / subs;
+    }
+    if (!pick) return false;
+    if (pick > a.n_d) {
+        pick = a.n_d;
+        a.sub = std::min(a.sub, pick);
+    }
+    *lds = plan_lds(a, lmax, pick);
+    a.n_tiles = (a.n_d + pick - 1) / pick;
+    return true;
+}
+
+template <typename InT, bool FUSED>
+static hipError_t launch_in(const MvArgs& a, size_t lds, hipStream_t stream) {
+    const uint32_t round = 8u * kXcdTile;
+    const dim3 grid((a.n_rx * a.n_tiles + round - 1) / round * round);
+    switch (mv_block_lmax(a.L)) {
+        case 16: hipLaunchKernelGGL((mv_block_kernel<InT, 16, FUSED>), grid, dim3(Cfg<16>::kThreads), lds, stream, a); break;
+        case 32: hipLaunchKernelGGL((mv_block_kernel<InT, 32, FUSED>), grid, dim3(Cfg<32>::kThreads), lds, stream, a); break;
+        default: hipLaunchKernelGGL((mv_block_kernel<InT, 64, FUSED>), grid, dim3(Cfg<64>::kThreads), lds, stream, a); break;
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_mv_block(const MvArgs& a, int32_t in_dtype, bool fused, size_t lds, hipStream_t stream) {
+    if (in_dtype == SUPRA_INT16)
+        return fused ? launch_in<int16_t, true>(a, lds, stream) : launch_in<int16_t, false>(a, lds, stream);
+    return fused ? launch_in<float, true>(a, lds, stream) : launch_in<float, false>(a, lds, stream);
+}
+
+template <typename InT>
+static hipError_t launch_batch_in(const MvBatchArgs& b, uint32_t lmax, uint32_t workgroups, size_t lds, hipStream_t stream) {
+    const dim3 grid(workgroups);
+    if (lmax == 16) hipLaunchKernelGGL((mv_block_batch_kernel<InT, 16>), grid, dim3(Cfg<16>::kThreads), lds, stream, b);
+    else if (lmax == 32) hipLaunchKernelGGL((mv_block_batch_kernel<InT, 32>), grid, dim3(Cfg<32>::kThreads), lds, stream, b);
+    else hipLaunchKernelGGL((mv_block_batch_kernel<InT, 64>), grid, dim3(Cfg<64>::kThreads), lds, stream, b);
+    return hipGetLastError();
+}
+
+hipError_t launch_mv_block_batch(const MvBatchArgs& b, uint32_t lmax, int32_t rf_dtype, uint32_t workgroups, size_t lds,
+                                 hipStream_t stream) {
+    return rf_dtype == SUPRA_INT16 ? launch_batch_in<int16_t>(b, lmax, workgroups, lds, stream)
+                                   : launch_batch_in<float>(b, lmax, workgroups, lds, stream);
+}
+
+}  // namespace supra_amd

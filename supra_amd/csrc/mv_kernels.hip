@@ -43,6 +43,7 @@
 #include "bf_internal.hpp"
 #include "das_device.hpp"
 #include "mv_launch.hpp"
+#include "mv_stage.hpp"
 #include "status.hpp"
 #include "supra_bf.h"
 
@@ -53,14 +54,6 @@ constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kMaxTile = 64;
 
-
-template <typename T> __device__ inline float in_f(T v) { return static_cast<float>(v); }
-
-template <typename T> __device__ inline T clamp_out(float x);
-template <> __device__ inline float clamp_out<float>(float x) { return fminf(fmaxf(x, -FLT_MAX), FLT_MAX); }
-template <> __device__ inline int16_t clamp_out<int16_t>(float x) {
-    return static_cast<int16_t>(fminf(fmaxf(x, -32767.0f), 32767.0f));
-}
 
 __device__ inline float wave_sum(float v) {
     for (int m = 32; m > 0; m >>= 1) v += __shfl_xor(v, m, 64);
@@ -84,11 +77,6 @@ __device__ inline double bcast(double v, int lane) {
     const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(u >> 32), lane));
     return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
-
-struct SampleMeta {
-    int32_t first, lt, kact;
-    int32_t bad;    // a non-finite channel value: every window holding it ends as NaN -> 0
-};
 
 __device__ inline uint32_t packed_index(uint32_t i, uint32_t j, uint32_t L) {
     // upper triangle, row-major: row i holds columns i..L-1
@@ -183,7 +171,6 @@ __device__ inline float sub_min(float v) {
 
 // Conditioning below which the FP64 residual check is skipped: the a-priori
 // bound 1 + n/alpha of a loaded system, or the squared-pivot ratio.
-constexpr float kKappaSafe = 1.0e4f;
 constexpr float kPivotRatioSafe = 64.0f;
 
 // Solve (G G^T) v = b for the sub-wave's pixel: G's row i is in lane i's
@@ -264,104 +251,6 @@ __device__ inline float pcg_solve(const float (&A)[LMAX], float mdiag, int n, in
     return x;
 }
 
-// Fused mode: the pre-delayed samples of scanline s, depths [h_lo, h_lo+H),
-// computed from the RF exactly as the pre-delay kernel writes them
-// (rawdelay2d_kernel in das_kernels.hip; RawDelay.cu:221-312, 404-468):
-// highest-weight transmit, aperture element c = e - first, w * interp * n/W
-// through clampCast<float>, 0 for c >= last - first.  Same operations in the
-// same order, so the values are bit-identical to the two-kernel path.
-template <typename RFT>
-__device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t s, uint32_t h_lo, int H,
-                                     float* xs, unsigned char* lds) {
-    const DasArgs& g = a.g;
-    const int n_ch = static_cast<int>(a.n_ch);
-    const int hstride = static_cast<int>(a.tile + 2 * a.T);
-    float* s_lut = reinterpret_cast<float*>(lds + a.off_fused);
-    float* s_xe = s_lut + kWindowEntries;
-    float* s_dx = s_xe + n_ch;
-    float* s_dx2 = s_dx + n_ch;
-    uint32_t* s_off = reinterpret_cast<uint32_t*>(s_dx2 + n_ch);
-    float* p_d = reinterpret_cast<float*>(s_off + n_ch);
-    float* p_adt = p_d + hstride;
-    float* p_inv = p_adt + hstride;
-    float* p_px = p_inv + hstride;
-    float* p_py2 = p_px + hstride;
-    float* p_scale = p_py2 + hstride;
-
-    const ScanView sc = scan_view(g.scans, s);
-    const int k = sc.sel();
-    TxDT tx{};
-    int cnt = 0;
-    if (k >= 0) {
-        tx = sc.tx(k);
-        cnt = tx.last_x > tx.first_x ? static_cast<int>(tx.last_x - tx.first_x) : 0;
-    }
-    for (int i = threadIdx.x; i < kWindowEntries; i += kThreads) s_lut[i] = lut[i];
-    for (int j = threadIdx.x; j < cnt; j += kThreads) {
-        const int e = static_cast<int>(tx.first_x) + j;
-        const float xe = g.ex[e];
-        const float dx = xe - sc.x();
-        s_xe[j] = xe;
-        s_dx[j] = dx;
-        s_dx2[j] = dx * dx;
-        s_off[j] = (static_cast<uint32_t>(e) % g.n_ch) * g.n_s;
-    }
-    __syncthreads();
-    // per-sample geometry and the aperture's weight sum and count
-    for (int h = threadIdx.x; h < H; h += kThreads) {
-        const float d = g.depths[h_lo + h];
-        const float aDT = (((d * g.dt) * g.c) / (2.0f * g.F)) / g.c / g.dt;
-        const float inv = 1.0f / fminf(aDT, sc.max_ed_x());
-        const float py = sc.dir_y() * d;
-        float wsum = 0.0f;
-        int nadd = 0;
-        for (int j = 0; j < cnt; j++) {
-            const float dx = s_dx[j];
-            if (fabsf(dx) <= aDT) {
-                wsum += s_lut[window_index(dx * inv)];
-                nadd++;
-            }
-        }
-        float scale = 1.0f;
-        if (nadd > 0) scale = 1.0f / wsum * static_cast<float>(nadd);
-        p_d[h] = d;
-        p_adt[h] = aDT;
-        p_inv[h] = inv;
-        p_px[h] = sc.x() + sc.dir_x() * d;
-        p_py2[h] = py * py;
-        p_scale[h] = scale;
-    }
-    __syncthreads();
-    const bool vertical = (sc.dir_x() == 0.0f);
-    const RFT* rf_tx = static_cast<const RFT*>(g.rf) + static_cast<uint64_t>(tx.tx_idx) * g.n_ch * g.n_s;
-    const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, g.n_ch * g.n_s * sizeof(RFT));
-    const int rs = static_cast<int>(a.rs);
-#pragma unroll 4
-    for (int idx = threadIdx.x; idx < H * rs; idx += kThreads) {
-        const int c = idx / H, h = idx % H;
-        float v = 0.0f;
-        if (c < cnt) {
-            float sample = 0.0f;
-            const float dx = s_dx[c];
-            if (fabsf(dx) <= p_adt[h]) {
-                const float w = s_lut[window_index(dx * p_inv[h])];
-                float q;
-                if (vertical) {
-                    q = s_dx2[c] + p_py2[h];
-                } else {
-                    const float e = s_xe[c] - p_px[h];
-                    q = e * e + p_py2[h];
-                }
-                const float tau = tx.t0 + (sqrt_rn(q) + p_d[h]);
-                gather<RFT, false>(rsrc, s_off[c], g.n_s, tau, w, sample);
-            }
-            v = clamp_cast<float>(sample * p_scale[h]);
-        }
-        xs[h * rs + c] = v;
-    }
-    __syncthreads();
-}
-
 // One workgroup tile: output depths [tile * a.tile, ...) of scanline s.
 // Diagonals da <= db of one sample's R (db == da: one diagonal), entries
 // (i, i + d) for i < L - d, given each first entry's sum
@@ -417,57 +306,11 @@ __device__ __attribute__((always_inline)) inline void mv_tile(const MvArgs& a, c
 
     // 1. stage x (zero padded to rs channels) and per-sample aperture
     if (FUSED) {
-        stage_delayed<InT>(a, lut, s, h_lo, H, xs, lds);
+        stage_delayed<InT, kThreads>(a, lut, s, h_lo, H, xs, lds);
     } else {
-        const InT* xin = static_cast<const InT*>(a.x) + static_cast<uint64_t>(s) * a.n_ch * a.n_d;
-        // batches of 8 loads per lane in flight before the LDS stores (the
-        // loop is otherwise one global-memory round trip per element)
-        constexpr int kBatch = 8;
-        const int total = H * rs, n_ch = static_cast<int>(a.n_ch);
-        for (int base = 0; base < total; base += kBatch * kThreads) {
-            float v[kBatch];
-#pragma unroll
-            for (int u = 0; u < kBatch; u++) {
-                const int idx = base + u * kThreads + static_cast<int>(threadIdx.x);
-                const int c = idx / H, h = idx % H;
-                v[u] = (idx < total && c < n_ch) ? in_f(xin[static_cast<uint64_t>(c) * a.n_d + h_lo + h]) : 0.0f;
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; u++) {
-                const int idx = base + u * kThreads + static_cast<int>(threadIdx.x);
-                const int c = idx / H, h = idx % H;
-                if (idx < total) xs[h * rs + c] = v[u];
-            }
-        }
-        __syncthreads();
+        stage_read<InT, kThreads>(a, s, h_lo, H, xs);
     }
-    // first / last channel with a non-zero sample (0 when there is none): one
-    // wave per sample, 64 channels per ballot
-    {
-        const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
-        const int n_ch = static_cast<int>(a.n_ch);
-        for (int h = wv; h < H; h += kWaves) {
-            const float* row = xs + h * rs;
-            int f = -1, l = 0;
-            for (int cb = 0; cb < n_ch; cb += 64) {
-                const int c = cb + ln;
-                const uint64_t nz = __ballot(c < n_ch && row[c] != 0.0f);
-                if (nz != 0) {
-                    if (f < 0) f = cb + __ffsll(static_cast<unsigned long long>(nz)) - 1;
-                    l = cb + 63 - __clzll(static_cast<long long>(nz));
-                }
-            }
-            if (f < 0) f = 0;
-            if (ln == 0) {
-                SampleMeta m;
-                m.first = f;
-                m.lt = min(L, l - f + 1);
-                m.kact = min(static_cast<int>(a.K), l - f - m.lt + 2);
-                m.bad = 0;
-                meta[h] = m;
-            }
-        }
-    }
+    find_apertures<kThreads>(a, xs, H, meta);
     __syncthreads();
     if (MEANS) {
         for (int idx = threadIdx.x; idx < H * L; idx += kThreads) {
@@ -645,13 +488,13 @@ __device__ __attribute__((always_inline)) inline void mv_tile(const MvArgs& a, c
             // (positive semi-definite), so with the loading delta = alpha trace/n
             // its condition number is at most (trace + delta) / delta = 1 + n/alpha;
             // the ratio of the largest to the smallest squared pivot is a lower
-            // bound on it.  Below kKappaSafe (bound) or kPivotRatioSafe (pivots)
+            // bound on it.  Below kMvKappaSafe (bound) or kPivotRatioSafe (pivots)
             // the FP32 factorisation already solves to about kappa * 6e-8.
             float dmax = (li < n) ? static_cast<float>(dd) : 0.0f;
             float dmin = (li < n) ? static_cast<float>(dd) : FLT_MAX;
             dmax = sub_max<PPW>(dmax);
             dmin = sub_min<PPW>(dmin);
-            const bool loaded_ok = a.alpha > 0.0f && 1.0f + static_cast<float>(n) / a.alpha <= kKappaSafe;
+            const bool loaded_ok = a.alpha > 0.0f && 1.0f + static_cast<float>(n) / a.alpha <= kMvKappaSafe;
             const bool suspect = ok && !loaded_ok && !(dmax <= kPivotRatioSafe * dmin);
             for (int it = 0; it < 3 && __any(suspect); it++) {
                 double r = 0.0;
@@ -723,7 +566,11 @@ hipError_t launch_lmax(const MvArgs& a, size_t lds, hipStream_t stream) {
 }
 
 template <bool FUSED>
-hipError_t launch_io(const MvArgs& a, int in_dtype, int out_dtype, size_t lds, hipStream_t hs) {
+hipError_t launch_io(MvArgs& a, int in_dtype, int out_dtype, size_t lds, hipStream_t hs) {
+    if (a.block) {
+        a.out_i16 = out_dtype == SUPRA_INT16 ? 1 : 0;
+        return launch_mv_block(a, in_dtype, FUSED, lds, hs);
+    }
     if (in_dtype == SUPRA_INT16)
         return (out_dtype == SUPRA_FLOAT32) ? launch_lmax<int16_t, float, FUSED>(a, lds, hs)
                                             : launch_lmax<int16_t, int16_t, FUSED>(a, lds, hs);
@@ -801,7 +648,7 @@ namespace supra_amd {
 // Argument checks and the LDS/tile plan shared by both entry points.
 int mv_prepare(MvArgs& a, uint32_t num_scanlines, uint32_t num_channels, uint32_t num_samples,
                uint32_t sub_array_size, uint32_t temporal_smoothing, double sub_array_scaling_power,
-               int32_t compute_means, double loading_factor, size_t lds_budget, size_t* lds_out) {
+               int32_t compute_means, double loading_factor, bool pcg, size_t lds_budget, size_t* lds_out) {
     if (num_scanlines == 0 || num_channels == 0 || num_samples == 0)
         return fail(SUPRA_ERR_INVALID_ARG, "mv: empty input");
     const uint32_t L = sub_array_size == 0 ? num_channels / 2 : sub_array_size;
@@ -817,13 +664,19 @@ int mv_prepare(MvArgs& a, uint32_t num_scanlines, uint32_t num_channels, uint32_
     a.L = L;
     a.T = temporal_smoothing;
     a.K = num_channels - L + 1;
-    a.rs = num_channels + L + 8;   // zero padding for the sliding windows of the covariance phase
     a.packed = L * (L + 1) / 2;
     a.p = static_cast<float>(sub_array_scaling_power);
     a.alpha = static_cast<float>(loading_factor);
     a.means = compute_means ? 1 : 0;
     const size_t budget = lds_budget ? std::min(lds_budget, static_cast<size_t>(max_lds_per_block()))
                                      : static_cast<size_t>(max_lds_per_block());
+    if (!pcg && mv_well_loaded(L, loading_factor) && mv_block_plan(a, budget, lds_out)) {
+        a.block = 1;
+        if (static_cast<uint64_t>(a.n_tiles) * num_scanlines >= (1ull << 31))
+            return fail(SUPRA_ERR_TOO_LARGE, "mv: too many workgroups");
+        return SUPRA_OK;
+    }
+    a.rs = num_channels + L + 8;   // zero padding for the sliding windows of the covariance phase
     // Without an explicit budget, prefer two workgroups per CU (the solve
     // phase is latency-bound; a second resident workgroup hides it) as long as
     // the tile keeps the temporal halo overhead moderate; else one workgroup
@@ -883,7 +736,7 @@ int launch_mv_fused(const DasArgs& g, int32_t rf_dtype, uint32_t sub_array_size,
     a.out = out;
     size_t lds = 0;
     int st = mv_prepare(a, g.n_rx, g.n_ch, g.n_depths, sub_array_size, temporal_smoothing, sub_array_scaling_power,
-                        compute_means, loading_factor, 0, &lds);
+                        compute_means, loading_factor, false, 0, &lds);
     if (st != SUPRA_OK) return st;
     hipError_t e = launch_io<true>(a, rf_dtype, out_dtype, lds, stream);
     if (e != hipSuccess) return fail(SUPRA_ERR_HIP, "mv: launch: %s", hipGetErrorString(e));
@@ -907,7 +760,7 @@ extern "C" int supra_mv_run(const void* raw_delayed, int32_t in_dtype, uint32_t 
     a.out = out;
     size_t lds = 0;
     int st = mv_prepare(a, num_scanlines, num_channels, num_samples, sub_array_size, temporal_smoothing,
-                        sub_array_scaling_power, compute_means, loading_factor, 0, &lds);
+                        sub_array_scaling_power, compute_means, loading_factor, false, 0, &lds);
     if (st != SUPRA_OK) return st;
     hipError_t e = launch_io<false>(a, in_dtype, out_dtype, lds, static_cast<hipStream_t>(stream));
     if (e != hipSuccess) return fail(SUPRA_ERR_HIP, "mv: launch: %s", hipGetErrorString(e));
@@ -935,7 +788,7 @@ extern "C" int supra_mvpcg_run(const void* raw_delayed, int32_t in_dtype, uint32
     size_t lds = 0;
     // loading trace / L_t as addDiagonalLoading (RxBeamformerMVpcg.cu:295-330)
     int st = mv_prepare(a, num_scanlines, num_channels, num_samples, sub_array_size, temporal_smoothing,
-                        sub_array_scaling_power, compute_means, 1.0, 0, &lds);
+                        sub_array_scaling_power, compute_means, 1.0, true, 0, &lds);
     if (st != SUPRA_OK) return st;
     // maxIterations = the sub-array size unless overridden (:649)
     a.pcg_iters = max_iterations_override ? max_iterations_override : a.L;

@@ -24,6 +24,9 @@ struct MvArgs {
     int means;
     uint32_t pcg_iters;     // 0: Cholesky solve; else at most this many PCG iterations
     float pcg_threshold;    // PCG stops once |1 - R~ w| <= this
+    int32_t block;          // planned for mv_block.hip (else mv_kernels.hip)
+    uint32_t sub;           // mv_block.hip: outputs per sub-block (at most 2T + 1)
+    int32_t out_i16;        // mv_block.hip: int16 output (else float)
     DasArgs g;              // fused mode: geometry and RF of the pre-delay
 };
 
@@ -47,11 +50,31 @@ struct MvBatchArgs {
 // built from different revisions of the struct must not be linked together).
 size_t mv_batch_frame_bytes();
 
-// Plan (tile of output depths, waves, LDS offsets) for a frame; lds_budget 0
-// picks the single-launch default.  Returns a SUPRA_* status.
+// Conditioning bound below which a loaded system needs no FP64 refinement:
+// R~ is positive semi-definite, so with the loading delta = alpha trace / n
+// its condition number is at most 1 + n / alpha, and the FP32 factorisation
+// solves to about that times 6e-8.
+constexpr float kMvKappaSafe = 1.0e4f;
+inline bool mv_well_loaded(uint32_t L, double alpha) {
+    const float al = static_cast<float>(alpha);
+    return al > 0.0f && 1.0f + static_cast<float>(L) / al <= kMvKappaSafe;
+}
+
+// Plan (kernel, tile of output depths, waves, LDS offsets) for a frame;
+// lds_budget 0 picks the single-launch default.  Well-loaded systems go to
+// mv_block.hip, weakly loaded ones (FP64 refinement) and conjugate gradients
+// (pcg) to mv_kernels.hip.  Returns a SUPRA_* status.
 int mv_prepare(MvArgs& a, uint32_t num_scanlines, uint32_t num_channels, uint32_t num_samples,
                uint32_t sub_array_size, uint32_t temporal_smoothing, double sub_array_scaling_power,
-               int32_t compute_means, double loading_factor, size_t lds_budget, size_t* lds_out);
+               int32_t compute_means, double loading_factor, bool pcg, size_t lds_budget, size_t* lds_out);
+
+// mv_block.hip: rows the kernel is built for (16, 32 or 64), the plan for an
+// LDS budget (false: does not fit), and the launches.
+uint32_t mv_block_lmax(uint32_t L);
+bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds);
+hipError_t launch_mv_block(const MvArgs& a, int32_t in_dtype, bool fused, size_t lds, hipStream_t stream);
+hipError_t launch_mv_block_batch(const MvBatchArgs& b, uint32_t lmax, int32_t rf_dtype, uint32_t workgroups, size_t lds,
+                                 hipStream_t stream);
 
 // Persistent work-queue launch over a batch's minimum-variance frames of one
 // kernel class (sub-array bound, RF type, mean removal); float output.
