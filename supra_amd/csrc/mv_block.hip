@@ -21,11 +21,7 @@
 //      upwards (added to what was stored).  No sum is ever subtracted from,
 //      so a weak window next to a strong echo keeps its precision, and about
 //      2 evaluations per output replace the 2T + 1 additions of stored
-//      covariances.  Along a block diagonal, block (r+1, c+1) differs from
-//      (r, c) by 16 entering and 16 leaving products, so with LMAX = 64 the first
-//      block column (and one more block, to even out the waves) is summed in
-//      full and the rest by differences (125 instead of 170 matrix
-//      instructions per sample with 65 sub-arrays);
+//      covariances;
 //   3. sixteen lanes per system, row 16 r + q in slot r of lane q: diagonal
 //      loading, then a right-looking Cholesky factorisation whose column is
 //      broadcast inside the FMAs (DPP row_newbcast), FP64 pivots and
@@ -34,11 +30,16 @@
 //      xs^T R~^-1 1 / 1^T R~^-1 1 = u.z / z.z: no backward substitution and
 //      no factor kept.
 //
-// Bound by vector instructions (56 % busy) and the matrix cores (24 % busy) at
-// L = 32; by the latency of one wave per SIMD at L = 64, whose matrices fill
-// the LDS.  128 x 2080 samples, L = 32, T = 5: 0.80 ms against 2.02 ms of
-// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 2.93 ms against
-// 9.54 ms; relative error of the image against FP64 1.1e-6 against 1.6e-6.
+// Bound by the FP64 pipe at L = 32: the matrix instructions (26 % of the time)
+// and the vector instructions (49 %) of the waves of a SIMD add up.  At L = 64
+// the matrices fill the LDS and one wave per SIMD waits for itself.
+// 128 x 2080 samples, L = 32, T = 5: 0.69 ms against 2.01 ms of
+// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 2.01 ms against
+// 9.49 ms; relative error of the image against FP64 1.4e-6 against 1.9e-6.
+// Summing the blocks off the first column by differences along the block
+// diagonals (fewer matrix instructions, but longer serial chains) and running
+// the two accumulations of a sub-block side by side were slower (2.49 and
+// 2.58 ms at L = 64).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -77,105 +78,120 @@ __device__ constexpr int diag_chunk(int chunk) { return chunk == 0 ? 0 : (chunk 
 
 struct Gram {
     const float* xs;
-    const SampleMeta* meta;
+    const uint32_t* code;  // per staged sample: first | active sub-arrays << 10, or 0 for one left out
     const float* mean;     // [h][16 kBlocks], nullptr without mean removal
     float* mats;
     int rs, mean_stride, matrix;
     int T, n_d, h_lo;
 };
 
-// The block diagonal chain (R0, C0), (R0+1, C0+1), ... of LEN blocks.
-template <int R0, int C0, int LEN>
-struct Chain {
-    double4v acc[LEN];     // block (R0, C0), then the differences to the previous block
+__device__ inline double4v mfma64(float a, float b, double4v c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(a), static_cast<double>(b), c, 0, 0, 0);
+}
+
+// The matrix blocks (row block, column block) that one wave accumulates;
+// chosen so that the blocks of a wave share operands.
+template <int LMAX, int WAVE> struct Deal;
+template <int WAVE> struct Deal<16, WAVE> {
+    static constexpr int n = 1, r[3] = {0, 0, 0}, c[3] = {0, 0, 0};
+};
+template <> struct Deal<32, 0> { static constexpr int n = 1, r[3] = {0, 0, 0}, c[3] = {0, 0, 0}; };
+template <> struct Deal<32, 1> { static constexpr int n = 1, r[3] = {1, 0, 0}, c[3] = {0, 0, 0}; };
+template <> struct Deal<32, 2> { static constexpr int n = 1, r[3] = {1, 0, 0}, c[3] = {1, 0, 0}; };
+template <> struct Deal<64, 0> { static constexpr int n = 3, r[3] = {0, 1, 1}, c[3] = {0, 0, 1}; };
+template <> struct Deal<64, 1> { static constexpr int n = 3, r[3] = {2, 2, 2}, c[3] = {0, 1, 2}; };
+template <> struct Deal<64, 2> { static constexpr int n = 2, r[3] = {3, 3, 0}, c[3] = {0, 1, 0}; };
+template <> struct Deal<64, 3> { static constexpr int n = 2, r[3] = {3, 3, 0}, c[3] = {2, 3, 0}; };
+
+// Accumulators of a wave's blocks.  Matrix-core operands: lane = (row or
+// column, term); D[j][i] holds row i of the block in lane % 16 and column
+// j = lane / 16 + 4 v in register v.
+template <typename D>
+struct Blocks {
+    double4v acc[D::n];
     __device__ inline void clear() {
 #pragma unroll
-        for (int d = 0; d < LEN; d++) acc[d] = double4v{0.0, 0.0, 0.0, 0.0};
+        for (int b = 0; b < D::n; b++) acc[b] = double4v{0.0, 0.0, 0.0, 0.0};
     }
-    // acc += covariance of sample tau.  Matrix-core operands: lane = (row or
-    // column i = lane % 16, term k = lane / 16); D[j][i] holds row i of the
-    // block in lane % 16 and column j = lane / 16 + 4 v in register v.
+    // acc += the covariance of sample tau: 16 terms at a time, all loads of a
+    // group before its first matrix instruction, then 4; the last step reads
+    // up to 3 terms past the aperture (in the zeroed padding) and masks them.
     __device__ inline void add(const Gram& g, int tau) {
         const int h = tau - g.h_lo;
-        const SampleMeta m = g.meta[h];
-        if (__builtin_amdgcn_readfirstlane(m.bad)) return;
-        const int kact = __builtin_amdgcn_readfirstlane(m.kact);
+        const uint32_t code = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(g.code[h])));
+        const int kact = static_cast<int>(code >> 10);
         const int lane = static_cast<int>(threadIdx.x % 64), i = lane % 16, kq = lane / 16;
-        const float* row = g.xs + h * g.rs + __builtin_amdgcn_readfirstlane(m.first) + i + kq;
-        const int steps = (kact + 3) / 4;
-#pragma unroll 4
-        for (int s = 0; s < steps; s++) {
-            const float vc = row[4 * s + 16 * C0];
-            const float vr = R0 == C0 ? vc : row[4 * s + 16 * R0];
-            const float va = 4 * s + kq < kact ? vc : 0.0f;
-            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(va), static_cast<double>(vr), acc[0], 0, 0, 0);
-        }
-        if constexpr (LEN > 1) {
-            // R[16+i][16+j] - R[i][j] = sum over the entering minus the leaving terms
-            const int n = min(kact, 16), p0 = max(kact, 16);
-#pragma unroll 4
-            for (int s = 0; s < (n + 3) / 4; s++) {
-                const bool in = 4 * s + kq < n;
-                const float* lo = row + 4 * s;
-                const float* hi = lo + p0;
+        const float* x = g.xs + h * g.rs + static_cast<int>(code & 1023u) + i + kq;
+        int k = 0;
+        for (; k + 16 <= kact; k += 16, x += 16) {
+            float v[4][4];       // [step][row block] (unused ones drop out)
 #pragma unroll
-                for (int d = 1; d < LEN; d++) {
-                    const float hc = hi[16 * (C0 + d - 1)], hr = R0 == C0 ? hc : hi[16 * (R0 + d - 1)];
-                    const float lc = lo[16 * (C0 + d - 1)], lr = R0 == C0 ? lc : lo[16 * (R0 + d - 1)];
-                    acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(static_cast<double>(in ? hc : 0.0f),
-                                                                  static_cast<double>(hr), acc[d], 0, 0, 0);
-                    acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(-static_cast<double>(in ? lc : 0.0f),
-                                                                  static_cast<double>(lr), acc[d], 0, 0, 0);
-                }
-            }
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) v[u][r] = used(r) ? x[4 * u + 16 * r] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int b = 0; b < D::n; b++) acc[b] = mfma64(v[u][D::c[b]], v[u][D::r[b]], acc[b]);
         }
-        if (g.mean) {   // - K m m^T
+#pragma unroll 1
+        for (; k < kact; k += 4, x += 4) {
+            const bool in = k + kq < kact;
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; r++) v[r] = used(r) ? x[16 * r] : 0.0f;
+#pragma unroll
+            for (int b = 0; b < D::n; b++) acc[b] = mfma64(in ? v[D::c[b]] : 0.0f, v[D::r[b]], acc[b]);
+        }
+        if (g.mean && kact) {   // - K m m^T
             const float* mu = g.mean + h * g.mean_stride + i;
-            const double k = static_cast<double>(kact);
-            acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(kq == 0 ? -k * static_cast<double>(mu[16 * C0]) : 0.0,
-                                                          static_cast<double>(mu[16 * R0]), acc[0], 0, 0, 0);
 #pragma unroll
-            for (int d = 1; d < LEN; d++) {
-                const int e = kq == 0 ? d : d - 1;
-                const double f = kq == 0 ? -k : (kq == 1 ? k : 0.0);
-                acc[d] = __builtin_amdgcn_mfma_f64_16x16x4f64(f * static_cast<double>(mu[16 * (C0 + e)]),
-                                                              static_cast<double>(mu[16 * (R0 + e)]), acc[d], 0, 0, 0);
-            }
+            for (int b = 0; b < D::n; b++)
+                acc[b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    kq == 0 ? -static_cast<double>(kact) * static_cast<double>(mu[16 * D::c[b]]) : 0.0,
+                    static_cast<double>(mu[16 * D::r[b]]), acc[b], 0, 0, 0);
         }
+    }
+    static constexpr bool used(int r) {
+        for (int b = 0; b < D::n; b++)
+            if (D::r[b] == r || D::c[b] == r) return true;
+        return false;
     }
     // Stores (ADD: adds) the blocks to output matrix o.
     template <bool ADD>
     __device__ inline void store(const Gram& g, int o) const {
         const int lane = static_cast<int>(threadIdx.x % 64), i = lane % 16, e = lane / 16;
-        double4v sum = acc[0];
 #pragma unroll
-        for (int d = 0; d < LEN; d++) {
-            if (d > 0) sum += acc[d];
-            float* blk = g.mats + o * g.matrix + block_at(R0 + d, C0 + d);
+        for (int b = 0; b < D::n; b++) {
+            const bool diagonal = D::r[b] == D::c[b];
+            float* blk = g.mats + o * g.matrix + block_at(D::r[b], D::c[b]);
 #pragma unroll
             for (int v = 0; v < 4; v++) {
-                float* p = R0 == C0 ? blk + diag_chunk(v) + (i - 4 * v) * 4 + e : blk + v * 64 + i * 4 + e;
-                if (R0 != C0 || i >= 4 * v) *p = ADD ? static_cast<float>(static_cast<double>(*p) + sum[v]) : static_cast<float>(sum[v]);
+                float* p = diagonal ? blk + diag_chunk(v) + (i - 4 * v) * 4 + e : blk + v * 64 + i * 4 + e;
+                const float x = static_cast<float>(acc[b][v]);
+                if (!diagonal || i >= 4 * v) *p = ADD ? *p + x : x;
             }
         }
     }
 };
 
-// Window sums of the outputs [ta, ta + n) into matrices o, o + 1, ...; n <= 2T + 1.
-template <int R0, int C0, int LEN>
+// Window sums of the outputs [ta, ta + n) into matrices o, o + 1, ...; n <=
+// 2T + 1: the core of samples common to all windows and, output by output
+// downwards, what lies below it; then what lies above it, upwards.
+template <typename D>
 __device__ inline void window_sums(const Gram& g, int ta, int n, int o) {
-    Chain<R0, C0, LEN> c;
-    c.clear();
-    for (int tau = max(0, ta + n - 1 - g.T); tau <= min(g.n_d - 1, ta + g.T); tau++) c.add(g, tau);
-    c.template store<false>(g, o + n - 1);
+    Blocks<D> s;
+    s.clear();
+    for (int tau = max(0, ta + n - 1 - g.T); tau <= min(g.n_d - 1, ta + g.T); tau++) s.add(g, tau);
+    s.template store<false>(g, o + n - 1);
     for (int j = n - 2; j >= 0; j--) {
-        if (ta + j - g.T >= 0) c.add(g, ta + j - g.T);
-        c.template store<false>(g, o + j);
+        if (ta + j - g.T >= 0) s.add(g, ta + j - g.T);
+        s.template store<false>(g, o + j);
     }
-    c.clear();
+    s.clear();
     for (int j = 1; j < n; j++) {
-        if (ta + j + g.T < g.n_d) c.add(g, ta + j + g.T);   // else the window ends with the last sample
-        c.template store<true>(g, o + j);
+        if (ta + j + g.T < g.n_d) s.add(g, ta + j + g.T);   // else the window ends with the last sample
+        s.template store<true>(g, o + j);
     }
 }
 
@@ -183,36 +199,24 @@ template <int LMAX>
 __device__ inline void all_window_sums(const Gram& g, int t0, int n_out, int sub, int wave) {
     if constexpr (LMAX == 16) {
         for (int b = wave * sub; b < n_out; b += Cfg<LMAX>::kWaves * sub)
-            window_sums<0, 0, 1>(g, t0 + b, min(sub, n_out - b), b);
+            window_sums<Deal<16, 0>>(g, t0 + b, min(sub, n_out - b), b);
     } else {
         for (int b = 0; b < n_out; b += sub) {
             const int ta = t0 + b, n = min(sub, n_out - b);
-            if constexpr (LMAX == 32) {
-                if (wave == 0) window_sums<0, 0, 1>(g, ta, n, b);
-                else if (wave == 1) window_sums<1, 0, 1>(g, ta, n, b);
-                else window_sums<1, 1, 1>(g, ta, n, b);
-            } else {
-                if (wave == 0) {
-                    window_sums<0, 0, 3>(g, ta, n, b);
-                } else if (wave == 1) {
-                    window_sums<1, 0, 3>(g, ta, n, b);
-                } else if (wave == 2) {
-                    window_sums<2, 0, 2>(g, ta, n, b);
-                } else {
-                    window_sums<3, 0, 1>(g, ta, n, b);
-                    window_sums<3, 3, 1>(g, ta, n, b);
-                }
-            }
+            if (wave == 0) window_sums<Deal<LMAX, 0>>(g, ta, n, b);
+            else if (wave == 1) window_sums<Deal<LMAX, 1>>(g, ta, n, b);
+            else if (wave == 2) window_sums<Deal<LMAX, 2>>(g, ta, n, b);
+            else if constexpr (LMAX == 64) window_sums<Deal<64, 3>>(g, ta, n, b);
         }
     }
 }
 
 // ---- the solver: 16 lanes per system -------------------------------------------
 
-// a[k] += (lane k's l of this row of 16 lanes) * nl for k = START .. 15, one
+// a[k] -= (lane k's lk of this row of 16 lanes) * l for k = START .. 15, one
 // v_fmac_f32_dpp row_newbcast each.  The leading s_nop covers the two wait
-// states between a VALU write of l and its DPP read.
-#define SUPRA_FM(K) "v_fmac_f32_dpp %" #K ", %16, %17 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"
+// states between a VALU write of lk and its DPP read.
+#define SUPRA_FM(K) "v_fmac_f32_dpp %" #K ", %16, -%17 row_newbcast:" #K " row_mask:0xf bank_mask:0xf\n\t"
 #define SUPRA_FM_15 SUPRA_FM(15)
 #define SUPRA_FM_14 SUPRA_FM(14) SUPRA_FM_15
 #define SUPRA_FM_13 SUPRA_FM(13) SUPRA_FM_14
@@ -231,13 +235,13 @@ __device__ inline void all_window_sums(const Gram& g, int t0, int n_out, int sub
 #define SUPRA_FM_0 SUPRA_FM(0) SUPRA_FM_1
 
 template <int START>
-__device__ __attribute__((always_inline)) inline void fmac16(float* a, float l, float nl) {
+__device__ __attribute__((always_inline)) inline void fmac16(float* a, float lk, float l) {
 #define SUPRA_FM_CASE(S)                                                                                               \
     if constexpr (START == S)                                                                                         \
         asm("s_nop 1\n\t" SUPRA_FM_##S                                                                                \
             : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7]),         \
               "+v"(a[8]), "+v"(a[9]), "+v"(a[10]), "+v"(a[11]), "+v"(a[12]), "+v"(a[13]), "+v"(a[14]), "+v"(a[15])    \
-            : "v"(l), "v"(nl))
+            : "v"(lk), "v"(l))
     SUPRA_FM_CASE(0);
     SUPRA_FM_CASE(1);
     SUPRA_FM_CASE(2);
@@ -262,9 +266,12 @@ template <int N> __device__ inline float row_bcast(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + N, 0xf, 0xf, true));
 }
 
-template <typename T> __device__ inline T row_sum(T v) {
-#pragma unroll
-    for (int m = 8; m > 0; m >>= 1) v += __shfl_xor(v, m, 16);
+// Sum over each row of 16 lanes, in every lane (DPP row_ror 8, 4, 2, 1).
+__device__ inline float row_sum(float v) {
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xf, 0xf, true));
+    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xf, 0xf, true));
     return v;
 }
 
@@ -279,47 +286,65 @@ template <int LMAX> struct System {
     float a[kB][LMAX];       // row 16 r + q in slot r; entries beyond column 16 r + 15 unused
     double dd[kB];           // running diagonal of the slot's row
     float b1[kB], b2[kB];    // right-hand sides
+    float invg;              // 1 / pivot of the next step
 };
+
+// 1/sqrt of row J's diagonal, in every lane of the system.
+template <int LMAX, int J>
+__device__ __attribute__((always_inline)) inline float inverse_pivot(const System<LMAX>& s) {
+    return row_bcast<J % 16>(static_cast<float>(rsqrt64(s.dd[J / 16])));
+}
 
 // Elimination step J: column J scaled by 1/pivot, then subtracted from the
 // rows below.  Rows at or above the pivot take a zero multiplier; entries
-// right of a row's own column are its unused upper part.
+// right of a row's own column are its unused upper part.  The diagonals do
+// not wait for the rows' updates, so the next pivot's FP64 chain runs beside
+// them.
 template <int LMAX, int J>
 __device__ __attribute__((always_inline)) inline void eliminate(System<LMAX>& s, int q) {
     constexpr int rj = J / 16, qj = J % 16, kB = LMAX / 16;
-    const float invg = row_bcast<qj>(static_cast<float>(rsqrt64(s.dd[rj])));
-    const float z1 = row_bcast<qj>(s.b1[rj]) * invg;
-    const float z2 = row_bcast<qj>(s.b2[rj]) * invg;
-    float l[kB], nl[kB];
+    const float invg = s.invg;
+    float l[kB];
 #pragma unroll
     for (int r = rj; r < kB; r++) {
         l[r] = s.a[r][J] * invg;
         if (r == rj) l[r] = q > qj ? l[r] : 0.0f;
-        nl[r] = -l[r];
         s.dd[r] = fma(-static_cast<double>(l[r]), static_cast<double>(l[r]), s.dd[r]);
-        s.b1[r] = fmaf(nl[r], z1, s.b1[r]);
-        s.b2[r] = fmaf(nl[r], z2, s.b2[r]);
     }
+    if constexpr (J + 1 < LMAX) s.invg = inverse_pivot<LMAX, J + 1>(s);
+    const float z1 = row_bcast<qj>(s.b1[rj] * invg), z2 = row_bcast<qj>(s.b2[rj] * invg);
 #pragma unroll
     for (int r = rj; r < kB; r++) {
-        if constexpr (qj < 15) fmac16<(qj + 1) % 16>(&s.a[r][16 * rj], l[rj], nl[r]);
+        if constexpr (qj < 15) fmac16<(qj + 1) % 16>(&s.a[r][16 * rj], l[rj], l[r]);
 #pragma unroll
-        for (int c = rj + 1; c <= r; c++) fmac16<0>(&s.a[r][16 * c], l[c], nl[r]);
+        for (int c = rj + 1; c <= r; c++) fmac16<0>(&s.a[r][16 * c], l[c], l[r]);
+        // (a select, not the zero multiplier: a step past the system's last
+        // row may have a NaN pivot)
+        const float n1 = fmaf(-l[r], z1, s.b1[r]), n2 = fmaf(-l[r], z2, s.b2[r]);
+        s.b1[r] = r > rj || q > qj ? n1 : s.b1[r];
+        s.b2[r] = r > rj || q > qj ? n2 : s.b2[r];
     }
 }
 
+// Steps J .. LMAX-1; steps past the wave's largest system are left out four
+// at a time (they would change unused rows only).
 template <int LMAX, int J>
 __device__ __attribute__((always_inline)) inline void eliminate_from(System<LMAX>& s, int q, int nmax) {
     if constexpr (J < LMAX) {
-        if (J < nmax) eliminate<LMAX, J>(s, q);   // uniform
-        eliminate_from<LMAX, J + 1>(s, q, nmax);
+        if (J < nmax) {   // uniform
+            eliminate<LMAX, J>(s, q);
+            eliminate<LMAX, J + 1>(s, q);
+            eliminate<LMAX, J + 2>(s, q);
+            eliminate<LMAX, J + 3>(s, q);
+        }
+        eliminate_from<LMAX, J + 4>(s, q, nmax);
     }
 }
 
 // The samples of outputs [t0, t0 + n_out) of scanline s.
 template <int LMAX>
 __device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int n_out, int h_lo, const float* xs,
-                                     const SampleMeta* meta, const float* mats, int wave) {
+                                     const SampleMeta* meta, const float* mats, float2* res, int wave) {
     constexpr int kB = LMAX / 16;
     const int lane = static_cast<int>(threadIdx.x % 64), q = lane % 16;
     const int rs = static_cast<int>(a.rs);
@@ -353,62 +378,82 @@ __device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int
         }
         const float trace = row_sum(tr);
         const float delta = ((1.0f / static_cast<float>(n)) * trace) * a.alpha;
-        int bad = 0;
+        int bad = 0;             // a window with a bad sample: output 0
         for (int h = max(0, ht - static_cast<int>(a.T)); h <= min(static_cast<int>(a.n_d) - 1 - h_lo, ht + static_cast<int>(a.T)); h++)
             bad |= meta[h].bad;
 #pragma unroll
         for (int r = 0; r < kB; r++) {
             s.dd[r] = static_cast<double>(diag[r] + delta);
             s.b1[r] = 1.0f;
-            // sub-array sums x_i = sum_k x[f+k+i] (applyWeights, RxBeamformerMV.cu:342-376)
-            float acc = 0.0f;
-            const float* x = xs + ht * rs + m.first + 16 * r + q;
-            for (int k = 0; k < m.kact; k++) acc += x[k];
-            s.b2[r] = acc;
+            s.b2[r] = 0.0f;
         }
+        // sub-array sums x_i = sum_k x[f+k+i] (applyWeights, RxBeamformerMV.cu:342-376)
+        const float* x = xs + ht * rs + m.first + q;
+        int k = 0;
+        for (; k + 8 <= m.kact; k += 8, x += 8) {
+            float v[kB][8];
+#pragma unroll
+            for (int r = 0; r < kB; r++)
+#pragma unroll
+                for (int u = 0; u < 8; u++) v[r][u] = x[u + 16 * r];
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+#pragma unroll
+                for (int r = 0; r < kB; r++) s.b2[r] += v[r][u];
+        }
+        for (; k < m.kact; k++, x++)
+#pragma unroll
+            for (int r = 0; r < kB; r++) s.b2[r] += x[16 * r];
         int nmax = n;
 #pragma unroll
         for (int p = 16; p < 64; p += 16) nmax = max(nmax, __shfl_xor(nmax, p, 64));
+        s.invg = inverse_pivot<LMAX, 0>(s);
         eliminate_from<LMAX, 0>(s, q, __builtin_amdgcn_readfirstlane(nmax));
-        double zz = 0.0, uz = 0.0;
+        float zz = 0.0f, uz = 0.0f;
 #pragma unroll
         for (int r = 0; r < kB; r++) {
             // row 16 r + q's right-hand sides and diagonal are final
             const float ginv = static_cast<float>(rsqrt64(s.dd[r]));
             const float z = s.b1[r] * ginv, u = s.b2[r] * ginv;
             if (16 * r + q < n) {
-                zz += static_cast<double>(z) * static_cast<double>(z);
-                uz += static_cast<double>(u) * static_cast<double>(z);
+                zz = fmaf(z, z, zz);
+                uz = fmaf(u, z, uz);
             }
         }
         zz = row_sum(zz);
         uz = row_sum(uz);
-        float y = static_cast<float>(uz) / (static_cast<float>(zz) * powf(static_cast<float>(m.kact), a.p));
-        if (fabsf(y) > 1e7f || isnan(y) || bad) y = 0.0f;
-        if (q == 0 && o0 + lane / 16 < n_out) {
-            const uint64_t at = static_cast<uint64_t>(t) * a.n_rx + scan;
-            y *= static_cast<float>(a.n_ch);
-            if (a.out_i16) static_cast<int16_t*>(a.out)[at] = clamp_out<int16_t>(y);
-            else static_cast<float*>(a.out)[at] = clamp_out<float>(y);
-        }
+        if (q == 0 && o0 + lane / 16 < n_out) res[o] = make_float2(uz, bad ? 0.0f : zz);   // zz 0: output 0
+    }
+    __syncthreads();
+    // outputs: one lane each (the power and the division once per workgroup)
+    if (static_cast<int>(threadIdx.x) < n_out) {
+        const int t = t0 + static_cast<int>(threadIdx.x);
+        const float2 r = res[threadIdx.x];
+        const float kact = static_cast<float>(meta[t - h_lo].kact);
+        float y = r.x / (r.y * powf(kact, a.p));
+        if (!(fabsf(y) <= 1e7f) || r.y == 0.0f) y = 0.0f;
+        y *= static_cast<float>(a.n_ch);
+        const uint64_t at = static_cast<uint64_t>(t) * a.n_rx + scan;
+        if (a.out_i16) static_cast<int16_t*>(a.out)[at] = clamp_out<int16_t>(y);
+        else static_cast<float*>(a.out)[at] = clamp_out<float>(y);
     }
 }
 
 // Marks the samples whose covariance is not finite in single precision (e.g.
 // from a -FLT_MAX pre-delayed value): by Cauchy-Schwarz those with a
-// non-finite diagonal entry, which is at most the sample's energy.
+// non-finite diagonal entry.  Only samples that find_apertures marked kHuge
+// are looked at.  Also packs what the covariance needs of each sample.
 template <int LMAX>
-__device__ inline void find_bad(const MvArgs& a, const float* xs, const float* mean, int H, SampleMeta* meta) {
+__device__ inline void find_bad(const MvArgs& a, const float* xs, const float* mean, int H, SampleMeta* meta, uint32_t* code) {
     constexpr int kWaves = Cfg<LMAX>::kWaves;
     const int wave = static_cast<int>(threadIdx.x / 64), lane = static_cast<int>(threadIdx.x % 64);
-    const int n_ch = static_cast<int>(a.n_ch), rs = static_cast<int>(a.rs);
+    const int rs = static_cast<int>(a.rs);
     for (int h = wave; h < H; h += kWaves) {
-        float e = 0.0f;
-        for (int c = lane; c < n_ch; c += 64) e += xs[h * rs + c] * xs[h * rs + c];
-#pragma unroll
-        for (int m = 32; m > 0; m >>= 1) e += __shfl_xor(e, m, 64);
-        if (e <= 1e38f) continue;      // uniform
         const SampleMeta m = meta[h];
+        if (__builtin_amdgcn_readfirstlane(m.bad) == 0) {
+            if (lane == 0) code[h] = static_cast<uint32_t>(m.first) | static_cast<uint32_t>(m.kact) << 10;
+            continue;
+        }
         double r = 0.0;
         if (lane < m.lt) {
             for (int k = 0; k < m.kact; k++) {
@@ -420,7 +465,11 @@ __device__ inline void find_bad(const MvArgs& a, const float* xs, const float* m
                 r -= static_cast<double>(m.kact) * mu * mu;
             }
         }
-        if (__ballot(!(fabsf(static_cast<float>(r)) <= FLT_MAX)) != 0 && lane == 0) meta[h].bad = 1;
+        const uint64_t over = __ballot(!(fabsf(static_cast<float>(r)) <= FLT_MAX));
+        if (lane == 0) {
+            meta[h].bad = over != 0 ? 1 : 0;
+            code[h] = over != 0 ? 0u : static_cast<uint32_t>(m.first) | static_cast<uint32_t>(m.kact) << 10;
+        }
     }
 }
 
@@ -431,6 +480,7 @@ __device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t
     SampleMeta* meta = reinterpret_cast<SampleMeta*>(lds + a.off_meta);
     float* mean = a.means ? reinterpret_cast<float*>(lds + a.off_mean) : nullptr;
     float* mats = reinterpret_cast<float*>(lds + a.off_r);
+    float2* res = reinterpret_cast<float2*>(lds + a.off_wave);
     const uint32_t t0 = tile * a.tile, t1 = min(t0 + a.tile, a.n_d);
     const uint32_t h_lo = t0 >= a.T ? t0 - a.T : 0;
     const int H = static_cast<int>(min(a.n_d - 1, t1 - 1 + a.T) - h_lo + 1);
@@ -438,7 +488,7 @@ __device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t
 
     if (FUSED) stage_delayed<InT, kThreads>(a, lut, scan, h_lo, H, xs, lds);
     else stage_read<InT, kThreads>(a, scan, h_lo, H, xs);
-    find_apertures<kThreads>(a, xs, H, meta);
+    find_apertures<kThreads, true>(a, xs, H, meta);
     __syncthreads();
     if (mean) {
         for (int idx = threadIdx.x; idx < H * LMAX; idx += kThreads) {
@@ -453,11 +503,12 @@ __device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t
         }
         __syncthreads();
     }
-    find_bad<LMAX>(a, xs, mean, H, meta);
+    uint32_t* code = reinterpret_cast<uint32_t*>(lds + a.off_code);
+    find_bad<LMAX>(a, xs, mean, H, meta, code);
     __syncthreads();
     Gram g;
     g.xs = xs;
-    g.meta = meta;
+    g.code = code;
     g.mean = mean;
     g.mats = mats;
     g.rs = static_cast<int>(a.rs);
@@ -469,7 +520,7 @@ __device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t
     const int n_out = static_cast<int>(t1 - t0);
     all_window_sums<LMAX>(g, static_cast<int>(t0), n_out, static_cast<int>(a.sub), wave);
     __syncthreads();
-    solve_outputs<LMAX>(a, scan, static_cast<int>(t0), n_out, g.h_lo, xs, meta, mats, wave);
+    solve_outputs<LMAX>(a, scan, static_cast<int>(t0), n_out, g.h_lo, xs, meta, mats, res, wave);
 }
 
 // Renumbers the workgroups as mv_logical_wg in mv_kernels.hip does: 32
@@ -518,6 +569,10 @@ size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
     off += static_cast<size_t>(H) * sizeof(SampleMeta);
     a.off_mean = static_cast<uint32_t>(off);
     off += a.means ? static_cast<size_t>(H) * lmax * 4 : 0;
+    a.off_wave = static_cast<uint32_t>(off);     // (u.z, z.z) of the outputs
+    off += static_cast<size_t>(tile + 1) / 2 * 16;
+    a.off_code = static_cast<uint32_t>(off);
+    off += static_cast<size_t>(H + 3) / 4 * 16;
     a.off_r = static_cast<uint32_t>(off);
     // the pre-delay tables are only read before the matrices are written
     const size_t mats = static_cast<size_t>(tile) * (blocks * 160 + blocks * (blocks - 1) / 2 * 256) * 4;
@@ -532,14 +587,15 @@ uint32_t mv_block_lmax(uint32_t L) { return L <= 16 ? 16 : (L <= 32 ? 32 : 64); 
 
 bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds) {
     const uint32_t lmax = mv_block_lmax(a.L), w = 2 * a.T + 1;
-    // zero padding: the last 4-term step and the unused rows read past the aperture
+    // zero padding: the last step and the unused rows read past the aperture
     a.rs = a.n_ch + lmax + 4;
     // Of the tiles that fit, the one with the least modelled time per output:
-    // subs (w - 1) + tile covariance evaluations on the busiest wave (9 or 41
-    // matrix instructions of 64 cycles; the waves share them with 16 rows) and
-    // one round of 4 systems per wave.
+    // subs (w - 1) + tile covariance evaluations on the busiest wave (9 matrix
+    // instructions of 64 cycles with 32 rows, up to 51 with 64, fewer where the
+    // aperture is small; with 16 rows the waves share the outputs) and one
+    // round of 4 systems per wave.
     const uint32_t waves = lmax == 32 ? 3 : 4;
-    const double eval = lmax == 64 ? 2600.0 : (lmax == 32 ? 580.0 : 320.0);
+    const double eval = lmax == 64 ? 1400.0 : (lmax == 32 ? 580.0 : 320.0);
     const double solve = lmax == 64 ? 23000.0 : (lmax == 32 ? 6000.0 : 2000.0);
     double best = 0;
     uint32_t pick = 0;

@@ -310,7 +310,7 @@ __device__ __attribute__((always_inline)) inline void mv_tile(const MvArgs& a, c
     } else {
         stage_read<InT, kThreads>(a, s, h_lo, H, xs);
     }
-    find_apertures<kThreads>(a, xs, H, meta);
+    find_apertures<kThreads, false>(a, xs, H, meta);
     __syncthreads();
     if (MEANS) {
         for (int idx = threadIdx.x; idx < H * L; idx += kThreads) {

@@ -25,6 +25,7 @@ struct MvArgs {
     uint32_t pcg_iters;     // 0: Cholesky solve; else at most this many PCG iterations
     float pcg_threshold;    // PCG stops once |1 - R~ w| <= this
     int32_t block;          // planned for mv_block.hip (else mv_kernels.hip)
+    uint32_t off_code;      // mv_block.hip: LDS byte offset of the samples' packed apertures
     uint32_t sub;           // mv_block.hip: outputs per sub-block (at most 2T + 1)
     int32_t out_i16;        // mv_block.hip: int16 output (else float)
     DasArgs g;              // fused mode: geometry and RF of the pre-delay

@@ -127,27 +127,30 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
 }
 
 // Reads the pre-delayed samples of scanline s, depths [h_lo, h_lo + H), into
-// xs[h * rs + channel], zero for channels n_ch .. rs-1.  Batches of 8 loads
-// per lane are in flight before the LDS stores.
+// xs[h * rs + channel], zero for channels n_ch .. rs-1.  Half-waves take one
+// channel each (lanes = depths, no index division); 8 channels per half-wave
+// are in flight before the LDS stores.
 template <typename InT, int NT>
 __device__ inline void stage_read(const MvArgs& a, uint32_t s, uint32_t h_lo, int H, float* xs) {
-    const InT* xin = static_cast<const InT*>(a.x) + static_cast<uint64_t>(s) * a.n_ch * a.n_d;
-    constexpr int kBatch = 8;
-    const int rs = static_cast<int>(a.rs);
-    const int total = H * rs, n_ch = static_cast<int>(a.n_ch);
-    for (int base = 0; base < total; base += kBatch * NT) {
-        float v[kBatch];
+    const InT* xin = static_cast<const InT*>(a.x) + static_cast<uint64_t>(s) * a.n_ch * a.n_d + h_lo;
+    constexpr int kBatch = 8, kRows = NT / 32;
+    const int rs = static_cast<int>(a.rs), n_ch = static_cast<int>(a.n_ch);
+    const int hl = static_cast<int>(threadIdx.x % 32), cl = static_cast<int>(threadIdx.x / 32);
+    for (int h0 = 0; h0 < H; h0 += 32) {
+        const int h = h0 + hl;
+        if (h >= H) continue;
+        for (int c0 = cl; c0 < rs; c0 += kBatch * kRows) {
+            float v[kBatch];
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int idx = base + u * NT + static_cast<int>(threadIdx.x);
-            const int c = idx / H, h = idx % H;
-            v[u] = (idx < total && c < n_ch) ? in_f(xin[static_cast<uint64_t>(c) * a.n_d + h_lo + h]) : 0.0f;
-        }
+            for (int u = 0; u < kBatch; u++) {
+                const int c = c0 + u * kRows;
+                v[u] = c < n_ch ? in_f(xin[static_cast<uint64_t>(c) * a.n_d + h]) : 0.0f;
+            }
 #pragma unroll
-        for (int u = 0; u < kBatch; u++) {
-            const int idx = base + u * NT + static_cast<int>(threadIdx.x);
-            const int c = idx / H, h = idx % H;
-            if (idx < total) xs[h * rs + c] = v[u];
+            for (int u = 0; u < kBatch; u++) {
+                const int c = c0 + u * kRows;
+                if (c < rs) xs[h * rs + c] = v[u];
+            }
         }
     }
     __syncthreads();
@@ -156,16 +159,23 @@ __device__ inline void stage_read(const MvArgs& a, uint32_t s, uint32_t h_lo, in
 // First / last channel with a non-zero sample (0 when there is none), the
 // sub-array length and the number of active sub-arrays
 // (RxBeamformerMV.cu:44-113): one wave per sample, 64 channels per ballot.
-template <int NT>
+// `bad` is set to 0, or to kHuge for a sample with a NaN or a value whose
+// square may leave single precision.
+constexpr int32_t kHuge = 2;
+
+template <int NT, bool HUGE>
 __device__ inline void find_apertures(const MvArgs& a, const float* xs, int H, SampleMeta* meta) {
     const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
     const int n_ch = static_cast<int>(a.n_ch), L = static_cast<int>(a.L), rs = static_cast<int>(a.rs);
     for (int h = wv; h < H; h += NT / 64) {
         const float* row = xs + h * rs;
         int f = -1, l = 0;
+        bool huge = false;
         for (int cb = 0; cb < n_ch; cb += 64) {
             const int c = cb + ln;
-            const uint64_t nz = __ballot(c < n_ch && row[c] != 0.0f);
+            const float v = c < n_ch ? row[c] : 0.0f;
+            const uint64_t nz = __ballot(v != 0.0f);
+            if (HUGE) huge |= __ballot(!(fabsf(v) <= 5e17f)) != 0;   // 256 squares of it stay below 1e38
             if (nz != 0) {
                 if (f < 0) f = cb + __ffsll(static_cast<unsigned long long>(nz)) - 1;
                 l = cb + 63 - __clzll(static_cast<long long>(nz));
@@ -177,7 +187,7 @@ __device__ inline void find_apertures(const MvArgs& a, const float* xs, int H, S
             m.first = f;
             m.lt = min(L, l - f + 1);
             m.kact = min(static_cast<int>(a.K), l - f - m.lt + 2);
-            m.bad = 0;
+            m.bad = huge ? kHuge : 0;
             meta[h] = m;
         }
     }
