@@ -315,7 +315,7 @@ __global__ __launch_bounds__(256) void das2d_adjoint_kernel(const AdjointArgs a)
             const float fr = tau - static_cast<float>(i);
             const uint32_t ui = static_cast<uint32_t>(i);
             const float bw = bt * w;
-            const bool inr = take && ui < a.n_s - 1u;
+            const bool inr = take && ui < a.n_s - 1u && tau == tau;   // (a NaN delay converts to sample 0)
             const bool edge = take && ui == a.n_s - 1u && fr == 0.0f;
             float g0 = 0.0f, g1 = 0.0f;
             if (want_dc) {

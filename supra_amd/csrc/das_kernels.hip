@@ -101,7 +101,7 @@ __device__ inline Gather2D<RFT> gather2d_issue(__amdgpu_buffer_rsrc_t rf, uint32
         g.add = member & (tau >= 0.0f) & (tau <= last);
         g.edge = false;
     } else {
-        const bool inr = ui < n_s - 1u;
+        const bool inr = (ui < n_s - 1u) & (tau == tau);
         g.edge = (ui == n_s - 1u) & (g.f == 0.0f);
         g.add = member & (inr | g.edge);
     }
@@ -468,7 +468,7 @@ __device__ inline void elements2d_frames(const __amdgpu_buffer_rsrc_t (&rs)[FB],
 #pragma unroll
             for (int fb = 0; fb < FB; fb++) sample[fb] += w_eff * (omf * v0[fb] + f * v1[fb]);
         } else {
-            const bool inr = ui < n_s - 1u;
+            const bool inr = (ui < n_s - 1u) & (tau == tau);
             const bool edge = (ui == n_s - 1u) & (f == 0.0f);
             float v0[FB], v1[FB];
 #pragma unroll
@@ -618,10 +618,10 @@ __device__ inline Gather3D<RFT> gather3d_issue(__amdgpu_buffer_rsrc_t rf, uint32
     g.v1 = load_rf<RFT>(rf, off + ui + 1u);
     if constexpr (std::is_same_v<RFT, int16_t>) {
         const float last = static_cast<float>(n_s - 1u);
-        g.add = member & !(tau > last) & !(tau < (n_s > 1u ? -INFINITY : 0.0f));
+        g.add = member & (tau <= last) & !(tau < (n_s > 1u ? -INFINITY : 0.0f));
         g.edge = false;
     } else {
-        const bool inr = ui < n_s - 1u;
+        const bool inr = (ui < n_s - 1u) & (tau == tau);
         g.edge = (ui == n_s - 1u) & (g.f == 0.0f);
         g.add = member & (inr | g.edge);
     }

@@ -49,11 +49,11 @@ __device__ inline float interp_at(__amdgpu_buffer_rsrc_t rf, uint32_t off, uint3
     if constexpr (std::is_same_v<RFT, int16_t>) {
         const float last = static_cast<float>(n_s - 1u);
         bool in;
-        if constexpr (SAT_UINT) in = !(tau > last) & !(tau < (n_s > 1u ? -INFINITY : 0.0f));
+        if constexpr (SAT_UINT) in = (tau <= last) & !(tau < (n_s > 1u ? -INFINITY : 0.0f));
         else in = (tau >= 0.0f) & (tau <= last);
         return in ? ((1.0f - f) * v0 + f * v1) : 0.0f;
     } else {
-        const bool inr = ui < n_s - 1u;
+        const bool inr = (ui < n_s - 1u) & (tau == tau);
         const bool edge = (ui == n_s - 1u) & (f == 0.0f);
         return inr ? ((1.0f - f) * v0 + f * v1) : (edge ? v0 : 0.0f);
     }
