@@ -51,6 +51,11 @@ void build_dt_tables(supra_bf_ctx* ctx, double dt, double c) {
         ctx->h_ex[i] = static_cast<float>(ctx->ex_mm[i] * factor);
         ctx->h_ey[i] = static_cast<float>(ctx->ey_mm[i] * factor);
     }
+    ctx->grid_ok = ctx->is3d;
+    for (uint32_t e = 0; ctx->grid_ok && e < ctx->n_el; e++) {
+        const uint32_t ix = e % ctx->el_layout[0], iy = e / ctx->el_layout[0];
+        ctx->grid_ok = ctx->h_ex[e] == ctx->h_ex[ix] && ctx->h_ey[e] == ctx->h_ey[iy * ctx->el_layout[0]];
+    }
     auto connected = [&](uint32_t e) { return ctx->e2c.empty() || ctx->e2c[e] >= 0; };
     ctx->h_scans.resize(ctx->n_rx);
     for (uint32_t i = 0; i < ctx->n_rx; i++) {
@@ -226,6 +231,8 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
                 delete ctx;
                 return fail(SUPRA_ERR_INVALID_ARG, "create: scanline %u transmit %d aperture exceeds the array", i, k);
             }
+            if (t.last_active_element[1] > t.first_active_element[1])
+                ctx->max_rows = std::max<uint32_t>(ctx->max_rows, t.last_active_element[1] - t.first_active_element[1]);
             if (t.last_active_element[0] > t.first_active_element[0])
                 ctx->max_aperture = std::max<uint32_t>(ctx->max_aperture,
                                                        t.last_active_element[0] - t.first_active_element[0]);
@@ -350,6 +357,7 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
     a.c = static_cast<float>(speed_of_sound_mm_per_s);
     a.offset = static_cast<float>(additional_offset);
     a.far_ok = ctx->far_ok ? 1 : 0;
+    a.grid_ok = ctx->grid_ok && ctx->max_rows <= 32 ? 1 : 0;
     build_window_lut(window_type, window_parameter, a.lut);
 
     hipError_t e;

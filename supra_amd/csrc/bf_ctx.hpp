@@ -36,6 +36,8 @@ struct supra_bf_ctx {
     hipEvent_t tables_used = nullptr;
     bool tables_used_recorded = false;
     bool far_ok = false;   // dt-space depths are >= 0 and non-decreasing
+    bool grid_ok = false;     // 3D: dt-space element (ix, iy) is at (X[ix], Z[iy])
+    uint32_t max_rows = 0;    // 3D: largest last_y - first_y over scanlines and transmits
     bool far_ok_mm = false;   // the same for the millimetre depths (any c)
     std::mutex mu;
 

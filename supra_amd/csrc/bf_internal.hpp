@@ -62,6 +62,7 @@ struct DasArgs {
     float F, dt, c;             // fNumber, 1/fs, speed of sound [mm/s] as floats
     float offset;               // (float) additionalOffset
     int32_t max_aperture;       // unused (0)
+    int32_t grid_ok;            // 3D: element (ix, iy) is at (X[ix], Z[iy]), apertures of at most 32 rows
     int32_t far_ok;             // depth table is non-negative and non-decreasing
     // Per-frame geometry (one speed of sound per frame, 2D): strides between
     // the frames' tables (0: all frames share one table) and the per-frame c

@@ -865,6 +865,244 @@ __global__ __launch_bounds__(kThreads) void das3d_kernel(const DasArgs a) {
     }
 }
 
+// ---- 3D, separable element grid ---------------------------------------------
+//
+// A matrix probe's element (ex, ey) sits at (X[ex], Z[ey]): the delay's x part
+// depends on ex only, its z part and the z window index on ey only.  Where the
+// tables say so (grid_ok), the aperture has at most kGridY rows and every
+// element has a channel, the z parts of all rows stay in registers while the
+// columns go by, so an element costs two additions and a square root for its
+// delay and one byte-selecting addition for its near-field window weight.
+// The kernel is bound by VALU issue, so further work leaves the loop per wave:
+//  * far field: weights as in elements3d;
+//  * interior: when there is no additional offset and the first depth's lower
+//    and every lane's upper bound of the delay (the same roundings on the
+//    extreme operands, all of them monotone) lie in [0, N-1], no element needs
+//    the offset, a range test or a clamped floor;
+//  * a wave whose aperture rows all have a vertical distance above 0 needs no
+//    guard for a zero square root argument.
+// 32 x 32 probe, 64 x 64 x 1000 volume: 3.45 ms against 3.79 ms of
+// das3d_kernel (VALU 77 % busy, 22 to 28 instructions per element and pixel in
+// the interior).  112 registers leave four waves per SIMD; forcing five spills
+// (6.75 ms), and holding a second batch of gathers per wave was slower too
+// (7.5 ms).
+constexpr int kGridY = 32;      // aperture rows held in registers
+constexpr int kGridX = 32;      // aperture columns staged per LDS pass
+
+struct Grid3D {
+    float az2[kGridY];          // (Z[ey] - pz)^2
+    uint32_t iz4[kGridY / 4];   // near field: 4 x window index of four rows, one byte each
+};
+
+// Square root of a positive normal x (see sqrt_rn).
+__device__ inline float sqrt_pos(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+
+// Columns [0, nx) of the staged pass; `ex` and `off` of the first one.
+template <typename RFT, bool FAR, bool INTERIOR>
+__device__ inline void grid3d(__amdgpu_buffer_rsrc_t rf, const DasArgs& a, const TxDT& tx, const Pixel3D& p,
+                              const Grid3D& g, const float* s_r2, const float* s_w, const char* s_w2, const float* s_dx,
+                              uint32_t ex0, int nx, int ny, float& sample, float& wsum, int& nadd) {
+    const float last = static_cast<float>(a.n_s - 1u);
+    const uint32_t wrap = a.n_ch * a.n_s, row_step = (a.layout_x % a.n_ch) * a.n_s;
+    for (int x = 0; x < nx; x++) {
+        const float ax = load_uniform_float(a.ex, ex0 + x + tx.first_y * a.layout_x) - p.px;
+        const float ax2 = ax * ax;
+        const char* w2row = nullptr;
+        if (!FAR) w2row = s_w2 + window_index(s_dx[x] * p.invx) * kWindowEntries * 4;
+        uint32_t off = ((ex0 + x + tx.first_y * a.layout_x) % a.n_ch) * a.n_s;
+#pragma unroll
+        for (int b = 0; b < kGridY / 4; b++) {
+            if (4 * b < ny) {       // uniform
+                const float4 r2 = *reinterpret_cast<const float4*>(s_r2 + x * kGridY + 4 * b);
+                const float r2s[4] = {r2.x, r2.y, r2.z, r2.w};
+                bool member[4];
+                bool any = FAR;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    // (a row past the aperture is staged with an infinite distance)
+                    member[u] = FAR || r2s[u] <= p.aDT;
+                    any |= member[u];
+                }
+                uint32_t offs[4];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    offs[u] = off;
+                    off += row_step;
+                    off = off >= wrap ? off - wrap : off;
+                }
+                if (FAR || __builtin_amdgcn_ballot_w64(any) != 0) {     // uniform
+                    float ws[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (FAR) {
+                        const float4 w = *reinterpret_cast<const float4*>(s_w + x * kGridY + 4 * b);
+                        ws[0] = w.x, ws[1] = w.y, ws[2] = w.z, ws[3] = w.w;
+                    } else {
+#pragma unroll
+                        for (int u = 0; u < 4; u++) {
+                            const float w = *reinterpret_cast<const float*>(w2row + ((g.iz4[b] >> (8 * u)) & 0xffu));
+                            ws[u] = member[u] ? w : 0.0f;
+                        }
+                    }
+                    float f[4], v0[4], v1[4];
+                    bool add[4], edge[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        const float q = (ax2 + g.az2[4 * b + u]) + p.py2;
+                        float tau = tx.t0 + ((FAR ? sqrt_pos(q) : sqrt_rn(q)) + p.d);
+                        if (!INTERIOR) tau = tau + a.offset;
+                        uint32_t ui;
+                        if (INTERIOR) {
+                            ui = static_cast<uint32_t>(tau);
+                            f[u] = __builtin_amdgcn_fractf(tau);
+                            add[u] = true;
+                        } else {
+                            const float fl = fmaxf(floorf(tau), 0.0f);
+                            ui = static_cast<uint32_t>(fl);
+                            f[u] = tau - fl;
+                            add[u] = (tau <= last) & !(tau < (a.n_s > 1u ? -INFINITY : 0.0f));
+                        }
+                        v0[u] = load_rf<RFT>(rf, ui + offs[u]);
+                        v1[u] = load_rf<RFT>(rf, ui + offs[u] + 1u);
+                        if (std::is_same_v<RFT, float>) {
+                            edge[u] = (ui == a.n_s - 1u) & (f[u] == 0.0f);
+                            add[u] = (INTERIOR || ((ui < a.n_s - 1u) & (tau == tau)) || edge[u]) &&
+                                     (FAR ? 4 * b + u < ny : member[u]);
+                        }
+                    }
+#pragma unroll
+                    for (int u = 0; u < 4; u++) {
+                        wsum += ws[u];
+                        if (!FAR) nadd += member[u] ? 1 : 0;
+                        if constexpr (std::is_same_v<RFT, int16_t>) {
+                            // outside its aperture an element has weight 0 and adds +-0
+                            const float contrib = ws[u] * ((1.0f - f[u]) * v0[u] + f[u] * v1[u]);
+                            sample += INTERIOR || add[u] ? contrib : 0.0f;
+                        } else {
+                            const float val = edge[u] ? v0[u] : ((1.0f - f[u]) * v0[u] + f[u] * v1[u]);
+                            const float contrib = ws[u] * val;
+                            sample = add[u] ? sample + contrib : sample;
+                        }
+                    }
+                }
+            }
+        }
+        if (FAR) nadd += ny;
+    }
+}
+
+template <typename RFT, typename OutT, bool INTERP_TX>
+__global__ __launch_bounds__(kThreads, 4) void das3d_grid_kernel(const DasArgs a) {
+    __shared__ __align__(16) float s_w2[kW2Entries];
+    __shared__ __align__(16) float s_r2[kGridX * kGridY];
+    __shared__ __align__(16) float s_w[kGridX * kGridY];
+    __shared__ float s_dx[kGridX];
+
+    const uint32_t lb = logical_wg_2d(a.depth_tiles);
+    if (lb >= a.depth_tiles * a.n_rx * a.n_frames) return;   // whole workgroup
+    const Tile t = decode_tile(a, lb);
+    for (int i = threadIdx.x; i < kW2Entries; i += kThreads)
+        s_w2[i] = sqrtf(a.lut[i / kWindowEntries] * a.lut[i % kWindowEntries]);
+
+    const ScanView sc = scan_view(a.scans, t.s);
+    Pixel3D p;
+    p.d = t.valid ? a.depths[t.r] : 0.0f;
+    {
+        const float ap = (((p.d * a.dt) * a.c) / (2.0f * a.F)) / a.c / a.dt;
+        p.aDT = ap * ap;
+        const float sq = sqrtf(p.aDT);
+        p.invx = 1.0f / fminf(sq, sc.max_ed_x());
+        p.invz = 1.0f / fminf(sq, sc.max_ed_y());
+    }
+    p.px = sc.x() + sc.dir_x() * p.d;
+    p.pz = sc.z() + sc.dir_z() * p.d;
+    {
+        const float py = sc.dir_y() * p.d;
+        p.py2 = py * py;
+    }
+    // far-field test per wave, at the wave's first (smallest) depth
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64)));
+    const float d0 = load_uniform_float(a.depths, min(t.r0 + wave * 64u, a.n_depths - 1u));
+    const float ap0 = (((d0 * a.dt) * a.c) / (2.0f * a.F)) / a.c / a.dt;
+    const float aDT0 = ap0 * ap0;
+    const float sq0 = sqrtf(aDT0);
+    const float invx_far = 1.0f / sc.max_ed_x(), invz_far = 1.0f / sc.max_ed_y();
+
+    const RFT* rf_frame = static_cast<const RFT*>(a.rf) + static_cast<uint64_t>(t.frame) * a.rf_frame_stride;
+    float s_interp = 0.0f;
+
+    for (int k = 0; k < 4; k++) {
+        const bool use = INTERP_TX ? ((sc.active_mask() >> k) & 1) != 0 : (k == sc.sel());
+        if (!use) continue;
+        const TxDT tx = sc.tx(k);
+        const RFT* rf_tx = rf_frame + static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
+        const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
+        const int ny = (tx.last_y > tx.first_y) ? tx.last_y - tx.first_y : 0;
+        const int nx = (tx.last_x > tx.first_x) ? tx.last_x - tx.first_x : 0;
+        float sample = 0.0f, wsum = 0.0f;
+        int nadd = 0;
+        if (nx > 0 && ny > 0) {
+            // z parts of the rows, and the largest x and z parts of this pixel
+            Grid3D g;
+            float z2max = 0.0f, x2max = 0.0f;
+#pragma unroll
+            for (int b = 0; b < kGridY / 4; b++) {
+                uint32_t pack = 0;
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int y = min(4 * b + u, ny - 1);
+                    const float ze = load_uniform_float(a.ey, tx.first_x + (tx.first_y + y) * a.layout_x);
+                    const float az = ze - p.pz;
+                    g.az2[4 * b + u] = az * az;
+                    z2max = fmaxf(z2max, az * az);
+                    pack |= static_cast<uint32_t>(window_index((ze - sc.z()) * p.invz) * 4) << (8 * u);
+                }
+                g.iz4[b] = pack;
+            }
+            for (int x = 0; x < nx; x++) {
+                const float ax = load_uniform_float(a.ex, tx.first_x + x + tx.first_y * a.layout_x) - p.px;
+                x2max = fmaxf(x2max, ax * ax);
+            }
+            const float hi = tx.t0 + (sqrt_rn((x2max + z2max) + p.py2) + p.d);
+            const bool interior = a.far_ok && a.offset == 0.0f && tx.t0 + d0 >= 0.0f &&
+                                  __builtin_amdgcn_ballot_w64(!(hi <= static_cast<float>(a.n_s - 1u))) == 0;
+            const bool far = a.far_ok && aDT0 >= tx.far_thr && sq0 >= sc.max_ed_x() && sq0 >= sc.max_ed_y() &&
+                             __builtin_amdgcn_ballot_w64(!(p.py2 >= 1e-20f) && t.valid) == 0;
+            for (int base = 0; base < nx; base += kGridX) {
+                const int cx = min(kGridX, nx - base);
+                __syncthreads();
+                for (int j = threadIdx.x; j < cx * kGridY; j += kThreads) {
+                    const int x = j / kGridY, y = j % kGridY;
+                    const uint32_t e = tx.first_x + base + x + (tx.first_y + min(y, ny - 1)) * a.layout_x;
+                    const float dx = a.ex[e] - sc.x(), dz = a.ey[e] - sc.z();
+                    s_r2[j] = y < ny ? dx * dx + dz * dz : INFINITY;
+                    s_w[j] = y < ny ? s_w2[window_index(dx * invx_far) * kWindowEntries + window_index(dz * invz_far)] : 0.0f;
+                    if (y == 0) s_dx[x] = dx;
+                }
+                __syncthreads();
+                const uint32_t ex0 = tx.first_x + base;
+                const char* w2 = reinterpret_cast<const char*>(s_w2);
+                if (far) {
+                    if (interior) grid3d<RFT, true, true>(rsrc, a, tx, p, g, s_r2, s_w, w2, s_dx, ex0, cx, ny, sample, wsum, nadd);
+                    else grid3d<RFT, true, false>(rsrc, a, tx, p, g, s_r2, s_w, w2, s_dx, ex0, cx, ny, sample, wsum, nadd);
+                } else {
+                    if (interior) grid3d<RFT, false, true>(rsrc, a, tx, p, g, s_r2, s_w, w2, s_dx, ex0, cx, ny, sample, wsum, nadd);
+                    else grid3d<RFT, false, false>(rsrc, a, tx, p, g, s_r2, s_w, w2, s_dx, ex0, cx, ny, sample, wsum, nadd);
+                }
+            }
+        }
+        const float s_local = (nadd > 0) ? (sample / wsum) * static_cast<float>(nadd) : 0.0f;
+        if (INTERP_TX) s_interp += sc.txw(k) * s_local;
+        else s_interp += s_local;
+    }
+    if (t.valid) {
+        OutT* out = static_cast<OutT*>(a.out) + static_cast<uint64_t>(t.frame) * a.out_frame_stride;
+        out[static_cast<uint64_t>(t.r) * a.n_rx + t.s] = clamp_cast<OutT>(s_interp);
+    }
+}
+
 // ---- RawDelay (2D) -----------------------------------------------------------
 
 // rxDelayDTSPACEKernel + sampleDelay2D (src/SupraLib/Beamformer/RawDelay.cu:221-312,
@@ -1144,7 +1382,10 @@ static hipError_t launch_typed(const DasArgs& a, bool is3d, bool testsig, bool i
             else hipLaunchKernelGGL((KERNEL<RFT, OutT, false, false, false>), grid, block, 0, stream, a);           \
         }                                                                                                           \
     } while (0)
-    if (is3d) {
+    if (is3d && a.grid_ok && !testsig && !map) {
+        if (interp_tx) hipLaunchKernelGGL((das3d_grid_kernel<RFT, OutT, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((das3d_grid_kernel<RFT, OutT, false>), grid, block, 0, stream, a);
+    } else if (is3d) {
         SUPRA_DAS_DISPATCH(das3d_kernel);
     } else if (!testsig && !interp_tx && a.n_frames >= 2 && a.scan_frame_stride == 0 && a.depth_frame_stride == 0 &&
                a.el_frame_stride == 0 && a.frame_c == nullptr && a.norm_out == nullptr) {
