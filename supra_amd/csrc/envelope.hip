@@ -6,18 +6,29 @@
 //   LogCompressor (src/SupraLib/Beamformer/LogCompressor.cu:20-64,
 //     LogCompressorNode.cpp:42-45).
 //
-// Envelope layout: one workgroup of 4 waves per (64 scanlines, 32 output
-// samples, frame) of images [frame][sample][scanline]; lane = scanline, so
-// every row of the window is one coalesced 256-byte load.  The workgroup
-// stages the column window (32 + N - 1 rows) in LDS, loads issued eight
-// rows at a time per wave before they are written, and each wave then
-// computes every fourth output row from LDS.  Samples outside the image are
-// staged as 0, which adds +-0 to the FIR sum where the reference skips them
-// (the same value).  The FIR sum runs over the taps in ascending order in
-// single precision without contraction, as the host restatement does, so
-// the envelope is bit for bit the oracle's.  The fused variant applies the
-// log compression to the float envelope in registers (the same operations
-// as the two-step path with a float intermediate).
+// Envelope layout: one workgroup per (64 scanlines, ROWS output samples,
+// frame) of images [frame][sample][scanline]; lane = scanline, so every row of
+// the window is one coalesced 256-byte load.  The workgroup stages the column
+// window (ROWS + N - 1 rows) in LDS, loads issued eight rows at a time per
+// wave before they are written.  Samples outside the image are staged as 0,
+// which adds +-0 to the FIR sum where the reference skips them (the same
+// value).  The FIR sum runs over the taps in ascending order in single
+// precision without contraction, as the host restatement does, so the envelope
+// is bit for bit the oracle's.
+//
+// Every second tap of a Hilbert transformer is 0.  It adds +-0 to the sum of a
+// window of finite samples, so it is left out there: a lane takes 8 output
+// rows of one parity, reads each input row of the other parity once and adds
+// it to the up to 8 sums it belongs to, half the multiplications and a sixth
+// of the LDS reads of a sum per row.  A workgroup whose window holds an
+// infinity or a NaN (0 times it is NaN), and filters whose other taps are not
+// all 0, sum every tap.  Bound by VALU: 64 multiplications and additions of a
+// 65-tap filter per sample, about as many instructions again for the square
+// root and the logarithm.  32 frames of 2080 x 128 to uint8: 28.3 us, 48.1 us with
+// every tap and one sum per row.  ROWS is 64 where that leaves at least two
+// workgroups per CU (fewer halo rows staged per output), else 32.  The fused
+// variant applies the log compression to the float envelope in registers (the
+// same operations as the two-step path with a float intermediate).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -32,8 +43,8 @@
 namespace supra_amd {
 namespace {
 
-constexpr int kEnvRows = 32;          // output samples per workgroup
-constexpr int kEnvWaves = 4;          // waves per workgroup
+constexpr int kEnvOut = 8;            // output rows per lane, every second row of 16
+constexpr int kEnvPadRows = 14;       // zero rows after the window: padded taps read them
 constexpr int kMaxTaps = 257;         // HilbertFirEnvelopeNode's filterLength range (1..257)
 
 struct EnvArgs {
@@ -41,8 +52,10 @@ struct EnvArgs {
     void* out;
     uint32_t n_rx, n_s, n_taps, half;  // half = n_taps / 2 (window t - half .. t + half)
     uint32_t used_taps;               // taps that exist: min(n_taps, 2 half + 1)
+    uint32_t parity, groups;          // taps parity, parity + 2, ... as groups of 8 in odd[]; groups 0: sum every tap
     float in_scale, scale_den;        // log compression (fused variant)
     float h[kMaxTaps];
+    float odd[(kMaxTaps + 1) / 2 + 8];   // zero padded to whole groups
 };
 
 struct LogArgs {
@@ -72,21 +85,42 @@ __device__ inline float log_compress(float a, float in_scale, float scale_den) {
     return log10f(fabsf(a) * in_scale + 1.0f) * scale_den;
 }
 
-template <typename InT, typename OutT, bool LOG>
-__global__ __launch_bounds__(64 * kEnvWaves) void envelope_kernel(const EnvArgs a) {
-    extern __shared__ float win[];                 // [32 + 2 half rows][64 lanes]
-    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+// Correctly rounded sqrt(x) of a finite x >= 2^-96 by one Newton step, as
+// sqrt_rn in das_device.hpp; sqrtf where a lane of the wave has another x.
+__device__ inline float wave_sqrt(float x) {
+    if (__builtin_amdgcn_ballot_w64(!(x >= 0x1p-96f && x <= FLT_MAX)) != 0) return sqrtf(x);
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+
+template <typename OutT, bool LOG>
+__device__ inline void store_envelope(const EnvArgs& a, OutT* out, uint64_t at, float v, float acc) {
+    float env = wave_sqrt(v * v + acc * acc);
+    // the fused path sees the envelope as the float image the two-node
+    // chain passes on: clampCast<float> first (NaN -> -FLT_MAX, inf -> FLT_MAX)
+    if (LOG) env = log_compress(clamp_to<float>(env), a.in_scale, a.scale_den);
+    out[at] = clamp_to<OutT>(env);
+}
+
+template <typename InT, typename OutT, bool LOG, int ROWS>
+__global__ __launch_bounds__(ROWS * 8) void envelope_kernel(const EnvArgs a) {
+    constexpr uint32_t kWaves = ROWS / 8;
+    extern __shared__ float win[];                 // [ROWS + 2 half + kEnvPadRows rows][64 lanes]
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6)));
     const uint32_t s = blockIdx.x * 64u + lane;
-    const uint32_t t0 = blockIdx.y * kEnvRows;
+    const uint32_t t0 = blockIdx.y * ROWS;
     const uint64_t frame = static_cast<uint64_t>(blockIdx.z) * a.n_s * a.n_rx;
-    const uint32_t rows = kEnvRows + 2u * a.half;
+    const uint32_t rows = ROWS + 2u * a.half, staged = rows + kEnvPadRows;
     const bool col = s < a.n_rx;
     const InT* in = static_cast<const InT*>(a.in) + frame;
-    for (uint32_t r0 = wave; r0 < rows; r0 += 8u * kEnvWaves) {
+    bool odd_value = false;                        // a staged value that is not finite
+    for (uint32_t r0 = wave; r0 < staged; r0 += 8u * kWaves) {
         float v[8];
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const uint32_t r = r0 + u * kEnvWaves;
+            const uint32_t r = r0 + u * kWaves;
             const int64_t c = static_cast<int64_t>(t0) + r - a.half;
             v[u] = 0.0f;
             if (r < rows && col && c >= 0 && c < static_cast<int64_t>(a.n_s))
@@ -94,25 +128,68 @@ __global__ __launch_bounds__(64 * kEnvWaves) void envelope_kernel(const EnvArgs 
         }
 #pragma unroll
         for (int u = 0; u < 8; u++) {
-            const uint32_t r = r0 + u * kEnvWaves;
-            if (r < rows) win[r * 64u + lane] = v[u];
+            const uint32_t r = r0 + u * kWaves;
+            if (r < staged) win[r * 64u + lane] = v[u];
+            if (sizeof(InT) == 4) odd_value |= !(fabsf(v[u]) <= FLT_MAX);
         }
     }
-    __syncthreads();
-    if (!col) return;
+    const bool every_tap = __syncthreads_or(odd_value) || a.groups == 0;
     OutT* out = static_cast<OutT*>(a.out) + frame;
-    for (uint32_t i = wave; i < kEnvRows; i += kEnvWaves) {
-        const uint32_t t = t0 + i;
-        if (t >= a.n_s) break;
-        float acc = 0.0f;
+    if (every_tap) {
+        if (!col) return;
+        for (uint32_t i = wave; i < ROWS; i += kWaves) {
+            const uint32_t t = t0 + i;
+            if (t >= a.n_s) break;
+            float acc = 0.0f;
 #pragma unroll 8
-        for (uint32_t j = 0; j < a.used_taps; j++) acc += win[(i + j) * 64u + lane] * a.h[j];
-        const float v = win[(i + a.half) * 64u + lane];
-        float env = sqrtf(v * v + acc * acc);
-        // the fused path sees the envelope as the float image the two-node
-        // chain passes on: clampCast<float> first (NaN -> -FLT_MAX, inf -> FLT_MAX)
-        if (LOG) env = log_compress(clamp_to<float>(env), a.in_scale, a.scale_den);
-        out[static_cast<uint64_t>(t) * a.n_rx + s] = clamp_to<OutT>(env);
+            for (uint32_t j = 0; j < a.used_taps; j++) acc += win[(i + j) * 64u + lane] * a.h[j];
+            store_envelope<OutT, LOG>(a, out, static_cast<uint64_t>(t) * a.n_rx + s, win[(i + a.half) * 64u + lane], acc);
+        }
+        return;
+    }
+    // output rows i0 + 2 m; tap parity + 2 q of row i0 + 2 m is window row
+    // i0 + parity + 2 (m + q)
+    const uint32_t i0 = (wave >> 1) * 16u + (wave & 1u);
+    const float* x = win + (i0 + a.parity) * 64u + lane;
+    float acc[kEnvOut], hp[8], hc[8];
+#pragma unroll
+    for (int m = 0; m < kEnvOut; m++) acc[m] = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 8; q++) hc[q] = a.odd[q];
+#pragma unroll
+    for (int i = 0; i < 8; i++) {                  // rows m + q = 0 .. 7
+        const float v = x[i * 128];
+#pragma unroll
+        for (int m = 0; m <= i; m++) acc[m] += v * hc[i - m];
+    }
+    for (uint32_t g = 1; g < a.groups; g++) {
+        x += 8 * 128;
+#pragma unroll
+        for (int q = 0; q < 8; q++) {
+            hp[q] = hc[q];
+            hc[q] = a.odd[8 * g + q];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            const float v = x[i * 128];
+#pragma unroll
+            for (int m = 0; m < kEnvOut; m++) acc[m] += v * (i >= m ? hc[(i - m) & 7] : hp[(8 + i - m) & 7]);
+        }
+    }
+    x += 8 * 128;
+#pragma unroll
+    for (int i = 0; i < 7; i++) {
+        const float v = x[i * 128];
+#pragma unroll
+        for (int m = i + 1; m < kEnvOut; m++) acc[m] += v * hc[8 + i - m];
+    }
+    if (!col) return;
+#pragma unroll
+    for (int m = 0; m < kEnvOut; m++) {
+        const uint32_t t = t0 + i0 + 2 * m;
+        if (t < a.n_s)                             // uniform
+            store_envelope<OutT, LOG>(a, out, static_cast<uint64_t>(t) * a.n_rx + s,
+                                      win[(i0 + 2 * m + a.half) * 64u + lane], acc[m]);
     }
 }
 
@@ -160,8 +237,16 @@ int check_types(const char* what, int in_dtype, int out_dtype, bool allow_u8_in,
 }
 
 template <bool LOG, typename InT, typename OutT>
-void launch_env_typed(const EnvArgs& a, dim3 grid, size_t lds, hipStream_t s) {
-    hipLaunchKernelGGL((envelope_kernel<InT, OutT, LOG>), grid, dim3(64 * kEnvWaves), lds, s, a);
+void launch_env_typed(const EnvArgs& a, uint32_t n_frames, hipStream_t s) {
+    const uint32_t columns = (a.n_rx + 63) / 64;
+    const size_t window = static_cast<size_t>(2 * a.half + kEnvPadRows);
+    // tall tiles where at least 512 workgroups (two per CU) remain
+    if (static_cast<uint64_t>(columns) * ((a.n_s + 63) / 64) * n_frames >= 512)
+        hipLaunchKernelGGL((envelope_kernel<InT, OutT, LOG, 64>), dim3(columns, (a.n_s + 63) / 64, n_frames), dim3(512),
+                           (64 + window) * 256, s, a);
+    else
+        hipLaunchKernelGGL((envelope_kernel<InT, OutT, LOG, 32>), dim3(columns, (a.n_s + 31) / 32, n_frames), dim3(256),
+                           (32 + window) * 256, s, a);
 }
 
 template <bool LOG>
@@ -188,18 +273,24 @@ int launch_envelope(const char* what, const void* image, int in_dtype, uint32_t 
     a.in_scale = in_scale;
     a.scale_den = scale_den;
     hilbert_taps(filter_length, a.h);
-    const dim3 grid((n_rx + 63) / 64, (n_s + kEnvRows - 1) / kEnvRows, n_frames);
-    if (grid.y > 65535u) return fail(SUPRA_ERR_TOO_LARGE, "%s: too many samples per scanline", what);
-    const size_t lds = static_cast<size_t>(kEnvRows + 2 * a.half) * 64 * sizeof(float);
+    a.parity = ((filter_length - 1) / 2 + 1) % 2;
+    bool halved = filter_length > 1;
+    for (uint32_t j = 0; j < a.used_taps; j++) {
+        if (j % 2 == a.parity) a.odd[j / 2] = a.h[j];
+        else halved = halved && a.h[j] == 0.0f;
+    }
+    const uint32_t n_odd = a.used_taps > a.parity ? (a.used_taps - a.parity + 1) / 2 : 0;
+    a.groups = halved ? (n_odd + 7) / 8 : 0;
+    if ((n_s + 31) / 32 > 65535u) return fail(SUPRA_ERR_TOO_LARGE, "%s: too many samples per scanline", what);
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (in_dtype == SUPRA_INT16) {
-        if (out_dtype == SUPRA_FLOAT32) launch_env_typed<LOG, int16_t, float>(a, grid, lds, s);
-        else if (out_dtype == SUPRA_INT16) launch_env_typed<LOG, int16_t, int16_t>(a, grid, lds, s);
-        else launch_env_typed<LOG, int16_t, uint8_t>(a, grid, lds, s);
+        if (out_dtype == SUPRA_FLOAT32) launch_env_typed<LOG, int16_t, float>(a, n_frames, s);
+        else if (out_dtype == SUPRA_INT16) launch_env_typed<LOG, int16_t, int16_t>(a, n_frames, s);
+        else launch_env_typed<LOG, int16_t, uint8_t>(a, n_frames, s);
     } else {
-        if (out_dtype == SUPRA_FLOAT32) launch_env_typed<LOG, float, float>(a, grid, lds, s);
-        else if (out_dtype == SUPRA_INT16) launch_env_typed<LOG, float, int16_t>(a, grid, lds, s);
-        else launch_env_typed<LOG, float, uint8_t>(a, grid, lds, s);
+        if (out_dtype == SUPRA_FLOAT32) launch_env_typed<LOG, float, float>(a, n_frames, s);
+        else if (out_dtype == SUPRA_INT16) launch_env_typed<LOG, float, int16_t>(a, n_frames, s);
+        else launch_env_typed<LOG, float, uint8_t>(a, n_frames, s);
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(SUPRA_ERR_HIP, "%s: launch: %s", what, hipGetErrorString(e));
