@@ -20,8 +20,9 @@
 // The tables live in HBM: per pixel a uint32 sample index (0xffffffff
 // outside the scan) and two (2D) or three (3D) float weights.
 //
-// Conversion (supra_scanconv_run): one lane per output pixel, x fastest;
-// each lane reads its table entry once and converts `num_frames` frames
+// Conversion (supra_scanconv_run): 2D in tiles of 64 x 16 output pixels from
+// LDS, 3D one to four output pixels per lane, x fastest; each lane reads its
+// table entries once and converts `num_frames` frames
 // (scanConvert2D :350-381, scanConvert3D :384-428), clampCast to the output
 // type.  Arithmetic is the reference's expression, in float, unfused.
 //
@@ -256,6 +257,8 @@ struct ConvArgs {
     uint64_t in_frame;      // elements per input frame (n_samples * n_rx)
     uint32_t n_rx_x, n_rx;
     uint32_t num_frames;
+    uint32_t size_x, size_y;         // 2D: pixels of a row, rows
+    uint32_t frames_per_group;       // 2D: frames of one workgroup
 };
 
 template <typename T> __device__ inline float in_at(const T* p, uint64_t i) { return static_cast<float>(p[i]); }
@@ -270,14 +273,14 @@ template <> __device__ inline uint8_t clamp_out<uint8_t>(float x) {
     return static_cast<uint8_t>(fminf(fmaxf(x, 0.0f), 255.0f));
 }
 
-// V pixels per thread, consecutive in the output: V = 4 stores each frame's
+// 3D: V pixels per thread, consecutive in the output: V = 4 stores each frame's
 // 4 pixels with one packed store; the host takes it when the pixel count is a
 // multiple of 4 and the output is aligned to the packed size.
 template <typename OutT, int V> struct alignas(V * sizeof(OutT)) OutPack {
     OutT v[V];
 };
 
-template <typename InT, typename OutT, bool IS3D, int V>
+template <typename InT, typename OutT, int V>
 __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
     const uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * V;
     if (i0 >= a.n_pixels) return;
@@ -289,11 +292,10 @@ __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
         const uint64_t i = i0 + v;
         const uint32_t s32 = a.idx[i];
         s[v] = s32;
-        // the last sample row has no successor: the reference's 3D guard, used in 2D too
-        valid[v] = s32 != kOutside && (IS3D ? s[v] + 1 + nx + n : s[v] + 1 + n) < a.in_frame;
+        valid[v] = s32 != kOutside && s[v] + 1 + nx + n < a.in_frame;
         wx[v] = valid[v] ? a.wx[i] : 0.0f;
         wy[v] = valid[v] ? a.wy[i] : 0.0f;
-        wz[v] = (IS3D && valid[v]) ? a.wz[i] : 0.0f;
+        wz[v] = valid[v] ? a.wz[i] : 0.0f;
     }
     const InT* in = static_cast<const InT*>(a.in);
     OutT* out = static_cast<OutT*>(a.out);
@@ -303,16 +305,11 @@ __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
             float val = 0.0f;
             if (valid[v]) {
                 const uint64_t q = s[v];
-                if (!IS3D) {
-                    val = (1 - wy[v]) * ((1 - wx[v]) * in_at(in, q) + wx[v] * in_at(in, q + 1)) +
-                          wy[v] * ((1 - wx[v]) * in_at(in, q + n) + wx[v] * in_at(in, q + 1 + n));
-                } else {
-                    val = (1 - wy[v]) * ((1 - wz[v]) * ((1 - wx[v]) * in_at(in, q) + wx[v] * in_at(in, q + 1)) +
-                                         wz[v] * ((1 - wx[v]) * in_at(in, q + nx) + wx[v] * in_at(in, q + 1 + nx))) +
-                          wy[v] * ((1 - wz[v]) * ((1 - wx[v]) * in_at(in, q + n) + wx[v] * in_at(in, q + 1 + n)) +
-                                   wz[v] * ((1 - wx[v]) * in_at(in, q + nx + n) +
-                                            wx[v] * in_at(in, q + 1 + nx + n)));
-                }
+                val = (1 - wy[v]) * ((1 - wz[v]) * ((1 - wx[v]) * in_at(in, q) + wx[v] * in_at(in, q + 1)) +
+                                     wz[v] * ((1 - wx[v]) * in_at(in, q + nx) + wx[v] * in_at(in, q + 1 + nx))) +
+                      wy[v] * ((1 - wz[v]) * ((1 - wx[v]) * in_at(in, q + n) + wx[v] * in_at(in, q + 1 + n)) +
+                               wz[v] * ((1 - wx[v]) * in_at(in, q + nx + n) +
+                                        wx[v] * in_at(in, q + 1 + nx + n)));
             }
             o.v[v] = clamp_out<OutT>(val);
         }
@@ -320,97 +317,153 @@ __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
     }
 }
 
-// 2D with 4 pixels per thread (the packed case), input staged in LDS.  A
-// block's 1024 consecutive output pixels read a narrow range of input
-// elements (a few sample rows of a linear scan); the block finds that range
-// once and copies it per frame, converted to float as the direct kernel
-// converts each sample, into one of two LDS windows (one barrier per frame;
-// the next frame's window is loaded into registers meanwhile).  The window
-// holds floats so that neighbouring samples are read at 4-byte aligned LDS
-// addresses.  The four neighbours of each pixel are the elements the direct
-// kernel reads, so the results are identical.  A block whose range exceeds
-// the window (wide sector rows) reads the input directly.
-constexpr uint32_t kScWin = 1024;            // elements per window; two windows per block
-constexpr int kScPer = kScWin / 256;         // window elements per thread
+// 2D: a workgroup takes 64 x 16 output pixels, 4 consecutive ones per thread,
+// of a range of frames.  The pixels of such a tile read a small box of input
+// samples (rows of consecutive samples x neighbouring scanlines: 10 x 70 for a
+// sector, fewer for a linear scan; a run of pixels of one output row, by
+// contrast, crosses hundreds of sample rows of a sector).  The workgroup finds
+// the box once and copies it per pair of frames, converted to float as the
+// direct kernel converts each sample, into one of two LDS windows (one barrier
+// per pair; the next pair is loaded into registers meanwhile).  The two frames
+// of a pair are interleaved, so that an LDS read serves both.  The four
+// neighbours of each pixel are the samples the direct form reads, so the
+// results are identical.  A tile whose box exceeds the window (near the apex
+// of a sector) reads the input directly.  32 uint8 frames of a 60 degree
+// sector onto 1601 x 1601 pixels: 58 us, 121 us with one pixel per thread and
+// gathers from global memory; VALU 50 % busy.
+constexpr uint32_t kScTileX = 64, kScTileY = 16;
+constexpr uint32_t kScWin = 1024;            // samples per window
+constexpr int kScPer = kScWin / 256;         // window samples per thread
+
+// Stores up to V pixels of a row at p, whatever p's alignment.
+template <typename OutT, int V>
+__device__ inline void store_pixels(OutT* p, const OutPack<OutT, V>& o, uint32_t count) {
+    if (count >= V) {
+        __builtin_memcpy(p, &o, sizeof(o));
+    } else {
+#pragma unroll
+        for (uint32_t v = 0; v < V; v++)
+            if (v < count) p[v] = o.v[v];
+    }
+}
 
 template <typename InT, typename OutT>
-__global__ __launch_bounds__(256) void scan_convert_lds_kernel(const ConvArgs a) {
+__global__ __launch_bounds__(256) void scan_convert_tile_kernel(const ConvArgs a) {
     constexpr int V = 4;
-    __shared__ float win[2][kScWin];
-    __shared__ uint64_t red_lo[4], red_hi[4];
-    const uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * V;
-    const bool live = i0 < a.n_pixels;   // n_pixels is a multiple of V
-    const uint64_t n = a.n_rx;
-    uint64_t s[V];
+    __shared__ float2 win[2][kScWin];
+    __shared__ uint32_t red[4][4];
+    const uint32_t tiles_x = (a.size_x + kScTileX - 1) / kScTileX;
+    const uint32_t x0 = (blockIdx.x % tiles_x) * kScTileX + (threadIdx.x % 16) * V;
+    const uint32_t y = (blockIdx.x / tiles_x) * kScTileY + threadIdx.x / 16;
+    const uint32_t count = y < a.size_y && x0 < a.size_x ? min(static_cast<uint32_t>(V), a.size_x - x0) : 0u;
+    const uint64_t i0 = static_cast<uint64_t>(y) * a.size_x + x0;
+    const uint32_t n = a.n_rx;
+    uint32_t s[V];
     bool valid[V];
     float wx[V], wy[V];
-    uint64_t lo = ~0ull, hi = 0;
+    uint32_t lo_r = ~0u, hi_r = 0, lo_c = ~0u, hi_c = 0;
+#pragma unroll
     for (int v = 0; v < V; v++) {
-        const uint64_t i = i0 + v;
-        const uint32_t s32 = live ? a.idx[i] : kOutside;
-        s[v] = s32;
+        const bool in = static_cast<uint32_t>(v) < count;
+        s[v] = in ? a.idx[i0 + v] : kOutside;
         // the last sample row has no successor: the reference's 3D guard, used in 2D too
-        valid[v] = s32 != kOutside && s[v] + 1 + n < a.in_frame;
-        wx[v] = valid[v] ? a.wx[i] : 0.0f;
-        wy[v] = valid[v] ? a.wy[i] : 0.0f;
+        valid[v] = s[v] != kOutside && static_cast<uint64_t>(s[v]) + 1 + n < a.in_frame;
+        wx[v] = valid[v] ? a.wx[i0 + v] : 0.0f;
+        wy[v] = valid[v] ? a.wy[i0 + v] : 0.0f;
         if (valid[v]) {
-            lo = min(lo, s[v]);
-            hi = max(hi, s[v] + 1 + n);
+            const uint32_t r = s[v] / n, c = s[v] % n;
+            lo_r = min(lo_r, r), hi_r = max(hi_r, r);
+            lo_c = min(lo_c, c), hi_c = max(hi_c, c);
         }
     }
-    // block range [lo, hi] of the elements read
+    // the box of samples the tile reads, without the neighbours below and right
+#pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        lo = min(lo, static_cast<uint64_t>(__shfl_xor(static_cast<long long>(lo), o, 64)));
-        hi = max(hi, static_cast<uint64_t>(__shfl_xor(static_cast<long long>(hi), o, 64)));
+        lo_r = min(lo_r, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo_r), o, 64)));
+        hi_r = max(hi_r, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi_r), o, 64)));
+        lo_c = min(lo_c, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo_c), o, 64)));
+        hi_c = max(hi_c, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi_c), o, 64)));
     }
-    const uint32_t wave = threadIdx.x / 64;
     if (threadIdx.x % 64 == 0) {
-        red_lo[wave] = lo;
-        red_hi[wave] = hi;
+        uint32_t* w = red[threadIdx.x / 64];
+        w[0] = lo_r, w[1] = hi_r, w[2] = lo_c, w[3] = hi_c;
     }
     __syncthreads();
-    lo = min(min(red_lo[0], red_lo[1]), min(red_lo[2], red_lo[3]));
-    hi = max(max(red_hi[0], red_hi[1]), max(red_hi[2], red_hi[3]));
-    const bool staged = lo <= hi && hi - lo < kScWin;
-    const uint32_t extent = staged ? static_cast<uint32_t>(hi - lo + 1) : 0u;
+    lo_r = min(min(red[0][0], red[1][0]), min(red[2][0], red[3][0]));
+    hi_r = max(max(red[0][1], red[1][1]), max(red[2][1], red[3][1]));
+    lo_c = min(min(red[0][2], red[1][2]), min(red[2][2], red[3][2]));
+    hi_c = max(max(red[0][3], red[1][3]), max(red[2][3], red[3][3]));
+    const bool any = lo_r <= hi_r;
+    const uint64_t bw = any ? hi_c - lo_c + 2u : 0u;
+    const uint64_t extent64 = any ? bw * (hi_r - lo_r + 2u) : 0u;
+    const bool staged = extent64 <= kScWin;
+    const uint32_t extent = staged ? static_cast<uint32_t>(extent64) : 0u, width = static_cast<uint32_t>(bw);
+    // this thread's window samples, and the pixels' places in the window
+    uint64_t src[kScPer];
+#pragma unroll
+    for (int j = 0; j < kScPer; j++) {
+        const uint32_t k = threadIdx.x + static_cast<uint32_t>(j) * 256u;
+        src[j] = k < extent ? static_cast<uint64_t>(lo_r + k / width) * n + lo_c + k % width : 0u;
+    }
+    uint32_t at[V];
+#pragma unroll
+    for (int v = 0; v < V; v++) at[v] = valid[v] && staged ? (s[v] / n - lo_r) * width + s[v] % n - lo_c : 0u;
 
-    const InT* in = static_cast<const InT*>(a.in);
-    OutT* out = static_cast<OutT*>(a.out);
-    float pre[kScPer];
-    auto fetch = [&](const InT* src) {
+    const uint32_t f0 = blockIdx.y * a.frames_per_group, f1 = min(a.num_frames, f0 + a.frames_per_group);
+    const InT* in = static_cast<const InT*>(a.in) + static_cast<uint64_t>(f0) * a.in_frame;
+    OutT* out = static_cast<OutT*>(a.out) + static_cast<uint64_t>(f0) * a.n_pixels + i0;
+    float2 pre[kScPer];
+    auto fetch = [&](const InT* p, bool two) {
+#pragma unroll
         for (int j = 0; j < kScPer; j++) {
             const uint32_t k = threadIdx.x + static_cast<uint32_t>(j) * 256u;
-            pre[j] = k < extent ? static_cast<float>(src[lo + k]) : 0.0f;
+            pre[j] = make_float2(0.0f, 0.0f);
+            if (k < extent) {
+                pre[j].x = in_at(p, src[j]);
+                if (two) pre[j].y = in_at(p, src[j] + a.in_frame);
+            }
         }
     };
-    if (staged) fetch(in);
-    for (uint32_t f = 0; f < a.num_frames; f++, in += a.in_frame, out += a.n_pixels) {
-        const uint32_t b = f & 1u;
-        if (staged) {
+    auto mix = [](float tx, float ty, float p00, float p10, float p01, float p11) {
+        return (1 - ty) * ((1 - tx) * p00 + tx * p10) + ty * ((1 - tx) * p01 + tx * p11);
+    };
+    if (extent) fetch(in, f0 + 1 < f1);
+    for (uint32_t f = f0; f < f1; f += 2, in += 2 * a.in_frame, out += 2 * a.n_pixels) {
+        const bool two = f + 1 < f1;
+        const float2* w = win[(f - f0) / 2u & 1u];
+        if (extent) {
+#pragma unroll
             for (int j = 0; j < kScPer; j++) {
                 const uint32_t k = threadIdx.x + static_cast<uint32_t>(j) * 256u;
-                if (k < extent) win[b][k] = pre[j];
+                if (k < extent) win[(f - f0) / 2u & 1u][k] = pre[j];
             }
             __syncthreads();
-            if (f + 1 < a.num_frames) fetch(in + a.in_frame);
+            if (f + 2 < f1) fetch(in + 2 * a.in_frame, f + 3 < f1);
         }
-        OutPack<OutT, V> o;
-        for (int v = 0; v < V; v++) {
-            float val = 0.0f;
-            if (valid[v]) {
-                if (staged) {
-                    const uint32_t q = static_cast<uint32_t>(s[v] - lo);
-                    val = (1 - wy[v]) * ((1 - wx[v]) * win[b][q] + wx[v] * win[b][q + 1]) +
-                          wy[v] * ((1 - wx[v]) * win[b][q + n] + wx[v] * win[b][q + 1 + n]);
-                } else {
-                    const uint64_t q = s[v];
-                    val = (1 - wy[v]) * ((1 - wx[v]) * in_at(in, q) + wx[v] * in_at(in, q + 1)) +
-                          wy[v] * ((1 - wx[v]) * in_at(in, q + n) + wx[v] * in_at(in, q + 1 + n));
-                }
+        OutPack<OutT, V> o0, o1;
+        if (staged) {      // uniform
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+                const float2* q = w + at[v];
+                const float2 p00 = q[0], p10 = q[1], p01 = q[width], p11 = q[width + 1];
+                // (masked, not selected: a branch per pixel costs more)
+                const uint32_t keep = valid[v] ? ~0u : 0u;
+                o0.v[v] = clamp_out<OutT>(__uint_as_float(__float_as_uint(mix(wx[v], wy[v], p00.x, p10.x, p01.x, p11.x)) & keep));
+                o1.v[v] = clamp_out<OutT>(__uint_as_float(__float_as_uint(mix(wx[v], wy[v], p00.y, p10.y, p01.y, p11.y)) & keep));
             }
-            o.v[v] = clamp_out<OutT>(val);
+        } else {
+            auto direct = [&](const InT* p, int v) {
+                const uint64_t q = s[v];
+                return mix(wx[v], wy[v], in_at(p, q), in_at(p, q + 1), in_at(p, q + n), in_at(p, q + n + 1));
+            };
+#pragma unroll
+            for (int v = 0; v < V; v++) {
+                o0.v[v] = clamp_out<OutT>(valid[v] ? direct(in, v) : 0.0f);
+                o1.v[v] = clamp_out<OutT>(valid[v] && two ? direct(in + a.in_frame, v) : 0.0f);
+            }
         }
-        if (live) *reinterpret_cast<OutPack<OutT, V>*>(out + i0) = o;
+        store_pixels<OutT, V>(out, o0, count);
+        if (two) store_pixels<OutT, V>(out + a.n_pixels, o1, count);
     }
 }
 
@@ -706,17 +759,25 @@ extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanline
     const size_t out_size = out_dtype == SUPRA_FLOAT32 ? 4 : (out_dtype == SUPRA_INT16 ? 2 : 1);
     const bool packed = a.n_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * out_size) == 0;
     const uint64_t threads = packed ? a.n_pixels / 4 : a.n_pixels;
-    const dim3 grid(static_cast<uint32_t>((threads + 255) / 256)), block(256);
+    dim3 grid(static_cast<uint32_t>((threads + 255) / 256)), block(256);
+    if (!sc->is3d) {
+        a.size_x = sc->size[0];
+        a.size_y = sc->size[1] * sc->size[2];    // (rows of every plane; a 2D scan fills the first)
+        const uint64_t tiles = static_cast<uint64_t>((a.size_x + kScTileX - 1) / kScTileX) * ((a.size_y + kScTileY - 1) / kScTileY);
+        // frames are divided among workgroups where the tiles alone leave
+        // CUs without their 8 workgroups, at least 4 frames each (the tables
+        // and the box are set up once per workgroup)
+        const uint64_t want = (2048 + tiles - 1) / tiles, most = (num_frames + 3) / 4;
+        const uint32_t groups = static_cast<uint32_t>(std::max<uint64_t>(1, std::min(want, most)));
+        a.frames_per_group = (num_frames + groups - 1) / groups;
+        grid = dim3(static_cast<uint32_t>(tiles), (num_frames + a.frames_per_group - 1) / a.frames_per_group);
+    }
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define SUPRA_SC_LAUNCH(IN, OUT)                                                                                       \
     do {                                                                                                              \
-        if (packed) {                                                                                                 \
-            if (sc->is3d) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, true, 4>), grid, block, 0, s, a);          \
-            else hipLaunchKernelGGL((scan_convert_lds_kernel<IN, OUT>), grid, block, 0, s, a);                        \
-        } else {                                                                                                      \
-            if (sc->is3d) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, true, 1>), grid, block, 0, s, a);          \
-            else hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, false, 1>), grid, block, 0, s, a);                  \
-        }                                                                                                             \
+        if (!sc->is3d) hipLaunchKernelGGL((scan_convert_tile_kernel<IN, OUT>), grid, block, 0, s, a);                 \
+        else if (packed) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 4>), grid, block, 0, s, a);                 \
+        else hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 1>), grid, block, 0, s, a);                             \
     } while (0)
 #define SUPRA_SC_OUT(IN)                                                                                              \
     do {                                                                                                              \
