@@ -361,7 +361,9 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
     build_window_lut(window_type, window_parameter, a.lut);
 
     hipError_t e;
-    if (sample_beamformer == SUPRA_BF_DELAY_AND_STD_DEV || sample_beamformer == SUPRA_BF_COHERENCE_FACTOR)
+    if (sample_beamformer == SUPRA_BF_COHERENCE_FACTOR && !ctx->is3d)
+        e = launch_coherence_2d(a, rf_dtype, out_dtype, interpolate_transmits != 0, ctx->d_e2c != nullptr, hs);
+    else if (sample_beamformer == SUPRA_BF_DELAY_AND_STD_DEV || sample_beamformer == SUPRA_BF_COHERENCE_FACTOR)
         e = launch_das_variant(a, rf_dtype, out_dtype, ctx->is3d, sample_beamformer, interpolate_transmits != 0, hs);
     else
         e = launch_das(a, rf_dtype, out_dtype, ctx->is3d, sample_beamformer == SUPRA_BF_TEST_SIGNAL,

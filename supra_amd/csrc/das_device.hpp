@@ -27,13 +27,23 @@ template <> __device__ inline int16_t clamp_cast<int16_t>(float x) {
     return static_cast<int16_t>(fminf(fmaxf(x, -32767.0f), 32767.0f));
 }
 
-// WindowFunctionGpu::get (WindowFunction.h:58-64): roundf of a value in
-// [0, 63], computed as truncation plus a half-up step (identical to roundf
-// for non-negative arguments).
+// WindowFunctionGpu::get (WindowFunction.h:58-64): roundf of a value x in
+// [0, 63].  Truncating x + 0.49999997 (the float below 0.5) rounds half up for
+// every float in that range, which is roundf for non-negative values.  A NaN
+// clamps to -1, as fminf(fmaxf()) would clamp it.
 __device__ inline int window_index(float rel) {
-    const float x = 31.5f * (fminf(fmaxf(rel, -1.0f), 1.0f) + 1.0f);
-    const uint32_t t = static_cast<uint32_t>(x);
-    return static_cast<int>(t + ((x - static_cast<float>(t)) >= 0.5f ? 1u : 0u));
+    const float x = 31.5f * (__builtin_amdgcn_fmed3f(rel, -1.0f, 1.0f) + 1.0f);
+    return static_cast<int>(static_cast<uint32_t>(x + 0.49999997f));
+}
+
+// Bits of the last sample's index as a float: a delay tau lies in [0, N-1]
+// where its own bits, compared as unsigned integers, are not larger (negative
+// and NaN delays compare larger; no delay is ever -0, since none of the sums
+// it is made of can be).
+__device__ inline uint32_t last_sample_bits(uint32_t n_s) {
+    const float f = static_cast<float>(n_s - 1u);
+    const uint32_t b = __float_as_uint(f);
+    return static_cast<uint32_t>(f) > n_s - 1u ? b - 1u : b;    // (rounded up above 2^24 samples)
 }
 
 // Correctly rounded single-precision square root for x == 0 or normal x

@@ -83,69 +83,80 @@ struct Pixel2D {
 template <typename RFT>
 struct Gather2D {
     float v0, v1, f, w;
-    bool add;    // int16: member and 0 <= tau <= N-1; float: member and (inr | edge)
-    bool edge;   // float: the last sample with zero fraction
+    bool member, add;   // add: member and 0 <= tau <= N-1
+    bool edge;          // float RF: the last sample with zero fraction
 };
 
-template <typename RFT>
-__device__ inline Gather2D<RFT> gather2d_issue(__amdgpu_buffer_rsrc_t rf, uint32_t off, uint32_t n_s, float tau,
-                                               float w, bool member) {
-    Gather2D<RFT> g;
-    const uint32_t ui = static_cast<uint32_t>(static_cast<int32_t>(floorf(tau)));
-    g.f = __builtin_amdgcn_fractf(tau);
-    g.w = w;
-    g.v0 = load_rf<RFT>(rf, off + ui);
-    g.v1 = load_rf<RFT>(rf, off + ui + 1u);
-    if constexpr (std::is_same_v<RFT, int16_t>) {
-        const float last = static_cast<float>(n_s - 1u);
-        g.add = member & (tau >= 0.0f) & (tau <= last);
-        g.edge = false;
-    } else {
-        const bool inr = (ui < n_s - 1u) & (tau == tau);
-        g.edge = (ui == n_s - 1u) & (g.f == 0.0f);
-        g.add = member & (inr | g.edge);
+// What a pixel adds up over its aperture: KIND SUPRA_BF_DELAY_AND_SUM needs
+// the weighted values, the weights and their count; the coherence factor
+// (RxSampleBeamformerCoherenceFactorDelayAndSum.h:152-258) also the values and
+// their squares, which do not depend on the delay-and-sum: one pass gives all.
+template <int KIND>
+struct Sums2D {
+    float sample = 0.0f, wsum = 0.0f, cs = 0.0f, te = 0.0f;
+    int nadd = 0;
+    // The element's contribution in gather()'s operations.  A skipped element
+    // adds +0 (int16: no sum is ever -0) or leaves the sums selected unchanged.
+    template <typename RFT>
+    __device__ inline void add(Gather2D<RFT> g) {
+        // (opaque: the compiler would otherwise branch around the weight's
+        // table read, and a batch's gathers would no longer go out together)
+        asm volatile("" : "+v"(g.w));
+        g.w = g.member ? g.w : 0.0f;
+        // a skipped element adds +0 to wsum (never -0: window weights are >= 0) and 0 to n
+        wsum += g.w;
+        nadd += g.member ? 1 : 0;
+        const float lerp = (1.0f - g.f) * g.v0 + g.f * g.v1;
+        if constexpr (KIND == SUPRA_BF_COHERENCE_FACTOR) {
+            float v = std::is_same_v<RFT, int16_t> ? lerp : (g.edge ? g.v0 : lerp);
+            v = g.add ? v : 0.0f;
+            sample += g.w * v;
+            cs += v;
+            te += v * v;
+        } else if constexpr (std::is_same_v<RFT, int16_t>) {
+            const float contrib = g.w * lerp;
+            sample += g.add ? contrib : 0.0f;
+        } else {
+            const float contrib = g.w * (g.edge ? g.v0 : lerp);
+            sample = g.add ? sample + contrib : sample;
+        }
     }
-    return g;
-}
-
-// The element's contribution in gather()'s operations; a skipped element adds
-// +0 (int16: the sum is never -0) or leaves the sum selected unchanged.
-template <typename RFT>
-__device__ inline void gather2d_consume(const Gather2D<RFT>& g, float& sample) {
-    if constexpr (std::is_same_v<RFT, int16_t>) {
-        const float contrib = g.w * ((1.0f - g.f) * g.v0 + g.f * g.v1);
-        sample += g.add ? contrib : 0.0f;
-    } else {
-        const float val = g.edge ? g.v0 : ((1.0f - g.f) * g.v0 + g.f * g.v1);
-        const float contrib = g.w * val;
-        sample = g.add ? sample + contrib : sample;
+    __device__ inline float result() const {
+        float r = (nadd > 0) ? (sample / wsum) * static_cast<float>(nadd) : 0.0f;
+        if constexpr (KIND == SUPRA_BF_COHERENCE_FACTOR) r = (nadd > 0) ? cs * cs / te / static_cast<float>(nadd) * r : 0.0f;
+        return r;
     }
-}
+};
 
 // Elements [0, cnt) of the current LDS chunk for one 2D pixel
 // (RxSampleBeamformerDelayAndSum.h:150-199), in batches of kBatch2D whose
-// delays and gathers all go out before the first is consumed (as in 3D);
-// weights, counts and samples are added in element order.
+// delays and gathers all go out before the first is consumed; weights, counts
+// and samples are added in element order.  One linear_2d frame (128 lines x
+// 2080 depths x 64-element aperture, int16) takes 17.5 us with this loop, no branch
+// per element and the near field's range below (25.7 us with a branch around
+// each element's aperture test and its own range test); it is bound by the
+// VALU, ~30 instructions per element with two waves per SIMD.  Batches of 2,
+// 4, 8 and 16 elements (frame / four transmits / coherence factor, us):
+// 24.9/58.4/46.0, 20.9/45.4/38.5, 21.1/56.7/46.9, 30.6/91.8/60.5 (before the
+// range: past 8 the registers cost a wave per SIMD).
 constexpr int kBatch2D = 4;
 
 template <typename RFT, bool FAR, bool VERT, bool MAP>
-__device__ inline Gather2D<RFT> element2d_issue(__amdgpu_buffer_rsrc_t rf, uint32_t n_s, float t0, float offset,
+__device__ inline Gather2D<RFT> element2d_issue(__amdgpu_buffer_rsrc_t rf, uint32_t last_bits, float t0, float offset,
                                                 const Pixel2D& p, const float* s_xe, const float* s_dx,
                                                 const float* s_dx2, const float* s_w, const uint32_t* s_off,
-                                                const float* s_lut, int j, float& wsum, int& nadd) {
+                                                const float* s_lut, int j) {
+    Gather2D<RFT> g;
     const uint32_t off = s_off[j];
     bool member = !MAP || off != kNotConnected;
-    float w;
     if (FAR) {
-        w = member ? s_w[j] : 0.0f;
+        g.w = s_w[j];
     } else {
         const float dx = s_dx[j];
         member = member && (fabsf(dx) <= p.aDT);
-        w = member ? s_lut[window_index(dx * p.inv)] : 0.0f;
+        g.w = s_lut[window_index(dx * p.inv)];
     }
-    // a skipped element adds +0 to wsum (never -0: window weights are >= 0) and 0 to n
-    wsum += w;
-    nadd += member ? 1 : 0;
+    g.member = member;
     float q;
     if (VERT) {
         q = s_dx2[j] + p.py2;
@@ -155,38 +166,49 @@ __device__ inline Gather2D<RFT> element2d_issue(__amdgpu_buffer_rsrc_t rf, uint3
     }
     float tau = t0 + (sqrt_rn(q) + p.d);
     tau = tau + offset;
-    return gather2d_issue<RFT>(rf, off, n_s, tau, w, member);
+    const uint32_t ui = static_cast<uint32_t>(tau);     // (outside the RF: some sample, or none, that is not added)
+    g.f = __builtin_amdgcn_fractf(tau);
+    g.v0 = load_rf<RFT>(rf, off + ui);
+    g.v1 = load_rf<RFT>(rf, off + ui + 1u);
+    g.add = member & (__float_as_uint(tau) <= last_bits);
+    g.edge = !std::is_same_v<RFT, int16_t> && __float_as_uint(tau) == last_bits;
+    return g;
 }
 
-template <typename RFT, bool FAR, bool VERT, bool MAP>
-__device__ inline void elements2d(__amdgpu_buffer_rsrc_t rf, uint32_t n_s, float t0, float offset, const Pixel2D& p,
-                                  const float* s_xe, const float* s_dx, const float* s_dx2, const float* s_w,
-                                  const uint32_t* s_off, const float* s_lut, int cnt, float& sample, float& wsum,
-                                  int& nadd) {
+template <typename RFT, int KIND, bool FAR, bool VERT, bool MAP>
+__device__ inline void elements2d(__amdgpu_buffer_rsrc_t rf, uint32_t last_bits, float t0, float offset,
+                                  const Pixel2D& p, const float* s_xe, const float* s_dx, const float* s_dx2,
+                                  const float* s_w, const uint32_t* s_off, const float* s_lut, int cnt, float aDT_max,
+                                  Sums2D<KIND>& sums) {
     int j = 0;
-    for (; j + kBatch2D <= cnt; j += kBatch2D) {
-        if (!FAR) {
-            // near field: a batch that no lane of the wave has in its
-            // aperture adds nothing (+0 weights, no samples) and is skipped
-            bool any = false;
-#pragma unroll
-            for (int u = 0; u < kBatch2D; u++)
-                any |= (fabsf(s_dx[j + u]) <= p.aDT) && (!MAP || s_off[j + u] != kNotConnected);
-            if (__builtin_amdgcn_ballot_w64(any) == 0) continue;   // uniform
+    if (!FAR) {
+        // near field: only the elements between the first and the last that a
+        // lane of the wave has in its aperture; the others add nothing (+0
+        // weights, no samples)
+        const int lane = static_cast<int>(threadIdx.x % 64);
+        int lo = cnt, hi = 0;
+        for (int b = 0; b < cnt; b += 64) {
+            const bool in = b + lane < cnt && fabsf(s_dx[min(b + lane, cnt - 1)]) <= aDT_max;
+            const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+            if (m != 0) {
+                lo = min(lo, b + static_cast<int>(__builtin_ctzll(m)));
+                hi = b + 64 - static_cast<int>(__builtin_clzll(m));
+            }
         }
+        j = lo;
+        cnt = hi;
+    }
+    for (; j + kBatch2D <= cnt; j += kBatch2D) {
         Gather2D<RFT> g[kBatch2D];
 #pragma unroll
         for (int u = 0; u < kBatch2D; u++)
-            g[u] = element2d_issue<RFT, FAR, VERT, MAP>(rf, n_s, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off, s_lut,
-                                                        j + u, wsum, nadd);
+            g[u] = element2d_issue<RFT, FAR, VERT, MAP>(rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off,
+                                                        s_lut, j + u);
 #pragma unroll
-        for (int u = 0; u < kBatch2D; u++) gather2d_consume<RFT>(g[u], sample);
+        for (int u = 0; u < kBatch2D; u++) sums.add(g[u]);
     }
-    for (; j < cnt; j++) {
-        const Gather2D<RFT> g = element2d_issue<RFT, FAR, VERT, MAP>(rf, n_s, t0, offset, p, s_xe, s_dx, s_dx2, s_w,
-                                                                     s_off, s_lut, j, wsum, nadd);
-        gather2d_consume<RFT>(g, sample);
-    }
+    for (; j < cnt; j++)
+        sums.add(element2d_issue<RFT, FAR, VERT, MAP>(rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off, s_lut, j));
 }
 
 // RxSampleBeamformerTestSignal::sampleBeamform2D (RxSampleBeamformerTestSignal.h:87-133):
@@ -288,7 +310,7 @@ struct Lds2D {
 
 // One wave's 2D unit: 64 consecutive depths (t.r0 ...) of one scanline of one
 // frame, with the wave's own LDS tables (no workgroup barrier).
-template <typename RFT, typename OutT, bool TESTSIG, bool INTERP_TX, bool MAP>
+template <typename RFT, typename OutT, int KIND, bool INTERP_TX, bool MAP>
 __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile& t, Lds2D& L) {
     if (!__any(t.valid)) return;   // (wave-uniform) a unit past the end of the image or the list
     const int lane = static_cast<int>(threadIdx.x % 64);
@@ -319,6 +341,10 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
     // far-field path only for non-negative, non-decreasing depth tables)
     const float d0 = load_uniform_float(depths, t.r0);
     const float aDT0 = (((d0 * a.dt) * c) / (2.0f * a.F)) / c / a.dt;
+    // the largest aperture of the unit's lanes: at its last depth, where the
+    // depths do not decrease (far_ok)
+    const float d1 = load_uniform_float(depths, min(t.r0 + kWaveDepths, a.n_depths) - 1u);
+    const float aDT1 = a.far_ok ? (((d1 * a.dt) * c) / (2.0f * a.F)) / c / a.dt : INFINITY;
     const float inv_far = 1.0f / sc.max_ed_x();
     const size_t norm_slot_stride = static_cast<size_t>(a.n_rx) * a.n_depths;
     float* norm_px = a.norm_out ? a.norm_out + (static_cast<size_t>(t.frame) * (INTERP_TX ? 4 : 1) * a.n_rx + t.s) *
@@ -336,14 +362,14 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
         }
         const TxDT tx = sc.tx(k);
         float s_local;
-        if (TESTSIG) {
+        if (KIND == SUPRA_BF_TEST_SIGNAL) {
             s_local = test_signal_2d(sc.x(), sc.dir_x(), sc.dir_y(), p.d, a.dt, c);
         } else {
             const RFT* rf_tx = rf_frame + static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
             const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
+            const uint32_t last_bits = last_sample_bits(a.n_s);
             const bool far = a.far_ok && aDT0 >= tx.far_thr;
-            float sample = 0.0f, wsum = 0.0f;
-            int nadd = 0;
+            Sums2D<KIND> sums;
             const int first = tx.first_x, last = tx.last_x;
             for (int base = first; base < last; base += kChunk2D) {
                 const int cnt = min(kChunk2D, last - base);
@@ -368,23 +394,23 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
                 wave_sync_2d();
                 if (far) {
                     if (vertical)
-                        elements2d<RFT, true, true, MAP>(rsrc, a.n_s, tx.t0, a.offset, p, s_xe, s_dx, s_dx2, s_w,
-                                                         s_off, s_lut, cnt, sample, wsum, nadd);
+                        elements2d<RFT, KIND, true, true, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
+                                                               s_w, s_off, s_lut, cnt, aDT1, sums);
                     else
-                        elements2d<RFT, true, false, MAP>(rsrc, a.n_s, tx.t0, a.offset, p, s_xe, s_dx, s_dx2, s_w,
-                                                          s_off, s_lut, cnt, sample, wsum, nadd);
+                        elements2d<RFT, KIND, true, false, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
+                                                                s_w, s_off, s_lut, cnt, aDT1, sums);
                 } else {
                     if (vertical)
-                        elements2d<RFT, false, true, MAP>(rsrc, a.n_s, tx.t0, a.offset, p, s_xe, s_dx, s_dx2, s_w,
-                                                          s_off, s_lut, cnt, sample, wsum, nadd);
+                        elements2d<RFT, KIND, false, true, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
+                                                                s_w, s_off, s_lut, cnt, aDT1, sums);
                     else
-                        elements2d<RFT, false, false, MAP>(rsrc, a.n_s, tx.t0, a.offset, p, s_xe, s_dx, s_dx2, s_w,
-                                                           s_off, s_lut, cnt, sample, wsum, nadd);
+                        elements2d<RFT, KIND, false, false, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx,
+                                                                 s_dx2, s_w, s_off, s_lut, cnt, aDT1, sums);
                 }
             }
-            s_local = (nadd > 0) ? (sample / wsum) * static_cast<float>(nadd) : 0.0f;
+            s_local = sums.result();
             if (norm_px && t.valid) {
-                const float g = (nadd > 0) ? static_cast<float>(nadd) / wsum : 0.0f;
+                const float g = (sums.nadd > 0) ? static_cast<float>(sums.nadd) / sums.wsum : 0.0f;
                 norm_px[(INTERP_TX ? k : 0) * norm_slot_stride] = INTERP_TX ? sc.txw(k) * g : g;
             }
         }
@@ -401,11 +427,11 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
     }
 }
 
-template <typename RFT, typename OutT, bool TESTSIG, bool INTERP_TX, bool MAP>
+template <typename RFT, typename OutT, int KIND, bool INTERP_TX, bool MAP>
 __global__ __launch_bounds__(kThreads) void das2d_kernel(const DasArgs a) {
     __shared__ Lds2D lds[kWavesPerGroup];
     const uint32_t wave = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64)));
-    das2d_tile<RFT, OutT, TESTSIG, INTERP_TX, MAP>(a, a.lut, decode_wave_2d(a), lds[wave]);
+    das2d_tile<RFT, OutT, KIND, INTERP_TX, MAP>(a, a.lut, decode_wave_2d(a), lds[wave]);
 }
 
 // ---- 2D, several frames per wave ---------------------------------------------
@@ -1305,11 +1331,11 @@ __global__ __launch_bounds__(kThreads) void rawdelay3d_kernel(const DasArgs a) {
 template <typename RFT, typename OutT>
 __device__ inline void das2d_batch_tile(const DasBatchFrame& fr, const DasArgs& a, const Tile& t, Lds2D& L) {
     if (fr.interp) {
-        if (fr.map) das2d_tile<RFT, OutT, false, true, true>(a, fr.a.lut, t, L);
-        else das2d_tile<RFT, OutT, false, true, false>(a, fr.a.lut, t, L);
+        if (fr.map) das2d_tile<RFT, OutT, SUPRA_BF_DELAY_AND_SUM, true, true>(a, fr.a.lut, t, L);
+        else das2d_tile<RFT, OutT, SUPRA_BF_DELAY_AND_SUM, true, false>(a, fr.a.lut, t, L);
     } else {
-        if (fr.map) das2d_tile<RFT, OutT, false, false, true>(a, fr.a.lut, t, L);
-        else das2d_tile<RFT, OutT, false, false, false>(a, fr.a.lut, t, L);
+        if (fr.map) das2d_tile<RFT, OutT, SUPRA_BF_DELAY_AND_SUM, false, true>(a, fr.a.lut, t, L);
+        else das2d_tile<RFT, OutT, SUPRA_BF_DELAY_AND_SUM, false, false>(a, fr.a.lut, t, L);
     }
 }
 
@@ -1361,14 +1387,26 @@ static uint64_t pad_2d_grid(uint64_t blocks) {
     return (blocks + round - 1) / round * round;
 }
 
+// One wave per 64-depth unit, single frames (das2d_kernel).
+template <typename RFT, typename OutT, int KIND>
+static void launch_2d(const DasArgs& a, bool interp_tx, bool map, hipStream_t stream) {
+    const uint64_t units = static_cast<uint64_t>((a.n_depths + kWaveDepths - 1) / kWaveDepths) * a.n_rx * a.n_frames;
+    const dim3 grid(static_cast<uint32_t>(pad_2d_grid((units + kWavesPerGroup - 1) / kWavesPerGroup))), block(kThreads);
+    if (map) {
+        if (interp_tx) hipLaunchKernelGGL((das2d_kernel<RFT, OutT, KIND, true, true>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((das2d_kernel<RFT, OutT, KIND, false, true>), grid, block, 0, stream, a);
+    } else {
+        if (interp_tx) hipLaunchKernelGGL((das2d_kernel<RFT, OutT, KIND, true, false>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((das2d_kernel<RFT, OutT, KIND, false, false>), grid, block, 0, stream, a);
+    }
+}
+
 template <typename RFT, typename OutT>
 static hipError_t launch_typed(const DasArgs& a, bool is3d, bool testsig, bool interp_tx, bool map,
                                hipStream_t stream) {
-    const uint64_t units2d = static_cast<uint64_t>((a.n_depths + kWaveDepths - 1) / kWaveDepths) * a.n_rx * a.n_frames;
     const uint64_t round3d = static_cast<uint64_t>(kXcds) * a.depth_tiles;   // whole rounds of scanline tiles
-    const uint64_t blocks = is3d ? (static_cast<uint64_t>(a.depth_tiles) * a.n_rx * a.n_frames + round3d - 1) / round3d * round3d
-                                 : pad_2d_grid((units2d + kWavesPerGroup - 1) / kWavesPerGroup);
-    dim3 grid(static_cast<uint32_t>(blocks)), block(kThreads);
+    const uint64_t blocks = (static_cast<uint64_t>(a.depth_tiles) * a.n_rx * a.n_frames + round3d - 1) / round3d * round3d;
+    dim3 grid(static_cast<uint32_t>(blocks)), block(kThreads);    // 3D
 #define SUPRA_DAS_DISPATCH(KERNEL)                                                                                 \
     do {                                                                                                            \
         if (testsig) {                                                                                              \
@@ -1398,8 +1436,10 @@ static hipError_t launch_typed(const DasArgs& a, bool is3d, bool testsig, bool i
         dim3 g2(static_cast<uint32_t>(((units + kWavesPerGroup - 1) / kWavesPerGroup + round - 1) / round * round));
         if (map) hipLaunchKernelGGL((das2d_frames_kernel<RFT, OutT, FB, true>), g2, block, 0, stream, a);
         else hipLaunchKernelGGL((das2d_frames_kernel<RFT, OutT, FB, false>), g2, block, 0, stream, a);
+    } else if (testsig) {
+        launch_2d<RFT, OutT, SUPRA_BF_TEST_SIGNAL>(a, interp_tx, false, stream);
     } else {
-        SUPRA_DAS_DISPATCH(das2d_kernel);
+        launch_2d<RFT, OutT, SUPRA_BF_DELAY_AND_SUM>(a, interp_tx, map, stream);
     }
 #undef SUPRA_DAS_DISPATCH
     return hipGetLastError();
@@ -1433,6 +1473,19 @@ hipError_t launch_rawdelay(const DasArgs& a, int rf_dtype, int out_dtype, bool i
     } else {
         if (out_dtype == SUPRA_FLOAT32) hipLaunchKernelGGL((rawdelay2d_kernel<float, float>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((rawdelay2d_kernel<float, int16_t>), grid, block, 0, stream, a);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_coherence_2d(const DasArgs& a, int rf_dtype, int out_dtype, bool interp_tx, bool map,
+                               hipStream_t stream) {
+    constexpr int kCf = SUPRA_BF_COHERENCE_FACTOR;
+    if (rf_dtype == SUPRA_INT16) {
+        if (out_dtype == SUPRA_FLOAT32) launch_2d<int16_t, float, kCf>(a, interp_tx, map, stream);
+        else launch_2d<int16_t, int16_t, kCf>(a, interp_tx, map, stream);
+    } else {
+        if (out_dtype == SUPRA_FLOAT32) launch_2d<float, float, kCf>(a, interp_tx, map, stream);
+        else launch_2d<float, int16_t, kCf>(a, interp_tx, map, stream);
     }
     return hipGetLastError();
 }

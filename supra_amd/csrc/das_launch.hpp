@@ -19,6 +19,10 @@ hipError_t launch_das(const DasArgs& a, int rf_dtype, int out_dtype, bool is3d, 
 hipError_t launch_das_variant(const DasArgs& a, int rf_dtype, int out_dtype, bool is3d, int kind, bool interp_tx,
                               hipStream_t stream);
 
+// CoherenceFactorDelayAndSum, 2D (das_kernels.hip).
+hipError_t launch_coherence_2d(const DasArgs& a, int rf_dtype, int out_dtype, bool interp_tx, bool map,
+                               hipStream_t stream);
+
 // Launch the 2D or 3D pre-delay kernel (output [frame][scanline][channel][depth]).
 hipError_t launch_rawdelay(const DasArgs& a, int rf_dtype, int out_dtype, bool is3d, hipStream_t stream);
 

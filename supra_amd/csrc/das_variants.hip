@@ -1,7 +1,8 @@
 // The two other receive beamformers of SUPRA's BeamformingNode
-// (beamformerType DelayAndStdDev and CoherenceFactorDelayAndSum), 2D and 3D:
+// (beamformerType DelayAndStdDev and CoherenceFactorDelayAndSum):
 //   RxSampleBeamformerDelayAndStdDev.h:36-158 (3D), :161-270 (2D)
-//   RxSampleBeamformerCoherenceFactorDelayAndSum.h:33-150 (3D), :152-258 (2D)
+//   RxSampleBeamformerCoherenceFactorDelayAndSum.h:33-150 (3D)
+// (the 2D coherence factor needs no second pass: das2d_kernel forms it)
 // driven per pixel like the delay-and-sum kernels (RxBeamformerCuda.cu:109-323).
 //
 // Both make two passes over the aperture: the first is the delay-and-sum of
@@ -87,8 +88,8 @@ struct Second {
     }
 };
 
-template <typename RFT, typename OutT, int KIND, bool INTERP_TX>
-__global__ __launch_bounds__(kThreads) void das2d_variant_kernel(const DasArgs a) {
+template <typename RFT, typename OutT, bool INTERP_TX>
+__global__ __launch_bounds__(kThreads) void das2d_stddev_kernel(const DasArgs a) {
     __shared__ float s_lut[kWindowEntries];
     const uint32_t bid = blockIdx.x;
     const uint32_t s = (bid / a.depth_tiles) % a.n_rx;
@@ -116,7 +117,7 @@ __global__ __launch_bounds__(kThreads) void das2d_variant_kernel(const DasArgs a
         float sample = 0.0f, wsum = 0.0f;
         int nadd = 0;
         for (int pass = 0; pass < 2; pass++) {
-            Second<KIND> acc;
+            Second<SUPRA_BF_DELAY_AND_STD_DEV> acc;
             const float das = (nadd > 0) ? (sample / wsum) * static_cast<float>(nadd) : 0.0f;
             for (uint32_t e = tx.first_x; e < tx.last_x; e++) {
                 const uint32_t off = channel_offset(a, e);
@@ -220,27 +221,28 @@ __global__ __launch_bounds__(kThreads) void das3d_variant_kernel(const DasArgs a
     }
 }
 
-template <typename RFT, typename OutT, int KIND>
-void launch_kind(const DasArgs& a, bool is3d, bool interp_tx, dim3 grid, hipStream_t stream) {
-    if (is3d) {
-        if (interp_tx) hipLaunchKernelGGL((das3d_variant_kernel<RFT, OutT, KIND, true>), grid, dim3(kThreads), 0, stream, a);
-        else hipLaunchKernelGGL((das3d_variant_kernel<RFT, OutT, KIND, false>), grid, dim3(kThreads), 0, stream, a);
-    } else {
-        if (interp_tx) hipLaunchKernelGGL((das2d_variant_kernel<RFT, OutT, KIND, true>), grid, dim3(kThreads), 0, stream, a);
-        else hipLaunchKernelGGL((das2d_variant_kernel<RFT, OutT, KIND, false>), grid, dim3(kThreads), 0, stream, a);
-    }
+template <typename RFT, typename OutT, bool INTERP_TX>
+void launch_kind(const DasArgs& a, bool is3d, int kind, dim3 grid, hipStream_t stream) {
+    if (!is3d) hipLaunchKernelGGL((das2d_stddev_kernel<RFT, OutT, INTERP_TX>), grid, dim3(kThreads), 0, stream, a);
+    else if (kind == SUPRA_BF_DELAY_AND_STD_DEV)
+        hipLaunchKernelGGL((das3d_variant_kernel<RFT, OutT, SUPRA_BF_DELAY_AND_STD_DEV, INTERP_TX>), grid, dim3(kThreads),
+                           0, stream, a);
+    else
+        hipLaunchKernelGGL((das3d_variant_kernel<RFT, OutT, SUPRA_BF_COHERENCE_FACTOR, INTERP_TX>), grid, dim3(kThreads), 0,
+                           stream, a);
 }
 
 template <typename RFT, typename OutT>
 void launch_types(const DasArgs& a, bool is3d, int kind, bool interp_tx, dim3 grid, hipStream_t stream) {
-    if (kind == SUPRA_BF_DELAY_AND_STD_DEV) launch_kind<RFT, OutT, SUPRA_BF_DELAY_AND_STD_DEV>(a, is3d, interp_tx, grid, stream);
-    else launch_kind<RFT, OutT, SUPRA_BF_COHERENCE_FACTOR>(a, is3d, interp_tx, grid, stream);
+    if (interp_tx) launch_kind<RFT, OutT, true>(a, is3d, kind, grid, stream);
+    else launch_kind<RFT, OutT, false>(a, is3d, kind, grid, stream);
 }
 
 }  // namespace
 
 hipError_t launch_das_variant(const DasArgs& a, int rf_dtype, int out_dtype, bool is3d, int kind, bool interp_tx,
                               hipStream_t stream) {
+    if (!is3d && kind != SUPRA_BF_DELAY_AND_STD_DEV) return hipErrorInvalidValue;   // launch_coherence_2d
     // one workgroup per (frame, scanline, tile of kThreads depths); a.depth_tiles
     // is computed with the same tile (das_depth_tile() == kThreads)
     const uint64_t blocks = static_cast<uint64_t>(a.depth_tiles) * a.n_rx * a.n_frames;
