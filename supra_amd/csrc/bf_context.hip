@@ -848,13 +848,11 @@ extern "C" int supra_das_adjoint(supra_bf_ctx* ctx, uint32_t num_frames, const f
 
     std::lock_guard<std::mutex> lock(ctx->mu);
     if ((st = check_device(ctx)) != SUPRA_OK) return st;
-    // Waves (aperture elements) per workgroup: each accumulates its RF line in
-    // a fixed-size LDS ring, so any number of samples per channel fits.
     hipError_t e = hipSuccess;
-    const uint32_t waves = 4;
     const uint32_t slots = interpolate_transmits ? 4u : 1u;
-    const uint32_t egroups = std::max(1u, (ctx->max_aperture + waves - 1) / waves);
-    const uint64_t blocks = static_cast<uint64_t>(num_frames) * ctx->n_rx * slots * egroups;
+    // (the limit of one frame's work per call: groups of four elements)
+    const uint64_t blocks = static_cast<uint64_t>(num_frames) * ctx->n_rx * slots *
+                            std::max(1u, (ctx->max_aperture + 3u) / 4u);
     if (blocks >= (1ull << 31)) return fail(SUPRA_ERR_TOO_LARGE, "das adjoint: too many frames for one launch");
 
     if ((st = ensure_mm_geometry(ctx)) != SUPRA_OK) return st;
@@ -863,14 +861,15 @@ extern "C" int supra_das_adjoint(supra_bf_ctx* ctx, uint32_t num_frames, const f
     const double dt = 1.0 / sampling_frequency_hz;
     FrameTables ft;
     if ((st = build_frame_tables(ctx, num_frames, speed_of_sound_mm_per_s, dt, hs, &ft)) != SUPRA_OK) return st;
-    // beta, then the per-frame depth table (4 floats per depth), in one buffer
+    // beta, then the per-frame depth table (3 planes), in one buffer
     const size_t n_beta = static_cast<size_t>(num_frames) * slots * ctx->n_rx * ctx->n_depths;
     const size_t b_beta = align256(n_beta * sizeof(float));
-    const size_t b_dtab = static_cast<size_t>(num_frames) * ctx->n_depths * 4 * sizeof(float);
+    const size_t b_dtab = static_cast<size_t>(num_frames) * ctx->n_depths * 3 * sizeof(float);
     if ((st = ensure_capacity(&ctx->d_beta, &ctx->beta_cap, b_beta + b_dtab, "das adjoint: scratch")) != SUPRA_OK)
         return st;
     float* dtab = reinterpret_cast<float*>(static_cast<char*>(ctx->d_beta) + b_beta);
-    const size_t per_frame = static_cast<size_t>(ctx->n_rx) * slots * egroups * waves;
+    const uint32_t egroups = das_adjoint_groups(ctx->max_aperture);
+    const size_t per_frame = static_cast<size_t>(ctx->n_rx) * slots * egroups * das_adjoint_waves();
     if (grad_c && (st = ensure_capacity(&ctx->d_dc_part, &ctx->dc_part_cap, per_frame * num_frames * sizeof(double),
                                         "das adjoint: scratch")) != SUPRA_OK)
         return st;
@@ -902,7 +901,6 @@ extern "C" int supra_das_adjoint(supra_bf_ctx* ctx, uint32_t num_frames, const f
     a.dc_part = grad_c ? static_cast<double*>(ctx->d_dc_part) : nullptr;
     a.rf_frame_stride = rf_frame;
     a.scan_frame_stride = ctx->n_rx;
-    a.depth_frame_stride = ctx->n_depths;
     a.el_frame_stride = ctx->n_el;
     a.n_rx = ctx->n_rx;
     a.n_depths = ctx->n_depths;
@@ -910,11 +908,11 @@ extern "C" int supra_das_adjoint(supra_bf_ctx* ctx, uint32_t num_frames, const f
     a.n_s = num_samples;
     a.n_slots = slots;
     a.egroups = egroups;
-    a.waves = waves;
     a.F = static_cast<float>(f_number);
     a.dt = static_cast<float>(dt);
     a.offset = static_cast<float>(additional_offset);
     a.exclusive = ctx->lines_exclusive ? 1 : 0;
+    a.depths_sorted = ctx->far_ok_mm ? 1 : 0;
     a.interp_tx = interpolate_transmits ? 1 : 0;
     build_window_lut(window_type, window_parameter, a.lut);
     if ((e = launch_das_adjoint(a, num_frames, hs)) != hipSuccess) return hip_fail(e, "das adjoint: launch");

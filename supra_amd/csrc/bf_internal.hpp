@@ -102,17 +102,18 @@ struct AdjointArgs {
     const float* rf;                // [frame][tx][ch][s]
     const float* beta;              // [frame][slot][scanline][depth]: dL/dy * norm
     const ScanlineDT* scans;        // per frame (scan_frame_stride)
-    const float* dtab;              // per frame (depth_frame_stride): 4 floats {depth, aDT, 1/aDT, 0} per depth
+    const float* dtab;              // per frame: planes of depth, aDT and 1/aDT, n_depths each
     const float* ex;                // per frame (el_frame_stride)
     const float* frame_c;           // [frame] float c
     const int32_t* e2c;             // or nullptr
     float* grad_rf;                 // [frame][tx][ch][s] or nullptr
     double* dc_part;                // [frame][blocks_per_frame * waves] partial sums, or nullptr
     uint64_t rf_frame_stride;
-    uint32_t scan_frame_stride, depth_frame_stride, el_frame_stride;
-    uint32_t n_rx, n_depths, n_ch, n_s, n_slots, egroups, waves;
+    uint32_t scan_frame_stride, el_frame_stride;
+    uint32_t n_rx, n_depths, n_ch, n_s, n_slots, egroups;
     float F, dt, offset;
     int32_t exclusive;              // every written line has exactly one writer
+    int32_t depths_sorted;          // non-negative and non-decreasing
     int32_t interp_tx;
     float lut[kWindowEntries];
 };

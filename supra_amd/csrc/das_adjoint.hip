@@ -22,24 +22,35 @@
 //     dL/dc = -(1/c) sum beta w_e (rf[i+1] - rf[i]) geo        (interpolated samples)
 // and the delay tables are recomputed here, never stored by the forward.
 //
-// Launch layout (MI355X): one wave64 per (frame, scanline, slot, aperture
-// element), 4 waves per workgroup.  A wave walks all depths of its element,
-// lanes = 64 consecutive depths, and accumulates the element's RF line with
-// LDS float atomics in a ring of 256 samples: the delays grow with depth, so
-// the lanes of one instruction touch ~64 neighbouring samples, and samples
-// more than a guard below the delay of the chunk's first depth are final.
-// Those leave the ring in order, as coalesced stores when no other wave
-// writes that (transmit, channel) line (each focused transmit feeds one
+// Launch layout (MI355X): one wave64 per (frame, scanline, slot, pair of
+// aperture elements), 4 waves per workgroup.  A wave walks the depths of its
+// elements, lanes = 64 consecutive depths, and accumulates each element's RF
+// line in a ring of 256 samples in LDS: the delays grow with depth, so the
+// lanes of one instruction touch ~64 neighbouring samples, and samples more
+// than a guard below the delay of the chunk's first depth are final.  Those
+// leave the ring in order, 64 at a time, as coalesced stores when no other
+// wave writes that (transmit, channel) line (each focused transmit feeds one
 // scanline), else as global float atomics; a target outside the ring's window
 // (delays not sorted, or a chunk wider than the ring) is handled exactly by
-// moving the ring or adding to the flushed output.  1 KB of LDS per wave
-// instead of a whole line leaves room for the maximum number of waves per
-// SIMD.  d/dc partial sums go to a per-wave slot and are reduced per frame
-// in a fixed order, so the result does not depend on scheduling.  The
-// depth-only quantities (the F-number aperture aDT and 1/aDT, four IEEE
-// divisions per depth) come from a per-frame table built once, not once per
-// aperture element; neighbouring lanes exchange their sample indices by DPP
-// moves, which leave the LDS pipe to the atomics.
+// moving the ring or adding to the flushed output.  A sample's slot keeps the
+// lower shares of that sample and the upper shares of the one before, so the
+// lanes' delays meet only where two share a sample; the upper lane adds for
+// both, and one LDS read-add-write per lane does.  d/dc partial sums go to a
+// per-wave slot and are reduced per frame in a fixed order, so the result does
+// not depend on scheduling.  The depth-only quantities (the F-number aperture
+// aDT and 1/aDT, four IEEE divisions per depth) come from per-frame planes
+// built once.
+//
+// What bounds it: 16 frames of 128 lines x 2080 depths x 64 elements take
+// 0.56 ms (0.75 ms with one element per wave, a share handed from lane to
+// lane and an 8 + 4 byte depth entry): the address unit is busy 90 % and the
+// VALU 85 % of that time, HBM (0.45 GB read, 1.07 GB written) a third.  Two
+// elements per wave share a depth's position, aperture and beta; 3 and 4 cost
+// waves (their rings) and time the same and 7 % more.  Loads and stores
+// complete in one order, so the depth loop keeps a fixed number of stores per
+// chunk and uses its d/dc loads after them: a wait for loads then never
+// includes the chunk's own stores.  A window of the RF in LDS for d/dc waited
+// for its own loads in the loop and took 1.05 ms.
 #include <hip/hip_runtime.h>
 
 #include <cfloat>
@@ -64,10 +75,16 @@ __host__ __device__ inline uint32_t scan_items_start(uint32_t n_d, uint32_t n_el
 }
 constexpr int kBetaTile = 32;
 constexpr int kWave = 64;
-// Each adjoint wave accumulates its RF line in a ring of kRing samples of LDS;
+// Elements of one adjoint wave, waves per workgroup.
+constexpr uint32_t kAdjointElements = 2;
+constexpr uint32_t kAdjointWaves = 4;
+// Each adjoint wave accumulates its RF lines in rings of kRing samples of LDS;
 // samples more than kRingGuard below the delay of the chunk's first depth are
 // final and leave the ring.
 constexpr uint32_t kRing = 256;
+// Planes of the per-frame depth table.
+constexpr uint32_t kDepthPlanes = 3;
+constexpr uint32_t kRingWords = 2 * kRing + 2;
 constexpr int32_t kRingGuard = 32;
 
 // ---- per-frame tables --------------------------------------------------------
@@ -135,7 +152,7 @@ __global__ __launch_bounds__(kTableThreads) void frame_tables_kernel(const Frame
 
 // ---- per-frame depth table ----------------------------------------------------
 
-// {depth, aDT, 1/aDT, 0} per (frame, depth), aDT with the same single-precision
+// Planes of depth, aDT and 1/aDT per (frame, depth), aDT with the same single-precision
 // operations as the forward kernel (das_kernels.hip, after
 // RxSampleBeamformerDelayAndSum.h:167 and RxBeamformerCommon.h:27-33).
 __global__ __launch_bounds__(256) void depth_table_kernel(const float* depths, const float* frame_c, float dt,
@@ -147,7 +164,10 @@ __global__ __launch_bounds__(256) void depth_table_kernel(const float* depths, c
     const float d = depths[i];
     const float c = frame_c[f];
     const float aDT = (((d * dt) * c) / (2.0f * f_number)) / c / dt;
-    reinterpret_cast<float4*>(dtab)[i] = make_float4(d, aDT, 1.0f / aDT, 0.0f);
+    float* const o = dtab + static_cast<size_t>(f) * kDepthPlanes * n_d + r;
+    o[0] = d;
+    o[n_d] = aDT;
+    o[2 * static_cast<size_t>(n_d)] = 1.0f / aDT;
 }
 
 // ---- beta = dL/dy * norm, transposed to [frame][slot][scanline][depth] -------
@@ -184,46 +204,57 @@ __device__ inline double wave_sum(double v) {
     return v;
 }
 
-// Whole-wave DPP shifts by one lane (wave_shl:1, wave_shr:1): lane i reads
-// lane i + 1 (from_next) or lane i - 1 (from_prev); lane 63, resp. lane 0,
-// reads 0.  Called with every lane of the wave active.
-__device__ inline uint32_t from_next(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x130, 0xf, 0xf, false));
-}
-__device__ inline uint32_t from_prev(uint32_t v) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x138, 0xf, 0xf, false));
+// Whole-wave DPP shift by one lane (wave_shr:1): lane i reads lane i - 1,
+// lane 0 reads 0.  Called with every lane of the wave active.
+__device__ inline int32_t from_prev(int32_t v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, true); }
+__device__ inline float from_prev(float v) {
+    return __uint_as_float(static_cast<uint32_t>(from_prev(static_cast<int32_t>(__float_as_uint(v)))));
 }
 
-// Largest wave max of v over the wave (rare paths only).
-__device__ inline uint32_t wave_max(uint32_t v) {
-    for (int o = kWave / 2; o > 0; o >>= 1) v = max(v, static_cast<uint32_t>(__shfl_xor(static_cast<int>(v), o, kWave)));
+__device__ inline uint64_t ballot(bool v) { return __builtin_amdgcn_ballot_w64(v); }
+
+// Largest v of the wave (rare paths only).
+__device__ inline uint32_t wave_max(uint32_t v, uint32_t lane) {
+    for (uint32_t o = kWave / 2; o > 0; o >>= 1)
+        v = max(v, static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(static_cast<int>((lane ^ o) * 4u), static_cast<int>(v))));
     return v;
 }
 
-// Moves samples [from, to) of a wave's RF line from its ring to the output
-// line, in order, and clears their ring slots.  Samples at or beyond
-// from + kRing were never added to (every target lies below base + kRing when
-// it is added and base only grows), so they are written as 0.
-__device__ inline void ring_flush(float* ring, float* out, bool exclusive, uint32_t lane, int32_t from, int32_t to) {
-    for (int32_t u = from + static_cast<int32_t>(lane); u < to; u += kWave) {
-        float v = 0.0f;
-        if (u < from + static_cast<int32_t>(kRing)) {
-            float& slot = ring[static_cast<uint32_t>(u) & (kRing - 1u)];
-            v = slot;
-            slot = 0.0f;
-        }
-        if (exclusive) out[u] = v;
-        else if (v != 0.0f) atomicAdd(&out[u], v);
+// Takes the kWave samples from base on (a multiple of kWave) out of a ring and
+// clears them.  Sample u's slot holds the upper shares of u - 1 and the lower
+// shares of u; the upper shares of the last slot's sample are behind it, and
+// belong to the first slot's sample.  Samples at or beyond base + kRing - 1
+// were never added to, and the slots read for them hold 0 by then.
+__device__ inline float ring_take(float* ring, uint32_t lane, int32_t base) {
+    const uint32_t first = static_cast<uint32_t>(base) & (kRing - 1u);   // (uniform)
+    float2& at = reinterpret_cast<float2*>(ring)[first + lane];
+    float v = at.x + at.y;
+    at = make_float2(0.0f, 0.0f);
+    if (first == 0 && lane == 0) {
+        v += ring[2 * kRing];
+        ring[2 * kRing] = 0.0f;
     }
+    return v;
 }
 
-__global__ __launch_bounds__(256) void das2d_adjoint_kernel(const AdjointArgs a) {
-    extern __shared__ float s_mem[];
-    float* s_lut = s_mem;
-    const uint32_t wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    float* s_ring = s_mem + kWindowEntries + static_cast<size_t>(wave) * kRing;
+// The line's sample u: a store where the wave is its only writer (past the
+// line's end the buffer drops it), else a global atomic.
+template <bool EXCLUSIVE>
+__device__ inline void put_sample(__amdgpu_buffer_rsrc_t line, float* out, int32_t u, int32_t n_s, float v) {
+    if (EXCLUSIVE) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), line, u * 4, 0, 0);
+    else if (v != 0.0f && u < n_s) atomicAdd(&out[u], v);
+}
+
+template <bool GRAD, bool DC, bool EXCLUSIVE>
+__global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(const AdjointArgs a) {
+    __shared__ float s_lut[kWindowEntries];
+    __shared__ __align__(8) float s_rings[GRAD ? kAdjointWaves * kAdjointElements * kRingWords : 1];
+    const uint32_t wave = uniform_u32(threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    float* const s_ring = s_rings + (GRAD ? wave * kAdjointElements * kRingWords : 0);
     for (uint32_t i = threadIdx.x; i < kWindowEntries; i += blockDim.x) s_lut[i] = a.lut[i];
-    for (uint32_t i = lane; i < kRing; i += kWave) s_ring[i] = 0.0f;
+    if (GRAD)
+        for (uint32_t i = lane; i < kAdjointElements * kRingWords; i += kWave) s_ring[i] = 0.0f;
+    __syncthreads();
 
     uint32_t b = blockIdx.x;
     const uint32_t eg = b % a.egroups;
@@ -245,162 +276,225 @@ __global__ __launch_bounds__(256) void das2d_adjoint_kernel(const AdjointArgs a)
     }
     TxDT tx{};
     if (active) tx = sc.tx(k);
-    const int e = static_cast<int>(tx.first_x) + static_cast<int>(eg * a.waves + wave);
-    active = active && e < static_cast<int>(tx.last_x);
-    uint32_t ch = 0;
-    if (active) {
-        if (a.e2c) {
-            const int32_t m = a.e2c[e];
-            active = m >= 0;
-            ch = active ? static_cast<uint32_t>(m) : 0u;
-        } else {
-            ch = static_cast<uint32_t>(e) % a.n_ch;
-        }
-    }
-    __syncthreads();
+    const uint32_t first = tx.first_x + (eg * kAdjointWaves + wave) * kAdjointElements;
 
-    const size_t line = a.rf_frame_stride * f + (static_cast<size_t>(tx.tx_idx) * a.n_ch + ch) * a.n_s;
-    float dc = 0.0f;
-    if (active && a.n_depths > 0u) {
-        const float4* dtab =
-            reinterpret_cast<const float4*>(a.dtab) + static_cast<size_t>(f) * a.depth_frame_stride;
-        const float* beta = a.beta + ((static_cast<size_t>(f) * a.n_slots + q) * a.n_rx + s) * a.n_depths;
-        const float x = sc.x(), dir_x = sc.dir_x(), dir_y = sc.dir_y(), med = sc.max_ed_x();
+    // The wave's elements.  One that is past the aperture or not connected has
+    // an infinite distance, so that no lane takes it, and no lines.
+    float xe[kAdjointElements], dx[kAdjointElements], dc[kAdjointElements];
+    int32_t base[kAdjointElements];   // samples below it are final and in out[]; the ring holds the next kRing - 1
+    size_t line[kAdjointElements];
+    bool on[kAdjointElements];
+    __amdgpu_buffer_rsrc_t rf[kAdjointElements], grad[kAdjointElements];
+    float near = INFINITY;
+    bool any = false;
+    const float x = sc.x();
+#pragma unroll
+    for (uint32_t n = 0; n < kAdjointElements; n++) {
+        const uint32_t e = first + n;
+        on[n] = active && e < tx.last_x;
+        uint32_t ch = 0;
+        if (on[n]) {
+            const int32_t m = a.e2c ? a.e2c[e] : static_cast<int32_t>(e % a.n_ch);
+            on[n] = m >= 0;
+            ch = on[n] ? static_cast<uint32_t>(m) : 0u;
+        }
+        xe[n] = on[n] ? a.ex[static_cast<size_t>(f) * a.el_frame_stride + e] : 0.0f;
+        dx[n] = on[n] ? xe[n] - x : INFINITY;
+        near = fminf(near, fabsf(dx[n]));
+        any = any || on[n];
+        line[n] = a.rf_frame_stride * f + (static_cast<size_t>(tx.tx_idx) * a.n_ch + ch) * a.n_s;
+        if (GRAD) grad[n] = rf_resource(a.grad_rf + line[n], on[n] ? a.n_s * 4u : 0u);
+        if (DC) rf[n] = rf_resource(a.rf + line[n], on[n] ? a.n_s * 4u : 0u);
+        base[n] = 0;
+        dc[n] = 0.0f;
+    }
+    if (any && a.n_depths > 0u) {
+        // (reads past the last depth give 0: no aperture, no beta)
+        const float* const planes = a.dtab + static_cast<size_t>(f) * kDepthPlanes * a.n_depths;
+        const __amdgpu_buffer_rsrc_t depth = rf_resource(planes, a.n_depths * 4u);
+        const __amdgpu_buffer_rsrc_t aperture = rf_resource(planes + a.n_depths, a.n_depths * 4u);
+        const __amdgpu_buffer_rsrc_t inverse =
+            rf_resource(planes + 2 * static_cast<size_t>(a.n_depths), a.n_depths * 4u);
+        const __amdgpu_buffer_rsrc_t beta = rf_resource(
+            a.beta + ((static_cast<size_t>(f) * a.n_slots + q) * a.n_rx + s) * a.n_depths, a.n_depths * 4u);
+        const float dir_x = sc.dir_x(), dir_y = sc.dir_y(), med = sc.max_ed_x();
         // 1 / fminf(aDT, med) is 1/aDT below med and 1/med from there on.
         const float inv_med = 1.0f / med;
-        const float xe = a.ex[static_cast<size_t>(f) * a.el_frame_stride + e];
-        const float dx = xe - x;
-        const float* rf_line = a.rf + line;
-        const bool want_dc = a.dc_part != nullptr;
-        float* out = a.grad_rf ? a.grad_rf + line : nullptr;
-        const bool exclusive = a.exclusive != 0;
         const int32_t n_s = static_cast<int32_t>(a.n_s);
-        // Samples below base are final and in out[]; [base, base + kRing)
-        // are accumulated in the ring (slot = sample mod kRing).
-        int32_t base = 0;
-        const uint32_t last = a.n_depths - 1u;
-        // This iteration's depth entry and beta; the next iteration's are
-        // loaded at the top of each iteration (clamped to the last depth).
-        float4 dv = dtab[min(lane, last)];
-        float btv = beta[min(lane, last)];
-        // Lanes are consecutive depths, so their delays (never decreasing with
-        // depth) are sorted across the wave.  A lane whose upper sample ui+1
-        // is the next lane's lower sample hands its share to that lane, which
-        // adds it with its own: one add instead of two for that sample.
-        for (uint32_t r0 = 0; r0 < a.n_depths; r0 += kWave) {
-            const uint32_t r = r0 + lane;
-            const bool valid = r < a.n_depths;
-            const float d = dv.x, aDT = dv.y;
-            const float inv = aDT < med ? dv.z : inv_med;
-            const float bt = valid ? btv : 0.0f;
-            {
-                const uint32_t rn = min(r + kWave, last);
-                dv = dtab[rn];
-                btv = beta[rn];
+        const uint32_t last_bits = last_sample_bits(a.n_s);
+        float w_far[kAdjointElements];
+        bool empty[kAdjointElements];   // nothing was added to the ring yet
+#pragma unroll
+        for (uint32_t n = 0; n < kAdjointElements; n++) {
+            w_far[n] = s_lut[window_index(dx[n] * inv_med)];
+            empty[n] = true;
+        }
+        // The first chunk with a depth whose aperture reaches the wave's nearest
+        // element, where the depths do not decrease: the chunks above add
+        // nothing.  (Not a test in the loop: a chunk that is passed over there
+        // would leave the loop without its stores, and with their number open
+        // every wait for a load would be a wait for the stores as well.)
+        uint32_t chunk = 0;
+        if (a.depths_sorted) {
+            const uint32_t chunks = (a.n_depths + kWave - 1u) / kWave;
+            for (; chunk < chunks; chunk += kWave) {
+                const uint32_t r = min((chunk + lane) * kWave + kWave, a.n_depths) - 1u;
+                const uint64_t reached = ballot(near <= load_rf<float>(aperture, r));
+                if (reached != 0) {
+                    chunk += static_cast<uint32_t>(__builtin_ctzll(reached));
+                    break;
+                }
             }
+        }
+        // This iteration's depth entry and beta; the next iteration's are
+        // loaded at the top of each iteration.
+        using Quad = uint32_t __attribute__((ext_vector_type(4)));
+        uint32_t r0 = chunk * kWave;
+        float next_d = load_rf<float>(depth, r0 + lane), next_aDT = load_rf<float>(aperture, r0 + lane);
+        float next_inv = load_rf<float>(inverse, r0 + lane), next_beta = load_rf<float>(beta, r0 + lane);
+        // (waited for here: inside the loop they are older than the d/dc loads
+        // and need no wait of their own, which would reach the stores)
+        asm volatile("" ::"v"(next_d), "v"(next_aDT), "v"(next_inv), "v"(next_beta));
+        for (; r0 < a.n_depths; r0 += kWave) {
+            float d = next_d;
+            const float aDT = next_aDT, inv_aDT = next_inv, bt = next_beta;
+            const uint32_t rn = r0 + kWave + lane;
+            next_d = load_rf<float>(depth, rn);
+            next_aDT = load_rf<float>(aperture, rn);
+            next_inv = load_rf<float>(inverse, rn);
+            next_beta = load_rf<float>(beta, rn);
+            const uint64_t has_beta = ballot(bt != 0.0f);
+            if (r0 + kWave > a.n_depths) {   // (uniform)
+                // lanes past the last depth go on in steps of two samples, so
+                // that their samples stay sorted and apart; they add nothing
+                const uint32_t last = a.n_depths - 1u - r0;
+                const float d_last = __uint_as_float(
+                    static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(__float_as_uint(d)), last)));
+                if (lane > last) d = d_last + 2.0f * static_cast<float>(lane - last);
+            }
+            // (uniform) every lane's aperture is at its largest: one weight per element
+            const bool far = ballot(aDT < med) == 0;
+            const float inv = aDT < med ? inv_aDT : inv_med;
             // Same single-precision operations as the forward kernel.
-            const bool take = valid && bt != 0.0f && fabsf(dx) <= aDT;
-            // No lane of this chunk in the element's aperture (shallow depths
-            // of the outer elements): nothing to add; the ring catches up at
-            // the next chunk that has work.
-            if (__ballot(take) == 0ull) continue;
-            const float w = s_lut[window_index(dx * inv)];
             const float px = x + dir_x * d;
             const float py = dir_y * d;
-            const float ee = xe - px;
-            const float geo = sqrt_rn(ee * ee + py * py) + d;
-            float tau = tx.t0 + geo;
-            tau = tau + a.offset;
-            const int32_t i = static_cast<int32_t>(floorf(tau));
-            const float fr = tau - static_cast<float>(i);
-            const uint32_t ui = static_cast<uint32_t>(i);
-            const float bw = bt * w;
-            const bool inr = take && ui < a.n_s - 1u && tau == tau;   // (a NaN delay converts to sample 0)
-            const bool edge = take && ui == a.n_s - 1u && fr == 0.0f;
-            float g0 = 0.0f, g1 = 0.0f;
-            if (want_dc) {
-                // the two samples of d/dc, issued before the LDS adds
-                g0 = rf_line[inr ? ui : 0u];
-                g1 = rf_line[inr ? ui + 1u : 0u];
+            const float py2 = py * py;
+            float bw[kAdjointElements], fr[kAdjointElements], geo[kAdjointElements];
+            float g0[kAdjointElements], g1[kAdjointElements];
+            int32_t idx[kAdjointElements];
+            uint64_t act[kAdjointElements];   // lanes that have the element in their aperture and their delay in the RF
+            int32_t i_first[kAdjointElements], i_last[kAdjointElements];
+            uint64_t same_prev[kAdjointElements];
+            bool sorted[kAdjointElements];
+#pragma unroll
+            for (uint32_t n = 0; n < kAdjointElements; n++) {
+                const float w = far ? w_far[n] : s_lut[window_index(dx[n] * inv)];
+                const float ee = xe[n] - px;
+                geo[n] = sqrt_rn(ee * ee + py2) + d;
+                float tau = tx.t0 + geo[n];
+                tau = tau + a.offset;
+                act[n] = has_beta & ballot(fabsf(dx[n]) <= aDT) & ballot(__float_as_uint(tau) <= last_bits);
+                const int32_t i = static_cast<int32_t>(tau);   // (a delay in the RF is not negative: its floor)
+                idx[n] = i;
+                fr[n] = __builtin_amdgcn_fractf(tau);
+                bw[n] = bt * w;
+                const int32_t prev = from_prev(i);
+                same_prev[n] = ballot(i == prev) & ~1ull;
+                sorted[n] = (ballot(i < prev) & ~1ull) == 0;
+                i_first[n] = __builtin_amdgcn_readfirstlane(i);
+                i_last[n] = __builtin_amdgcn_readlane(i, kWave - 1);
+                if (DC) {
+                    g0[n] = load_rf<float>(rf[n], static_cast<uint32_t>(i));
+                    g1[n] = load_rf<float>(rf[n], static_cast<uint32_t>(i) + 1u);
+                }
             }
-            if (out) {
-                const float lo = inr ? bw * (1.0f - fr) : (edge ? bw : 0.0f);
-                const float hi = inr ? bw * fr : 0.0f;
-                // link(L -> L+1) = inr(L) && valid(L+1) && ui(L+1) == ui(L) + 1, evaluated
-                // identically by both lanes
-                const uint32_t next_ui = from_next(ui);
-                const uint32_t next_fl = from_next((valid ? 1u : 0u) | (inr ? 2u : 0u));
-                const bool next_valid = (next_fl & 1u) != 0u, next_inr = (next_fl & 2u) != 0u;
-                const bool to_next = inr && next_valid && next_ui == ui + 1u;
-                const uint32_t prev_ui = from_prev(ui);
-                const bool prev_inr = from_prev(inr ? 1u : 0u) != 0u;
-                const float prev_hi = __uint_as_float(from_prev(__float_as_uint(hi)));
-                const bool from_prev_lane = prev_inr && valid && ui == prev_ui + 1u;
-                const float lo_sum = from_prev_lane ? lo + prev_hi : lo;
-                // Targets: ui (lo) and ui + 1 (hi), both below n_s.
-                const bool add_lo = inr || edge || from_prev_lane;
-                const bool add_hi = inr && !to_next;
+#pragma unroll
+            for (uint32_t n = 0; GRAD && n < kAdjointElements; n++) {
+                float* const ring = s_ring + n * kRingWords;
+                float* const out = a.grad_rf + line[n];
+                const int32_t i = idx[n];
+                const float lo = bw[n] * (1.0f - fr[n]), hi = bw[n] * fr[n];
                 // Samples more than a guard below lane 0's (this chunk's
-                // smallest delay) are final: flush them.
-                const int32_t i0 = max(__builtin_amdgcn_readfirstlane(i), -1);
-                const int32_t want = min(i0 - kRingGuard, n_s);
-                if (want > base) {
-                    ring_flush(s_ring, out, exclusive, lane, base, want);
-                    base = want;
+                // smallest delay) are final: flush them, kWave at a time, one
+                // store in every chunk (outside the line where there is
+                // nothing to flush).
+                const int32_t final_to = min(max(i_first[n], 0), n_s) - kRingGuard;
+                if (EXCLUSIVE && empty[n]) {   // (uniform) the samples above the aperture's first: 0
+                    for (; base[n] + 5 * kWave <= final_to; base[n] += 4 * kWave)
+                        __builtin_amdgcn_raw_buffer_store_b128(
+                            Quad{0, 0, 0, 0}, grad[n],
+                            static_cast<int>((static_cast<uint32_t>(base[n]) + 4u * lane) * 4u), 0, 0);
+                    empty[n] = false;
                 }
-                // A target beyond the ring moves the ring up to it (wide
-                // apertures per chunk only).
-                const uint32_t top = add_hi ? ui + 1u : (add_lo ? ui : 0u);
-                if (__ballot(static_cast<int32_t>(top) >= base + static_cast<int32_t>(kRing)) != 0ull) {
-                    const int32_t up = static_cast<int32_t>(__builtin_amdgcn_readfirstlane(wave_max(top))) -
-                                       static_cast<int32_t>(kRing) + 1;
-                    ring_flush(s_ring, out, exclusive, lane, base, up);
-                    base = up;
+                for (; base[n] + 2 * kWave <= final_to; base[n] += kWave)
+                    put_sample<EXCLUSIVE>(grad[n], out, base[n] + static_cast<int32_t>(lane), n_s,
+                                          ring_take(ring, lane, base[n]));
+                float v = 0.0f;
+                int32_t u = n_s;
+                if (base[n] + kWave <= final_to) {
+                    v = ring_take(ring, lane, base[n]);
+                    u = base[n] + static_cast<int32_t>(lane);
+                    base[n] += kWave;
                 }
-                const bool lo_ring = add_lo && static_cast<int32_t>(ui) >= base;
-                const bool hi_ring = add_hi && static_cast<int32_t>(ui + 1u) >= base;
-                const bool below = (add_lo && !lo_ring) || (add_hi && !hi_ring);
-                // Atomic-free form.  A lane whose next lane has the same
-                // sample (both in range) gives that lane its two shares, so
-                // that every sample is written by at most one lane of each of
-                // the two adds below: plain LDS read-add-write.  It holds
-                // when the samples are sorted across the wave, no three
-                // consecutive lanes share one and no other pair does.
-                const bool same_next = inr && next_inr && next_ui == ui;
-                const bool same_prev = prev_inr && inr && ui == prev_ui;
-                const float a_own = lo_sum, b_own = add_hi ? hi : 0.0f;
-                const float a_prev = __uint_as_float(from_prev(__float_as_uint(a_own)));
-                const float a_tot = same_prev ? a_own + a_prev : a_own;
-                const float b_tot = same_prev ? b_own + prev_hi : b_own;
-                const bool do_a = add_lo && !same_next;
-                const bool do_b = (add_hi && !same_next) || same_prev;
-                const uint32_t prev_do = from_prev((do_a ? 1u : 0u) | (do_b ? 2u : 0u));
-                const bool eq_prev = lane > 0u && valid && ui == prev_ui;
-                const bool eq_next = valid && next_valid && next_ui == ui;
-                const bool unsorted = lane > 0u && valid && i < static_cast<int32_t>(prev_ui);
-                const bool dup = eq_prev && (((prev_do & 1u) != 0u && do_a) || ((prev_do & 2u) != 0u && do_b));
-                if (__ballot(below || unsorted || (eq_prev && eq_next) || dup) == 0ull) {
-                    if (do_a) s_ring[ui & (kRing - 1u)] += a_tot;
-                    if (do_b) s_ring[(ui + 1u) & (kRing - 1u)] += b_tot;
-                } else {
-                    // A target below the ring (delays not sorted) is added to
-                    // the flushed output directly.
-                    if (__ballot(below) != 0ull) {
-                        __threadfence();
-                        if (add_lo && !lo_ring) atomicAdd(&out[ui], lo_sum);
-                        if (add_hi && !hi_ring) atomicAdd(&out[ui + 1u], hi);
+                put_sample<EXCLUSIVE>(grad[n], out, u, n_s, v);
+                // Delays do not decrease with depth, so the lanes' samples are
+                // sorted and, where a depth step is at least half a sample, no
+                // three lanes share one: of two lanes with one sample the
+                // upper one adds for both, and one plain LDS read-add-write
+                // per lane holds the sums.
+                const uint64_t pair = same_prev[n] & act[n] & (act[n] << 1);   // takes the lane below's share
+                const float lo_pair = lo + from_prev(lo), hi_pair = hi + from_prev(hi);
+                const bool in_ring = sorted[n] && i_first[n] >= base[n] && i_last[n] - base[n] <= static_cast<int32_t>(kRing) - 2;
+                if (in_ring && (same_prev[n] & (same_prev[n] >> 1)) == 0) {
+                    if (__builtin_amdgcn_inverse_ballot_w64(act[n] & ~(pair >> 1))) {
+                        float* const at = ring + 2u * (static_cast<uint32_t>(i) & (kRing - 1u));
+                        const bool both = __builtin_amdgcn_inverse_ballot_w64(pair);
+                        const float lo_sum = at[1], hi_sum = at[2];
+                        at[1] = lo_sum + (both ? lo_pair : lo);
+                        at[2] = hi_sum + (both ? hi_pair : hi);
                     }
-                    if (lo_ring) atomicAdd(&s_ring[ui & (kRing - 1u)], lo_sum);
-                    if (hi_ring) atomicAdd(&s_ring[(ui + 1u) & (kRing - 1u)], hi);
+                } else {
+                    // Any other chunk: the ring moves up to the largest target
+                    // (wide apertures per chunk only), a target that is then
+                    // below it is added to the flushed output, and the rest
+                    // goes to the ring with LDS atomics.
+                    const bool add = __builtin_amdgcn_inverse_ballot_w64(act[n]);
+                    const int32_t top = static_cast<int32_t>(
+                        uniform_u32(wave_max(add ? static_cast<uint32_t>(i) : 0u, lane)));
+                    for (; top - base[n] > static_cast<int32_t>(kRing) - 2; base[n] += kWave)
+                        put_sample<EXCLUSIVE>(grad[n], out, base[n] + static_cast<int32_t>(lane), n_s,
+                                              ring_take(ring, lane, base[n]));
+                    if (ballot(add && i < base[n]) != 0) {
+                        __threadfence();
+                        if (add && i < base[n]) atomicAdd(&out[i], lo);
+                        if (add && i + 1 < min(base[n], n_s)) atomicAdd(&out[i + 1], hi);
+                    }
+                    if (add) {
+                        float* const at = ring + 2u * (static_cast<uint32_t>(i) & (kRing - 1u));
+                        if (i >= base[n]) atomicAdd(&at[1], lo);
+                        if (i + 1 >= base[n]) atomicAdd(&at[2], hi);
+                    }
                 }
             }
-            if (want_dc && inr) dc += (bw * (g1 - g0)) * geo;
+#pragma unroll
+            for (uint32_t n = 0; DC && n < kAdjointElements; n++) {
+                // (the last sample, with zero fraction, has no slope)
+                const float slope = (bw[n] * (g1[n] - g0[n])) * geo[n];
+                dc[n] += __builtin_amdgcn_inverse_ballot_w64(act[n] & ballot(idx[n] < n_s - 1)) ? slope : 0.0f;
+            }
         }
-        if (out) ring_flush(s_ring, out, exclusive, lane, base, n_s);
+#pragma unroll
+        for (uint32_t n = 0; GRAD && n < kAdjointElements; n++)
+            for (; on[n] && base[n] < n_s; base[n] += kWave)
+                put_sample<EXCLUSIVE>(grad[n], a.grad_rf + line[n], base[n] + static_cast<int32_t>(lane), n_s,
+                                      ring_take(s_ring + n * kRingWords, lane, base[n]));
     }
-    if (a.dc_part) {
-        const double v = wave_sum(static_cast<double>(dc));
-        if (lane == 0) a.dc_part[static_cast<size_t>(blockIdx.x) * a.waves + wave] = v;
+    if (DC) {
+        double v = 0.0;
+#pragma unroll
+        for (uint32_t n = 0; n < kAdjointElements; n++) v += static_cast<double>(dc[n]);
+        v = wave_sum(v);
+        if (lane == 0) a.dc_part[static_cast<size_t>(blockIdx.x) * kAdjointWaves + wave] = v;
     }
 }
 
@@ -459,14 +553,20 @@ hipError_t launch_beta(const float* grad_image, const float* norm, float* beta, 
     return hipGetLastError();
 }
 
-size_t das_adjoint_lds_bytes(uint32_t waves) {
-    return (static_cast<size_t>(kWindowEntries) + static_cast<size_t>(waves) * kRing) * sizeof(float);
+uint32_t das_adjoint_groups(uint32_t aperture) {
+    constexpr uint32_t per_group = kAdjointElements * kAdjointWaves;
+    return aperture == 0 ? 1u : (aperture + per_group - 1u) / per_group;
 }
+uint32_t das_adjoint_waves() { return kAdjointWaves; }
 
 hipError_t launch_das_adjoint(const AdjointArgs& a, uint32_t frames, hipStream_t stream) {
     const uint64_t blocks = static_cast<uint64_t>(frames) * a.n_rx * a.n_slots * a.egroups;
-    dim3 grid(static_cast<uint32_t>(blocks)), block(a.waves * kWave);
-    hipLaunchKernelGGL(das2d_adjoint_kernel, grid, block, das_adjoint_lds_bytes(a.waves), stream, a);
+    dim3 grid(static_cast<uint32_t>(blocks)), block(kAdjointWaves * kWave);
+    if (!a.grad_rf && !a.dc_part) return hipSuccess;
+    auto kernel = das2d_adjoint_kernel<false, true, true>;
+    if (a.grad_rf && a.dc_part) kernel = a.exclusive ? das2d_adjoint_kernel<true, true, true> : das2d_adjoint_kernel<true, true, false>;
+    else if (a.grad_rf) kernel = a.exclusive ? das2d_adjoint_kernel<true, false, true> : das2d_adjoint_kernel<true, false, false>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
     return hipGetLastError();
 }
 
