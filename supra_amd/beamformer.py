@@ -41,8 +41,15 @@ def _dtype_code(t) -> int:
     raise TypeError(f"unsupported element type {t} (int16 or float32)")
 
 
+# The current stream's handle without a Stream object (0.3 us against 2.8 us
+# per call), where this torch has it.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream_handle(stream) -> int:
     if stream is None:
+        if _raw_stream is not None and torch.cuda.is_initialized():
+            return _raw_stream(torch.cuda.current_device())
         return torch.cuda.current_stream().cuda_stream
     if isinstance(stream, int):
         return stream
@@ -126,12 +133,13 @@ class RxBeamformer:
             out = torch.empty(shape, dtype=out_dtype, device=data.device)
         elif tuple(out.shape) != shape or out.dtype != out_dtype or not out.is_contiguous():
             raise ValueError(f"out must be a contiguous {out_dtype} tensor of shape {shape}")
+        n_tx, n_ch, n_s = data.shape[-3:]
         N.check(N.lib().supra_das_run_frames(
-            self._ctx, int(sample_beamformer), frames, C.c_void_p(data.data_ptr()), _dtype_code(data.dtype),
-            raw.num_scanlines, raw.num_received_channels, raw.num_samples, float(raw.sampling_frequency),
+            self._ctx, int(sample_beamformer), frames, data.data_ptr(), _dtype_code(data.dtype),
+            n_tx, n_ch, n_s, float(raw.sampling_frequency),
             float(f_number), float(speed_of_sound_mm_per_s), int(window_type), float(window_parameter),
-            int(bool(interpolate_transmits)), int(additional_offset), C.c_void_p(out.data_ptr()),
-            _dtype_code(out_dtype), C.c_void_p(_stream_handle(stream))))
+            int(bool(interpolate_transmits)), int(additional_offset), out.data_ptr(),
+            _dtype_code(out_dtype), _stream_handle(stream)))
         return USImage(out, (g.num_rx, g.num_depths), {"imageState": "RF", "geometry": g})
 
 

@@ -98,13 +98,35 @@ void build_dt_tables(supra_bf_ctx* ctx, double dt, double c) {
     }
 }
 
+// Kernels of earlier calls (possibly on several streams) may still read the
+// tables.  The wait is here, where they are replaced, and not an event behind
+// every launch: the event costs the host 1.5 us per call and the stream a
+// barrier between two kernels (one 128 x 2080 frame takes 17.4 us per call with
+// it, 14.6 without; another speed of sound uploads its tables anyway).
+static hipError_t wait_for_table_readers(supra_bf_ctx* ctx) {
+    if (!ctx->tables_used) return hipSuccess;
+    hipError_t e = hipDeviceSynchronize();
+    if (e != hipSuccess && !ctx->more_table_streams) {
+        // not allowed while another thread captures a graph: the launches'
+        // streams one by one (a stream that is gone has drained)
+        (void)hipGetLastError();
+        e = hipSuccess;
+        for (hipStream_t s : ctx->table_streams) {
+            const hipError_t es = hipStreamSynchronize(s);
+            if (es != hipSuccess && es != hipErrorInvalidHandle && es != hipErrorContextIsDestroyed) e = es;
+        }
+    }
+    if (e != hipSuccess) return e;
+    ctx->tables_used = ctx->more_table_streams = false;
+    ctx->table_streams.clear();
+    return hipSuccess;
+}
+
 int ensure_dt_tables(supra_bf_ctx* ctx, double dt, double c, hipStream_t stream) {
     if (ctx->cached_dt == dt && ctx->cached_c == c) return SUPRA_OK;
     build_dt_tables(ctx, dt, c);
     hipError_t e;
-    // Kernels of earlier calls (possibly on other streams) may still read the
-    // tables: the upload waits for the last of them.
-    if (ctx->tables_used_recorded && (e = hipStreamWaitEvent(stream, ctx->tables_used, 0)) != hipSuccess)
+    if ((e = wait_for_table_readers(ctx)) != hipSuccess)
         return hip_fail(e, "geometry upload: wait for earlier kernels");
     if ((e = hipMemcpyAsync(ctx->d_scans, ctx->h_scans.data(), ctx->n_rx * sizeof(ScanlineDT), hipMemcpyHostToDevice,
                             stream)) != hipSuccess)
@@ -125,12 +147,22 @@ int ensure_dt_tables(supra_bf_ctx* ctx, double dt, double c, hipStream_t stream)
     return SUPRA_OK;
 }
 
-// Marks the end of a launch that reads the context's dt-space tables.
-int tables_used_on(supra_bf_ctx* ctx, hipStream_t stream) {
-    hipError_t e = hipEventRecord(ctx->tables_used, stream);
-    if (e != hipSuccess) return hip_fail(e, "record table use");
-    ctx->tables_used_recorded = true;
-    return SUPRA_OK;
+// Notes a launch that reads the context's dt-space tables.
+void tables_used_on(supra_bf_ctx* ctx, hipStream_t stream) {
+    ctx->tables_used = true;
+    for (hipStream_t s : ctx->table_streams)
+        if (s == stream) return;
+    if (ctx->table_streams.size() < supra_bf_ctx::kTableStreams) ctx->table_streams.push_back(stream);
+    else ctx->more_table_streams = true;
+}
+
+void context_window_lut(supra_bf_ctx* ctx, int32_t window_type, float window_parameter, float* lut) {
+    if (ctx->lut_type != window_type || !(ctx->lut_parameter == window_parameter)) {
+        build_window_lut(window_type, window_parameter, ctx->lut);
+        ctx->lut_type = window_type;
+        ctx->lut_parameter = window_parameter;
+    }
+    std::memcpy(lut, ctx->lut, sizeof(ctx->lut));
 }
 
 int check_device(const supra_bf_ctx* ctx) {
@@ -222,6 +254,9 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
     // Aperture corners must address existing elements (the reference reads
     // element tables unchecked).
     for (uint32_t i = 0; i < ctx->n_rx; i++) {
+        int32_t sel, mask;
+        float w[4];
+        scanline_selection(ctx->scan_mm[i], &sel, &mask, w);
         for (int k = 0; k < 4; k++) {
             const supra_tx_params& t = ctx->scan_mm[i].tx[k];
             bool bad = ctx->is3d ? (t.last_active_element[0] > ctx->el_layout[0] ||
@@ -231,6 +266,8 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
                 delete ctx;
                 return fail(SUPRA_ERR_INVALID_ARG, "create: scanline %u transmit %d aperture exceeds the array", i, k);
             }
+            if (k == sel) ctx->tx_selected = std::max<uint64_t>(ctx->tx_selected, t.tx_scanline_idx + 1ull);
+            if ((mask >> k) & 1) ctx->tx_weighted = std::max<uint64_t>(ctx->tx_weighted, t.tx_scanline_idx + 1ull);
             if (t.last_active_element[1] > t.first_active_element[1])
                 ctx->max_rows = std::max<uint32_t>(ctx->max_rows, t.last_active_element[1] - t.first_active_element[1]);
             if (t.last_active_element[0] > t.first_active_element[0])
@@ -243,10 +280,7 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
         delete ctx;
         return fail(SUPRA_ERR_NO_DEVICE, "create: no HIP device: %s", hipGetErrorString(e));
     }
-    if ((e = hipEventCreateWithFlags(&ctx->tables_used, hipEventDisableTiming)) != hipSuccess) {
-        delete ctx;
-        return hip_fail(e, "create: event");
-    }
+    ctx->table_streams.reserve(supra_bf_ctx::kTableStreams);
     if ((e = hipMalloc(&ctx->d_scans, ctx->n_rx * sizeof(ScanlineDT))) != hipSuccess ||
         (e = hipMalloc(&ctx->d_depths, ctx->n_depths * sizeof(float))) != hipSuccess ||
         (e = hipMalloc(&ctx->d_ex, ctx->n_el * sizeof(float))) != hipSuccess ||
@@ -307,7 +341,7 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
                     num_channels);
     // Transmit indices the kernels will read (RxBeamformerCuda.cu:299-303
     // leaves such pixels unwritten; here the call is rejected instead).
-    for (uint32_t i = 0; i < ctx->n_rx; i++) {
+    for (uint32_t i = 0; (interpolate_transmits ? ctx->tx_weighted : ctx->tx_selected) > num_tx && i < ctx->n_rx; i++) {
         const supra_scanline_rx& s = ctx->scan_mm[i];
         int32_t sel, mask;
         float w[4];
@@ -358,7 +392,7 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
     a.offset = static_cast<float>(additional_offset);
     a.far_ok = ctx->far_ok ? 1 : 0;
     a.grid_ok = ctx->grid_ok && ctx->max_rows <= 32 ? 1 : 0;
-    build_window_lut(window_type, window_parameter, a.lut);
+    context_window_lut(ctx, window_type, window_parameter, a.lut);
 
     hipError_t e;
     if (sample_beamformer == SUPRA_BF_COHERENCE_FACTOR && !ctx->is3d)
@@ -369,7 +403,8 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
         e = launch_das(a, rf_dtype, out_dtype, ctx->is3d, sample_beamformer == SUPRA_BF_TEST_SIGNAL,
                        interpolate_transmits != 0, ctx->d_e2c != nullptr, hs);
     if (e != hipSuccess) return hip_fail(e, "das: launch");
-    return tables_used_on(ctx, hs);
+    tables_used_on(ctx, hs);
+    return SUPRA_OK;
 }
 
 extern "C" int supra_das_run(supra_bf_ctx* ctx, int32_t sample_beamformer, const void* rf, int32_t rf_dtype,
@@ -484,7 +519,7 @@ extern "C" int supra_rawdelay_run(supra_bf_ctx* ctx, const void* rf, int32_t rf_
     a.out = out;
     hipError_t e = launch_rawdelay(a, rf_dtype, out_dtype, ctx->is3d, hs);
     if (e != hipSuccess) return hip_fail(e, "rawdelay: launch");
-    if ((st = tables_used_on(ctx, hs)) != SUPRA_OK) return st;
+    tables_used_on(ctx, hs);
     if (out_sampling_frequency_hz) {
         // RawDelay.cu:48, :642: depth of the last sample / c / N_d.
         const double depth = ctx->depths_mm.back();
@@ -516,7 +551,8 @@ extern "C" int supra_mv_das_run(supra_bf_ctx* ctx, const void* rf, int32_t rf_dt
     st = launch_mv_fused(g, rf_dtype, sub_array_size, temporal_smoothing, sub_array_scaling_power, compute_means,
                          loading_factor, out, out_dtype, hs);
     if (st != SUPRA_OK) return st;
-    return tables_used_on(ctx, hs);
+    tables_used_on(ctx, hs);
+    return SUPRA_OK;
 }
 
 // ---- differentiable 2D DAS -----------------------------------------------------

@@ -31,10 +31,18 @@ struct supra_bf_ctx {
     std::vector<ScanlineDT> h_scans;
     std::vector<float> h_depths, h_ex, h_ey;
     double cached_dt = 0, cached_c = 0;
-    // Recorded after every launch that reads d_scans/d_depths/d_ex/d_ey; a
-    // table upload for another (dt, c) waits for it.
-    hipEvent_t tables_used = nullptr;
-    bool tables_used_recorded = false;
+    // Launches have read d_scans/d_depths/d_ex/d_ey since their upload, on
+    // these streams (the first kTableStreams distinct ones): an upload for
+    // another (dt, c) waits for them.
+    static constexpr size_t kTableStreams = 16;
+    bool tables_used = false, more_table_streams = false;
+    std::vector<hipStream_t> table_streams;
+    // Transmits that the selected, resp. all weighted transmits of the
+    // scanlines address (largest index + 1).
+    uint64_t tx_selected = 0, tx_weighted = 0;
+    // The last window table of the delay-and-sum entry points.
+    int32_t lut_type = -1;
+    float lut_parameter = 0.0f, lut[supra_amd::kWindowEntries];
     bool far_ok = false;   // dt-space depths are >= 0 and non-decreasing
     bool grid_ok = false;     // 3D: dt-space element (ix, iy) is at (X[ix], Z[iy])
     uint32_t max_rows = 0;    // 3D: largest last_y - first_y over scanlines and transmits
@@ -67,7 +75,6 @@ struct supra_bf_ctx {
     void* noalloc_scratch = nullptr;
 
     ~supra_bf_ctx() {
-        if (tables_used) (void)hipEventDestroy(tables_used);
         (void)hipFree(d_scans);
         (void)hipFree(d_depths);
         (void)hipFree(d_ex);
@@ -93,7 +100,9 @@ int hip_fail(hipError_t e, const char* what);
 void build_dt_tables(supra_bf_ctx* ctx, double dt, double c);
 int ensure_dt_tables(supra_bf_ctx* ctx, double dt, double c, hipStream_t stream);
 int check_device(const supra_bf_ctx* ctx);
-int tables_used_on(supra_bf_ctx* ctx, hipStream_t stream);
+void tables_used_on(supra_bf_ctx* ctx, hipStream_t stream);
+// build_window_lut() through the context's copy of the last table.
+void context_window_lut(supra_bf_ctx* ctx, int32_t window_type, float window_parameter, float* lut);
 int check_rawdelay_call(const supra_bf_ctx* ctx, const char* what, int32_t rf_dtype, uint32_t num_tx,
                         uint32_t num_channels, uint32_t num_samples, double fs, double f_number, double c,
                         int32_t window_type, bool allow3d);
