@@ -72,6 +72,13 @@ constexpr int kChunk3D = 128;
 constexpr int kW2Entries = kWindowEntries * kWindowEntries;
 constexpr uint32_t kNotConnected = 0xffffffffu;
 
+// Square root of a positive normal x (see sqrt_rn).
+__device__ inline float sqrt_pos(float x) {
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y;
+    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+}
+
 struct Pixel2D {
     float d, aDT, inv, px, py2;
 };
@@ -96,29 +103,33 @@ struct Sums2D {
     float sample = 0.0f, wsum = 0.0f, cs = 0.0f, te = 0.0f;
     int nadd = 0;
     // The element's contribution in gather()'s operations.  A skipped element
-    // adds +0 (int16: no sum is ever -0) or leaves the sums selected unchanged.
-    template <typename RFT>
+    // adds +-0 (int16: no sum is ever -0) or leaves the sums selected unchanged.
+    // ALL: every element adds (far field, all connected, interior).
+    template <typename RFT, bool PLAIN, bool ALL>
     __device__ inline void add(Gather2D<RFT> g) {
-        // (opaque: the compiler would otherwise branch around the weight's
-        // table read, and a batch's gathers would no longer go out together)
-        asm volatile("" : "+v"(g.w));
-        g.w = g.member ? g.w : 0.0f;
+        if (!ALL) {
+            // (opaque: the compiler would otherwise branch around the weight's
+            // table read, and a batch's gathers would no longer go out together)
+            asm volatile("" : "+v"(g.w));
+            g.w = g.member ? g.w : 0.0f;
+            nadd += g.member ? 1 : 0;
+        }
         // a skipped element adds +0 to wsum (never -0: window weights are >= 0) and 0 to n
         wsum += g.w;
-        nadd += g.member ? 1 : 0;
         const float lerp = (1.0f - g.f) * g.v0 + g.f * g.v1;
+        const bool in = PLAIN ? g.member : g.add;
         if constexpr (KIND == SUPRA_BF_COHERENCE_FACTOR) {
-            float v = std::is_same_v<RFT, int16_t> ? lerp : (g.edge ? g.v0 : lerp);
-            v = g.add ? v : 0.0f;
+            float v = PLAIN || std::is_same_v<RFT, int16_t> ? lerp : (g.edge ? g.v0 : lerp);
+            if (!ALL) v = in ? v : 0.0f;
             sample += g.w * v;
             cs += v;
             te += v * v;
         } else if constexpr (std::is_same_v<RFT, int16_t>) {
             const float contrib = g.w * lerp;
-            sample += g.add ? contrib : 0.0f;
+            sample += PLAIN || in ? contrib : 0.0f;
         } else {
-            const float contrib = g.w * (g.edge ? g.v0 : lerp);
-            sample = g.add ? sample + contrib : sample;
+            const float contrib = g.w * (!PLAIN && g.edge ? g.v0 : lerp);
+            sample = ALL || in ? sample + contrib : sample;
         }
     }
     __device__ inline float result() const {
@@ -131,17 +142,20 @@ struct Sums2D {
 // Elements [0, cnt) of the current LDS chunk for one 2D pixel
 // (RxSampleBeamformerDelayAndSum.h:150-199), in batches of kBatch2D whose
 // delays and gathers all go out before the first is consumed; weights, counts
-// and samples are added in element order.  One linear_2d frame (128 lines x
-// 2080 depths x 64-element aperture, int16) takes 17.5 us with this loop, no branch
-// per element and the near field's range below (25.7 us with a branch around
-// each element's aperture test and its own range test); it is bound by the
-// VALU, ~30 instructions per element with two waves per SIMD.  Batches of 2,
-// 4, 8 and 16 elements (frame / four transmits / coherence factor, us):
-// 24.9/58.4/46.0, 20.9/45.4/38.5, 21.1/56.7/46.9, 30.6/91.8/60.5 (before the
-// range: past 8 the registers cost a wave per SIMD).
+// and samples are added in element order.  It is bound by the VALU (83 % busy),
+// 24 to 34 instructions per element with four waves per SIMD.  One linear_2d
+// frame (128 lines x 2080 depths, 64-element aperture, int16) takes 14.2 us
+// per call with it: 25.7 with a branch around each element's aperture and
+// range tests, 17.5 without branches and with the near field's range below,
+// 14.6 without an event behind each launch, 14.2 with the plain form (four
+// transmits 38.4 -> 35.3, coherence factor 31.8 -> 30.3).  Batches of 4, 6 and
+// 8 elements (frame / four transmits / coherence factor, us): 14.2/35.3/30.3,
+// 13.3/37.9/31.2, 14.6/37.3/32.5; 2 and 16 lose 20 % and more.
 constexpr int kBatch2D = 4;
 
-template <typename RFT, bool FAR, bool VERT, bool MAP>
+// PLAIN: no offset, every delay in [0, N-1) and every vertical distance above 0
+// (decided per unit, see das2d_tile): nothing to add, test or guard.
+template <typename RFT, bool FAR, bool VERT, bool MAP, bool PLAIN>
 __device__ inline Gather2D<RFT> element2d_issue(__amdgpu_buffer_rsrc_t rf, uint32_t last_bits, float t0, float offset,
                                                 const Pixel2D& p, const float* s_xe, const float* s_dx,
                                                 const float* s_dx2, const float* s_w, const uint32_t* s_off,
@@ -164,22 +178,26 @@ __device__ inline Gather2D<RFT> element2d_issue(__amdgpu_buffer_rsrc_t rf, uint3
         const float e = s_xe[j] - p.px;
         q = e * e + p.py2;
     }
-    float tau = t0 + (sqrt_rn(q) + p.d);
-    tau = tau + offset;
+    float tau = t0 + ((PLAIN ? sqrt_pos(q) : sqrt_rn(q)) + p.d);
+    if (!PLAIN) tau = tau + offset;
     const uint32_t ui = static_cast<uint32_t>(tau);     // (outside the RF: some sample, or none, that is not added)
     g.f = __builtin_amdgcn_fractf(tau);
     g.v0 = load_rf<RFT>(rf, off + ui);
     g.v1 = load_rf<RFT>(rf, off + ui + 1u);
-    g.add = member & (__float_as_uint(tau) <= last_bits);
-    g.edge = !std::is_same_v<RFT, int16_t> && __float_as_uint(tau) == last_bits;
+    if (!PLAIN) {
+        g.add = member & (__float_as_uint(tau) <= last_bits);
+        g.edge = !std::is_same_v<RFT, int16_t> && __float_as_uint(tau) == last_bits;
+    }
     return g;
 }
 
-template <typename RFT, int KIND, bool FAR, bool VERT, bool MAP>
+template <typename RFT, int KIND, bool FAR, bool VERT, bool MAP, bool PLAIN>
 __device__ inline void elements2d(__amdgpu_buffer_rsrc_t rf, uint32_t last_bits, float t0, float offset,
                                   const Pixel2D& p, const float* s_xe, const float* s_dx, const float* s_dx2,
                                   const float* s_w, const uint32_t* s_off, const float* s_lut, int cnt, float aDT_max,
                                   Sums2D<KIND>& sums) {
+    constexpr bool ALL = PLAIN && FAR && !MAP;
+    if (ALL) sums.nadd += cnt;
     int j = 0;
     if (!FAR) {
         // near field: only the elements between the first and the last that a
@@ -202,13 +220,14 @@ __device__ inline void elements2d(__amdgpu_buffer_rsrc_t rf, uint32_t last_bits,
         Gather2D<RFT> g[kBatch2D];
 #pragma unroll
         for (int u = 0; u < kBatch2D; u++)
-            g[u] = element2d_issue<RFT, FAR, VERT, MAP>(rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off,
+            g[u] = element2d_issue<RFT, FAR, VERT, MAP, PLAIN>(rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off,
                                                         s_lut, j + u);
 #pragma unroll
-        for (int u = 0; u < kBatch2D; u++) sums.add(g[u]);
+        for (int u = 0; u < kBatch2D; u++) sums.template add<RFT, PLAIN, ALL>(g[u]);
     }
     for (; j < cnt; j++)
-        sums.add(element2d_issue<RFT, FAR, VERT, MAP>(rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off, s_lut, j));
+        sums.template add<RFT, PLAIN, ALL>(element2d_issue<RFT, FAR, VERT, MAP, PLAIN>(
+            rf, last_bits, t0, offset, p, s_xe, s_dx, s_dx2, s_w, s_off, s_lut, j));
 }
 
 // RxSampleBeamformerTestSignal::sampleBeamform2D (RxSampleBeamformerTestSignal.h:87-133):
@@ -369,6 +388,14 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
             const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
             const uint32_t last_bits = last_sample_bits(a.n_s);
             const bool far = a.far_ok && aDT0 >= tx.far_thr;
+            // far_thr bounds |xe - x| over the aperture's connected elements,
+            // so every delay of the lane lies between t0 + d and `hi` (with
+            // room for the roundings)
+            const float e_max = (tx.far_thr + fabsf(p.px - sc.x())) * 1.00001f;
+            const float hi = (tx.t0 + (sqrtf(e_max * e_max + p.py2) + p.d)) * 1.00001f + 0.01f;
+            const bool plain = a.far_ok && a.offset == 0.0f && tx.t0 + d0 >= 0.0f &&
+                               __builtin_amdgcn_ballot_w64(t.valid && !(hi < static_cast<float>(a.n_s - 1u) &&
+                                                                        p.py2 >= 1e-20f)) == 0;
             Sums2D<KIND> sums;
             const int first = tx.first_x, last = tx.last_x;
             for (int base = first; base < last; base += kChunk2D) {
@@ -392,20 +419,20 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
                     s_off[j] = (ch == kNotConnected) ? kNotConnected : ch * a.n_s;
                 }
                 wave_sync_2d();
+                const auto run = [&](auto is_far, auto is_vertical, auto is_plain) {
+                    elements2d<RFT, KIND, is_far.value, is_vertical.value, MAP, is_plain.value>(
+                        rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2, s_w, s_off, s_lut, cnt, aDT1, sums);
+                };
+                const auto with_plain = [&](auto is_far, auto is_vertical) {
+                    if (plain) run(is_far, is_vertical, std::true_type{});
+                    else run(is_far, is_vertical, std::false_type{});
+                };
                 if (far) {
-                    if (vertical)
-                        elements2d<RFT, KIND, true, true, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
-                                                               s_w, s_off, s_lut, cnt, aDT1, sums);
-                    else
-                        elements2d<RFT, KIND, true, false, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
-                                                                s_w, s_off, s_lut, cnt, aDT1, sums);
+                    if (vertical) with_plain(std::true_type{}, std::true_type{});
+                    else with_plain(std::true_type{}, std::false_type{});
                 } else {
-                    if (vertical)
-                        elements2d<RFT, KIND, false, true, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx, s_dx2,
-                                                                s_w, s_off, s_lut, cnt, aDT1, sums);
-                    else
-                        elements2d<RFT, KIND, false, false, MAP>(rsrc, last_bits, tx.t0, a.offset, p, s_xe, s_dx,
-                                                                 s_dx2, s_w, s_off, s_lut, cnt, aDT1, sums);
+                    if (vertical) with_plain(std::false_type{}, std::true_type{});
+                    else with_plain(std::false_type{}, std::false_type{});
                 }
             }
             s_local = sums.result();
@@ -919,13 +946,6 @@ struct Grid3D {
     float az2[kGridY];          // (Z[ey] - pz)^2
     uint32_t iz4[kGridY / 4];   // near field: 4 x window index of four rows, one byte each
 };
-
-// Square root of a positive normal x (see sqrt_rn).
-__device__ inline float sqrt_pos(float x) {
-    const float y = __builtin_amdgcn_rsqf(x);
-    const float g = x * y;
-    return fmaf(fmaf(-g, g, x), 0.5f * y, g);
-}
 
 // Columns [0, nx) of the staged pass; `ex` and `off` of the first one.
 template <typename RFT, bool FAR, bool INTERIOR>
