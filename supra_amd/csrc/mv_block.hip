@@ -33,9 +33,10 @@
 // Bound by the FP64 pipe at L = 32: the matrix instructions (26 % of the time)
 // and the vector instructions (49 %) of the waves of a SIMD add up.  At L = 64
 // the matrices fill the LDS and one wave per SIMD waits for itself.
-// 128 x 2080 samples, L = 32, T = 5: 0.69 ms against 2.01 ms of
-// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 2.01 ms against
-// 9.49 ms; relative error of the image against FP64 1.4e-6 against 1.9e-6.
+// 128 x 2080 samples, L = 32, T = 5: 0.66 ms against 2.01 ms of
+// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 0.95 ms against
+// 9.51 ms (in both, windows of few terms take the short way below);
+// relative error of the image against FP64 1.3e-6 against 2.1e-6.
 // Summing the blocks off the first column by differences along the block
 // diagonals (fewer matrix instructions, but longer serial chains) and running
 // the two accumulations of a sub-block side by side were slower (2.49 and
@@ -83,6 +84,12 @@ struct Gram {
     float* mats;
     int rs, mean_stride, matrix;
     int T, n_d, h_lo;
+    uint32_t zero_row;     // first of 16 kBlocks + 4 zeros in xs: row 0's padding
+    uint32_t codes;        // lane l: code[l] (the first 64 samples without a wait for LDS)
+    __device__ inline uint32_t code_of(int h) const {
+        return static_cast<uint32_t>(h < 64 ? __builtin_amdgcn_readlane(static_cast<int>(codes), h)
+                                            : __builtin_amdgcn_readfirstlane(static_cast<int>(code[h])));
+    }
 };
 
 __device__ inline double4v mfma64(float a, float b, double4v c) {
@@ -341,9 +348,198 @@ __device__ __attribute__((always_inline)) inline void eliminate_from(System<LMAX
     }
 }
 
+// ---- few terms: the system in the space of the terms ---------------------------
+
+// Where the apertures are hardly longer than the sub-arrays, a window holds
+// only a few sub-array vectors: with T = 5 and one sub-array per sample, 11.
+// For R~ = delta I + X X^T with the M <= 15 vectors x as columns of X,
+//     R~^-1 1 = (1 - X y) / delta,   (delta I + X^T X) y = X^T 1,
+// so with the Cholesky factor G of the M x M matrix, w = G^-1 X^T 1 and
+// u = G^-1 c (c marks the columns of the output's own sample, xs = X c)
+//     xs^T R~^-1 1 = c^T y = u.w,   1^T R~^-1 1 = (n - w.w) / delta.
+// Everything is FP64: X^T X comes from the matrix cores with the ones as 16th
+// column (its products are X^T 1), 16 lanes factorise a system, and n - w.w is
+// at least n delta / (delta + trace), 1e-4 n for the loadings that come here.
+constexpr int kTerms = 15;
+
+template <int N> __device__ inline double row_bcast(double v) {
+    const uint64_t b = __double_as_longlong(v);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b), 0x150 + N, 0xf, 0xf, true));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), 0x150 + N, 0xf, 0xf, true));
+    return __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo));
+}
+template <int CTRL> __device__ inline double row_ror(double v) {
+    const uint64_t b = __double_as_longlong(v);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b), CTRL, 0xf, 0xf, true));
+    const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), CTRL, 0xf, 0xf, true));
+    return __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi) << 32 | lo));
+}
+__device__ inline double row_sum(double v) {
+    v += row_ror<0x128>(v);
+    v += row_ror<0x124>(v);
+    v += row_ror<0x122>(v);
+    v += row_ror<0x121>(v);
+    return v;
+}
+
+// a -= (lane C's lk of this row of 16 lanes) * l.  The s_nop covers the wait
+// states between a VALU write of lk and its DPP read.
+template <int C> __device__ inline void fmac_bcast(double& a, double lk, double l) {
+    asm("s_nop 1\n\tv_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(a) : "v"(lk), "v"(l), "n"(C));
+}
+
+template <bool HALF> __device__ inline void swap_rows(double& x, double& y) {
+    uint64_t a = __double_as_longlong(x), b = __double_as_longlong(y);
+    uint32_t a0 = static_cast<uint32_t>(a), a1 = static_cast<uint32_t>(a >> 32);
+    uint32_t b0 = static_cast<uint32_t>(b), b1 = static_cast<uint32_t>(b >> 32);
+    const auto lo = HALF ? __builtin_amdgcn_permlane32_swap(a0, b0, false, false) : __builtin_amdgcn_permlane16_swap(a0, b0, false, false);
+    const auto hi = HALF ? __builtin_amdgcn_permlane32_swap(a1, b1, false, false) : __builtin_amdgcn_permlane16_swap(a1, b1, false, false);
+    x = __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi[0]) << 32 | lo[0]));
+    y = __longlong_as_double(static_cast<int64_t>(static_cast<uint64_t>(hi[1]) << 32 | lo[1]));
+}
+
+// Row q = lane % 16 of the system of lane / 16: columns 0 .. 14 and X^T 1.
+struct TermSystem {
+    double a[16];
+    double own;         // 1 / pivot of the lane's own row
+    double b1, b2;      // right-hand sides X^T 1 and c
+};
+
+template <int J, int C>
+__device__ __attribute__((always_inline)) inline void eliminate_terms(TermSystem& s, double l) {
+    if constexpr (C < kTerms) {
+        fmac_bcast<C>(s.a[C], l, l);
+        eliminate_terms<J, C + 1>(s, l);
+    }
+}
+template <int J>
+__device__ __attribute__((always_inline)) inline void factor_terms(TermSystem& s, int q, int terms) {
+    if constexpr (J < kTerms) {
+        if (J < terms) {   // uniform
+            const double inv = rsqrt64(row_bcast<J>(s.a[J]));
+            if (q == J) s.own = inv;
+            const double l = q > J ? s.a[J] * inv : 0.0;
+            const double z1 = row_bcast<J>(s.b1) * inv, z2 = row_bcast<J>(s.b2) * inv;
+            s.b1 = fma(-l, z1, s.b1);
+            s.b2 = fma(-l, z2, s.b2);
+            eliminate_terms<J, J + 1>(s, l);
+            factor_terms<J + 1>(s, q, terms);
+        }
+    }
+}
+
+// The outputs of the tile, if each of their windows has at most kTerms terms;
+// false without any work otherwise.  One tile of 16 outputs of 64 rows takes
+// 13 k cycles here and 75 to 98 k with window sums and 64 x 64 systems
+// (pre-delay + 128 x 1750 samples, L = 64, T = 5: 0.95 ms against 2.00).
+template <int LMAX>
+__device__ inline bool solve_few_terms(const MvArgs& a, const Gram& g, const SampleMeta* meta, int t0, int n_out, float2* res,
+                                       int wave) {
+    const int lane = static_cast<int>(threadIdx.x % 64), q = lane % 16, e = lane / 16;
+    if (g.mean || 2 * g.T + 1 > kTerms || n_out > 64) return false;
+    // lane o looks at output o
+    const int ht = t0 + min(lane, n_out - 1) - g.h_lo;
+    const int lo = max(0, ht - g.T), hi = min(g.n_d - 1 - g.h_lo, ht + g.T);
+    int terms = 0;
+    bool bad = false, single = true;
+#pragma unroll
+    for (int j = 0; j < kTerms; j++) {
+        const uint32_t own = g.code[min(lo + j, hi)] >> 10;    // sub-arrays of the sample; 0: a bad one
+        if (lo + j <= hi) {
+            terms += static_cast<int>(own);
+            bad |= own == 0;
+            single &= own == 1;
+        }
+    }
+    const int n_rows = meta[ht].lt;
+    if (__builtin_amdgcn_ballot_w64(terms > kTerms) != 0) return false;
+    const uint64_t bad_outputs = __builtin_amdgcn_ballot_w64(bad);       // output 0
+    const bool all_single = __builtin_amdgcn_ballot_w64(!single) == 0;   // one sub-array in every sample
+    for (int o0 = wave * 4; o0 < n_out; o0 += 4 * Cfg<LMAX>::kWaves) {
+        // column q of X for the four systems: where its samples are
+        const float* x[4];
+        int n[4], n_max = 0, m_max = 0;
+        double mark = 0.0;      // c of the lane's own system (lane / 16)
+#pragma unroll
+        for (int s = 0; s < 4; s++) {
+            const int o = min(o0 + s, n_out - 1);    // a spare system repeats the last sample
+            n[s] = __builtin_amdgcn_readlane(n_rows, o);
+            n_max = max(n_max, n[s]);
+            m_max = max(m_max, __builtin_amdgcn_readlane(terms, o));
+            const int h1 = __builtin_amdgcn_readlane(hi, o);
+            int at = static_cast<int>(g.zero_row), before = 0;      // unused columns read zeros
+            if (all_single) {
+                const int h = __builtin_amdgcn_readlane(lo, o) + q;
+                if (h <= h1) {
+                    at = h * g.rs + static_cast<int>(g.code[h] & 1023u);
+                    if (e == s && t0 + o - g.h_lo == h) mark = 1.0;
+                }
+            } else for (int h = __builtin_amdgcn_readlane(lo, o); h <= h1; h++) {
+                const uint32_t code = g.code_of(h);
+                const int k = q - before, own = static_cast<int>(code >> 10);
+                if (k >= 0 && k < own) {
+                    at = h * g.rs + static_cast<int>(code & 1023u) + k;
+                    if (e == s && t0 + o - g.h_lo == h) mark = 1.0;
+                }
+                before += own;
+            }
+            x[s] = g.xs + at + e;
+        }
+        double4v acc[4];
+#pragma unroll
+        for (int s = 0; s < 4; s++) acc[s] = double4v{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+        for (int i0 = 0; i0 < n_max; i0 += 16) {
+            float v[4][4];
+#pragma unroll
+            for (int s = 0; s < 4; s++)
+#pragma unroll
+                for (int u = 0; u < 4; u++) v[s][u] = x[s][i0 + 4 * u];
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int s = 0; s < 4; s++) {
+                    const float w = i0 + 4 * u + e < n[s] ? (q == kTerms ? 1.0f : v[s][u]) : 0.0f;
+                    acc[s] = mfma64(w, w, acc[s]);
+                }
+        }
+        // lane (e, q) holds columns e, e + 4, .. of row q of all four systems:
+        // transposed to all columns of row q of system e
+        TermSystem sys;
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            double c[4] = {acc[0][v], acc[1][v], acc[2][v], acc[3][v]};
+            swap_rows<true>(c[0], c[2]);
+            swap_rows<true>(c[1], c[3]);
+            swap_rows<false>(c[0], c[1]);
+            swap_rows<false>(c[2], c[3]);
+#pragma unroll
+            for (int k = 0; k < 4; k++) sys.a[4 * v + k] = c[k];
+        }
+        double diag = 0.0;
+#pragma unroll
+        for (int c = 0; c < kTerms; c++) diag = q == c ? sys.a[c] : diag;
+        const int rows = e == 0 ? n[0] : (e == 1 ? n[1] : (e == 2 ? n[2] : n[3]));
+        const double delta = row_sum(diag) / static_cast<double>(rows) * static_cast<double>(a.alpha);
+#pragma unroll
+        for (int c = 0; c < kTerms; c++) sys.a[c] = q == c ? sys.a[c] + delta : sys.a[c];
+        sys.b1 = sys.a[kTerms];
+        sys.b2 = mark;
+        sys.own = 0.0;
+        factor_terms<0>(sys, q, m_max);
+        const bool term = q < m_max;
+        const double w = term ? sys.b1 * sys.own : 0.0, u = term ? sys.b2 * sys.own : 0.0;
+        const double ww = row_sum(w * w), uw = row_sum(u * w);
+        if (q == 0 && o0 + e < n_out)
+            res[o0 + e] = (bad_outputs >> (o0 + e)) & 1 ? make_float2(0.0f, 0.0f)
+                                                        : make_float2(static_cast<float>(uw), static_cast<float>((static_cast<double>(rows) - ww) / delta));
+    }
+    return true;
+}
+
 // The samples of outputs [t0, t0 + n_out) of scanline s.
 template <int LMAX>
-__device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int n_out, int h_lo, const float* xs,
+__device__ inline void solve_outputs(const MvArgs& a, int t0, int n_out, int h_lo, const float* xs,
                                      const SampleMeta* meta, const float* mats, float2* res, int wave) {
     constexpr int kB = LMAX / 16;
     const int lane = static_cast<int>(threadIdx.x % 64), q = lane % 16;
@@ -424,8 +620,12 @@ __device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int
         uz = row_sum(uz);
         if (q == 0 && o0 + lane / 16 < n_out) res[o] = make_float2(uz, bad ? 0.0f : zz);   // zz 0: output 0
     }
-    __syncthreads();
-    // outputs: one lane each (the power and the division once per workgroup)
+}
+
+// The images' samples from (xs^T R~^-1 1, 1^T R~^-1 1): one lane each (the power
+// and the division once per workgroup).
+__device__ inline void write_outputs(const MvArgs& a, uint32_t scan, int t0, int n_out, int h_lo, const SampleMeta* meta,
+                                     const float2* res) {
     if (static_cast<int>(threadIdx.x) < n_out) {
         const int t = t0 + static_cast<int>(threadIdx.x);
         const float2 r = res[threadIdx.x];
@@ -446,29 +646,33 @@ __device__ inline void solve_outputs(const MvArgs& a, uint32_t scan, int t0, int
 template <int LMAX>
 __device__ inline void find_bad(const MvArgs& a, const float* xs, const float* mean, int H, SampleMeta* meta, uint32_t* code) {
     constexpr int kWaves = Cfg<LMAX>::kWaves;
-    const int wave = static_cast<int>(threadIdx.x / 64), lane = static_cast<int>(threadIdx.x % 64);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64));
+    const int lane = static_cast<int>(threadIdx.x % 64);
     const int rs = static_cast<int>(a.rs);
-    for (int h = wave; h < H; h += kWaves) {
-        const SampleMeta m = meta[h];
-        if (__builtin_amdgcn_readfirstlane(m.bad) == 0) {
-            if (lane == 0) code[h] = static_cast<uint32_t>(m.first) | static_cast<uint32_t>(m.kact) << 10;
-            continue;
-        }
-        double r = 0.0;
-        if (lane < m.lt) {
-            for (int k = 0; k < m.kact; k++) {
-                const double x = static_cast<double>(xs[h * rs + m.first + k + lane]);
-                r = fma(x, x, r);
+    for (int h0 = 0; h0 < H; h0 += 64) {
+        const int hl = h0 + lane;
+        const SampleMeta ml = hl < H ? meta[hl] : SampleMeta{0, 0, 0, 0};
+        if (wave == 0 && hl < H && ml.bad == 0) code[hl] = static_cast<uint32_t>(ml.first) | static_cast<uint32_t>(ml.kact) << 10;
+        for (uint64_t left = __builtin_amdgcn_ballot_w64(ml.bad != 0); left != 0; left &= left - 1) {
+            const int h = h0 + __builtin_ctzll(left);
+            if (h % kWaves != wave) continue;
+            const SampleMeta m = meta[h];
+            double r = 0.0;
+            if (lane < m.lt) {
+                for (int k = 0; k < m.kact; k++) {
+                    const double x = static_cast<double>(xs[h * rs + m.first + k + lane]);
+                    r = fma(x, x, r);
+                }
+                if (mean) {
+                    const double mu = static_cast<double>(mean[h * LMAX + lane]);
+                    r -= static_cast<double>(m.kact) * mu * mu;
+                }
             }
-            if (mean) {
-                const double mu = static_cast<double>(mean[h * LMAX + lane]);
-                r -= static_cast<double>(m.kact) * mu * mu;
+            const uint64_t over = __ballot(!(fabsf(static_cast<float>(r)) <= FLT_MAX));
+            if (lane == 0) {
+                meta[h].bad = over != 0 ? 1 : 0;
+                code[h] = over != 0 ? 0u : static_cast<uint32_t>(m.first) | static_cast<uint32_t>(m.kact) << 10;
             }
-        }
-        const uint64_t over = __ballot(!(fabsf(static_cast<float>(r)) <= FLT_MAX));
-        if (lane == 0) {
-            meta[h].bad = over != 0 ? 1 : 0;
-            code[h] = over != 0 ? 0u : static_cast<uint32_t>(m.first) | static_cast<uint32_t>(m.kact) << 10;
         }
     }
 }
@@ -518,9 +722,15 @@ __device__ inline void mv_block_tile(const MvArgs& a, const float* lut, uint32_t
     g.n_d = static_cast<int>(a.n_d);
     g.h_lo = static_cast<int>(h_lo);
     const int n_out = static_cast<int>(t1 - t0);
-    all_window_sums<LMAX>(g, static_cast<int>(t0), n_out, static_cast<int>(a.sub), wave);
+    g.codes = code[min(static_cast<int>(threadIdx.x % 64), H - 1)];
+    g.zero_row = a.n_ch;
+    if (!solve_few_terms<LMAX>(a, g, meta, static_cast<int>(t0), n_out, res, wave)) {   // uniform
+        all_window_sums<LMAX>(g, static_cast<int>(t0), n_out, static_cast<int>(a.sub), wave);
+        __syncthreads();
+        solve_outputs<LMAX>(a, static_cast<int>(t0), n_out, g.h_lo, xs, meta, mats, res, wave);
+    }
     __syncthreads();
-    solve_outputs<LMAX>(a, scan, static_cast<int>(t0), n_out, g.h_lo, xs, meta, mats, res, wave);
+    write_outputs(a, scan, static_cast<int>(t0), n_out, g.h_lo, meta, res);
 }
 
 // Renumbers the workgroups as mv_logical_wg in mv_kernels.hip does: 32

@@ -165,30 +165,43 @@ constexpr int32_t kHuge = 2;
 
 template <int NT, bool HUGE>
 __device__ inline void find_apertures(const MvArgs& a, const float* xs, int H, SampleMeta* meta) {
-    const int wv = threadIdx.x / 64, ln = threadIdx.x % 64;
+    const int wv = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / 64)), ln = threadIdx.x % 64;
     const int n_ch = static_cast<int>(a.n_ch), L = static_cast<int>(a.L), rs = static_cast<int>(a.rs);
-    for (int h = wv; h < H; h += NT / 64) {
-        const float* row = xs + h * rs;
-        int f = -1, l = 0;
-        bool huge = false;
+    constexpr int kSamples = 4, kStep = NT / 64;   // samples of a wave in flight at once
+    for (int h0 = wv; h0 < H; h0 += kSamples * kStep) {
+        int f[kSamples], l[kSamples];
+        bool huge[kSamples];
+#pragma unroll
+        for (int u = 0; u < kSamples; u++) f[u] = -1, l[u] = 0, huge[u] = false;
         for (int cb = 0; cb < n_ch; cb += 64) {
             const int c = cb + ln;
-            const float v = c < n_ch ? row[c] : 0.0f;
-            const uint64_t nz = __ballot(v != 0.0f);
-            if (HUGE) huge |= __ballot(!(fabsf(v) <= 5e17f)) != 0;   // 256 squares of it stay below 1e38
-            if (nz != 0) {
-                if (f < 0) f = cb + __ffsll(static_cast<unsigned long long>(nz)) - 1;
-                l = cb + 63 - __clzll(static_cast<long long>(nz));
+            float v[kSamples];
+#pragma unroll
+            for (int u = 0; u < kSamples; u++)
+                v[u] = c < n_ch && h0 + u * kStep < H ? xs[(h0 + u * kStep) * rs + c] : 0.0f;
+#pragma unroll
+            for (int u = 0; u < kSamples; u++) {
+                const uint64_t nz = __builtin_amdgcn_ballot_w64(v[u] != 0.0f);
+                if (HUGE) huge[u] |= __builtin_amdgcn_ballot_w64(!(fabsf(v[u]) <= 5e17f)) != 0;   // 256 squares of it stay below 1e38
+                if (nz != 0) {
+                    if (f[u] < 0) f[u] = cb + __builtin_ctzll(nz);
+                    l[u] = cb + 63 - __builtin_clzll(nz);
+                }
             }
         }
-        if (f < 0) f = 0;
-        if (ln == 0) {
-            SampleMeta m;
-            m.first = f;
-            m.lt = min(L, l - f + 1);
-            m.kact = min(static_cast<int>(a.K), l - f - m.lt + 2);
-            m.bad = huge ? kHuge : 0;
-            meta[h] = m;
+#pragma unroll
+        for (int u = 0; u < kSamples; u++) {
+            const int h = h0 + u * kStep;
+            if (h >= H) break;
+            if (f[u] < 0) f[u] = 0;
+            if (ln == 0) {
+                SampleMeta m;
+                m.first = f[u];
+                m.lt = min(L, l[u] - f[u] + 1);
+                m.kact = min(static_cast<int>(a.K), l[u] - f[u] - m.lt + 2);
+                m.bad = huge[u] ? kHuge : 0;
+                meta[h] = m;
+            }
         }
     }
 }
