@@ -787,7 +787,7 @@ size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
     // the pre-delay tables are only read before the matrices are written
     const size_t mats = static_cast<size_t>(tile) * (blocks * 160 + blocks * (blocks - 1) / 2 * 256) * 4;
     a.off_fused = static_cast<uint32_t>(off);
-    const size_t fused = a.g.rf ? (kWindowEntries + 4 * static_cast<size_t>(a.n_ch) + 6 * static_cast<size_t>(H)) * 4 : 0;
+    const size_t fused = a.g.rf ? delay_table_floats(a.n_ch, H) * 4 : 0;
     return off + std::max(mats, fused);
 }
 

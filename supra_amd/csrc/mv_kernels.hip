@@ -634,7 +634,7 @@ size_t plan_lds(MvArgs& a, uint32_t tile) {
     const uint32_t ppw = a.L <= 32 ? 2 : 1;   // pixels per wave in phase 3
     off += static_cast<size_t>(a.waves) * ppw * a.wave_bytes;
     a.off_fused = static_cast<uint32_t>(off);
-    if (a.g.rf) off += (kWindowEntries + 4 * static_cast<size_t>(a.n_ch) + 6 * static_cast<size_t>(H)) * 4;
+    if (a.g.rf) off += delay_table_floats(a.n_ch, H) * 4;
     return off;
 }
 

@@ -28,30 +28,42 @@ struct SampleMeta {
     int32_t bad;    // a non-finite covariance: every window holding it ends as NaN -> 0
 };
 
+// LDS floats set aside for the pre-delay tables of a tile of H staged samples
+// (it decides the sizes that fit at all; stage_delayed uses 3 n_ch and 2 H).
+__host__ __device__ inline size_t delay_table_floats(size_t n_ch, size_t H) { return kWindowEntries + 4 * n_ch + 6 * H; }
+
 // Fused mode: the pre-delayed samples of scanline s, depths [h_lo, h_lo+H),
 // computed from the RF exactly as the pre-delay kernel writes them
 // (rawdelay2d_kernel in das_kernels.hip; RawDelay.cu:221-312, 404-468):
 // highest-weight transmit, aperture element c = e - first, w * interp * n/W
 // through clampCast<float>, 0 for c >= last - first.  Same operations in the
 // same order, so the values are bit-identical to the two-kernel path.
+//
+// Half-waves take one element each, lanes = depths: a lane keeps its depth's
+// geometry in registers and no index is divided.  The window weights go to
+// xs first and are added up from there, one lane per depth in element order
+// (the sum is a serial chain, but of additions only); then the samples take
+// their place.  26 depths x 128 elements with 4 waves: 31.7 k cycles with one
+// lane per depth for geometry and weights, 15.5 k now (half of it memory latency).
 template <typename RFT, int NT>
 __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t s, uint32_t h_lo, int H,
                                      float* xs, unsigned char* lds) {
+    constexpr int kRows = NT / 32, kBatch = 8;
     const DasArgs& g = a.g;
-    const int n_ch = static_cast<int>(a.n_ch);
+    const int n_ch = static_cast<int>(a.n_ch), rs = static_cast<int>(a.rs);
     const int hstride = static_cast<int>(a.tile + 2 * a.T);
     float* s_lut = reinterpret_cast<float*>(lds + a.off_fused);
     float* s_xe = s_lut + kWindowEntries;
     float* s_dx = s_xe + n_ch;
-    float* s_dx2 = s_dx + n_ch;
-    uint32_t* s_off = reinterpret_cast<uint32_t*>(s_dx2 + n_ch);
-    float* p_d = reinterpret_cast<float*>(s_off + n_ch);
-    float* p_adt = p_d + hstride;
-    float* p_inv = p_adt + hstride;
-    float* p_px = p_inv + hstride;
-    float* p_py2 = p_px + hstride;
-    float* p_scale = p_py2 + hstride;
+    uint32_t* s_off = reinterpret_cast<uint32_t*>(s_dx + n_ch);
+    int* s_count = reinterpret_cast<int*>(s_off + n_ch);
+    float* s_scale = reinterpret_cast<float*>(s_count + hstride);
 
+    const int hl = static_cast<int>(threadIdx.x % 32), cl = static_cast<int>(threadIdx.x / 32);
+    // the first 32 depths stay in registers over the passes (all of them, mostly)
+    const float d_first = g.depths[h_lo + min(hl, H - 1)];
+    const auto aperture = [&](float d) { return (((d * g.dt) * g.c) / (2.0f * g.F)) / g.c / g.dt; };
+    const float aDT_first = aperture(d_first);
     const ScanView sc = scan_view(g.scans, s);
     const int k = sc.sel();
     TxDT tx{};
@@ -61,67 +73,87 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
         cnt = tx.last_x > tx.first_x ? static_cast<int>(tx.last_x - tx.first_x) : 0;
     }
     for (int i = threadIdx.x; i < kWindowEntries; i += NT) s_lut[i] = lut[i];
+    for (int i = threadIdx.x; i < H; i += NT) s_count[i] = 0;
     for (int j = threadIdx.x; j < cnt; j += NT) {
         const int e = static_cast<int>(tx.first_x) + j;
         const float xe = g.ex[e];
-        const float dx = xe - sc.x();
         s_xe[j] = xe;
-        s_dx[j] = dx;
-        s_dx2[j] = dx * dx;
+        s_dx[j] = xe - sc.x();
         s_off[j] = (static_cast<uint32_t>(e) % g.n_ch) * g.n_s;
     }
     __syncthreads();
-    // per-sample geometry and the aperture's weight sum and count
-    for (int h = threadIdx.x; h < H; h += NT) {
-        const float d = g.depths[h_lo + h];
-        const float aDT = (((d * g.dt) * g.c) / (2.0f * g.F)) / g.c / g.dt;
+    for (int h0 = 0; h0 < H; h0 += 32) {
+        const int h = h0 + hl;
+        const float aDT = h0 == 0 ? aDT_first : aperture(g.depths[h_lo + min(h, H - 1)]);
         const float inv = 1.0f / fminf(aDT, sc.max_ed_x());
-        const float py = sc.dir_y() * d;
-        float wsum = 0.0f;
-        int nadd = 0;
-        for (int j = 0; j < cnt; j++) {
-            const float dx = s_dx[j];
-            if (fabsf(dx) <= aDT) {
-                wsum += s_lut[window_index(dx * inv)];
-                nadd++;
-            }
+        int n = 0;
+#pragma unroll 4
+        for (int c = cl; c < cnt; c += kRows) {
+            const float dx = s_dx[c];
+            const float w = s_lut[window_index(dx * inv)];
+            const bool in = fabsf(dx) <= aDT;
+            if (h < H) xs[h * rs + c] = in ? w : 0.0f;     // (0 leaves a sum of weights as it is)
+            n += in ? 1 : 0;
         }
-        float scale = 1.0f;
-        if (nadd > 0) scale = 1.0f / wsum * static_cast<float>(nadd);
-        p_d[h] = d;
-        p_adt[h] = aDT;
-        p_inv[h] = inv;
-        p_px[h] = sc.x() + sc.dir_x() * d;
-        p_py2[h] = py * py;
-        p_scale[h] = scale;
+        if (h < H && n != 0) atomicAdd(&s_count[h], n);
+    }
+    __syncthreads();
+    for (int h = threadIdx.x; h < H; h += NT) {
+        const float* w = xs + h * rs;
+        const int nadd = s_count[h];
+        float wsum = 0.0f;
+        int c = 0;
+        for (; c + 16 <= cnt; c += 16) {
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) v[u] = w[c + u];
+#pragma unroll
+            for (int u = 0; u < 16; u++) wsum += v[u];
+        }
+        for (; c < cnt; c++) wsum += w[c];
+        s_scale[h] = nadd > 0 ? 1.0f / wsum * static_cast<float>(nadd) : 1.0f;
     }
     __syncthreads();
     const bool vertical = (sc.dir_x() == 0.0f);
     const RFT* rf_tx = static_cast<const RFT*>(g.rf) + static_cast<uint64_t>(tx.tx_idx) * g.n_ch * g.n_s;
     const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, g.n_ch * g.n_s * sizeof(RFT));
-    const int rs = static_cast<int>(a.rs);
-#pragma unroll 4
-    for (int idx = threadIdx.x; idx < H * rs; idx += NT) {
-        const int c = idx / H, h = idx % H;
-        float v = 0.0f;
-        if (c < cnt) {
-            float sample = 0.0f;
-            const float dx = s_dx[c];
-            if (fabsf(dx) <= p_adt[h]) {
-                const float w = s_lut[window_index(dx * p_inv[h])];
-                float q;
-                if (vertical) {
-                    q = s_dx2[c] + p_py2[h];
-                } else {
-                    const float e = s_xe[c] - p_px[h];
-                    q = e * e + p_py2[h];
-                }
-                const float tau = tx.t0 + (sqrt_rn(q) + p_d[h]);
-                gather<RFT, false>(rsrc, s_off[c], g.n_s, tau, w, sample);
+    const uint32_t last_bits = last_sample_bits(g.n_s);
+    for (int h0 = 0; h0 < H; h0 += 32) {
+        const int h = h0 + hl;
+        if (h >= H) continue;
+        const float d = h0 == 0 ? d_first : g.depths[h_lo + h];
+        const float aDT = h0 == 0 ? aDT_first : aperture(d);
+        const float px = sc.x() + sc.dir_x() * d;
+        const float py = sc.dir_y() * d;
+        const float py2 = py * py;
+        const float scale = s_scale[h];
+        float* row = xs + h * rs;
+        for (int c0 = cl; c0 < cnt; c0 += kBatch * kRows) {
+            float w[kBatch], f[kBatch], v0[kBatch], v1[kBatch];
+            bool add[kBatch], edge[kBatch];
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                const int c = min(c0 + u * kRows, cnt - 1);
+                const float dx = s_dx[c];
+                const float e = vertical ? dx : s_xe[c] - px;
+                const float tau = tx.t0 + (sqrt_rn(e * e + py2) + d);
+                const uint32_t ui = static_cast<uint32_t>(tau), off = s_off[c];
+                w[u] = row[c];
+                f[u] = __builtin_amdgcn_fractf(tau);
+                v0[u] = load_rf<RFT>(rsrc, off + ui);
+                v1[u] = load_rf<RFT>(rsrc, off + ui + 1u);
+                add[u] = (fabsf(dx) <= aDT) & (__float_as_uint(tau) <= last_bits);
+                edge[u] = !std::is_same_v<RFT, int16_t> && __float_as_uint(tau) == last_bits;
             }
-            v = clamp_cast<float>(sample * p_scale[h]);
+#pragma unroll
+            for (int u = 0; u < kBatch; u++) {
+                const int c = c0 + u * kRows;
+                const float val = edge[u] ? v0[u] : ((1.0f - f[u]) * v0[u] + f[u] * v1[u]);
+                const float sample = 0.0f + (add[u] ? w[u] * val : 0.0f);
+                if (c < cnt) row[c] = clamp_cast<float>(sample * scale);
+            }
         }
-        xs[h * rs + c] = v;
+        for (int c = cnt + cl; c < rs; c += kRows) row[c] = 0.0f;
     }
     __syncthreads();
 }
