@@ -1155,7 +1155,12 @@ __global__ __launch_bounds__(kThreads, 4) void das3d_grid_kernel(const DasArgs a
 // 404-468): for the highest-weight transmit, every aperture element's delayed,
 // apodised sample times n/W goes to out[(s*N_ch + j)*N_d + r], j = e - first;
 // slots j >= last - first are written as 0.  Lanes = depths, so each channel
-// row of the output tile is one coalesced 256-sample store.
+// row of the output tile is one coalesced 256-sample store.  Elements go in
+// batches whose gathers all precede the batch's stores: loads and stores
+// complete in order, so a load after a store waits for it (128 lines x 1750
+// depths x 128 elements: 74 us one by one, 62 in batches).
+constexpr int kBatchDelay = 8;
+
 template <typename RFT, typename OutT>
 __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
     __shared__ float s_lut[kWindowEntries];
@@ -1184,6 +1189,7 @@ __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
         const RFT* rf_tx = static_cast<const RFT*>(a.rf) + static_cast<uint64_t>(t.frame) * a.rf_frame_stride +
                            static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
         const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
+        const uint32_t last_bits = last_sample_bits(a.n_s);
         const int first = tx.first_x, last = tx.last_x;
         // pass 1: aperture weight sum and count
         float wsum = 0.0f;
@@ -1193,11 +1199,19 @@ __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
             __syncthreads();
             for (int j = threadIdx.x; j < cnt; j += kThreads) s_dx[j] = a.ex[base + j] - sc.x();
             __syncthreads();
-            for (int j = 0; j < cnt; j++) {
-                const float dx = s_dx[j];
-                if (fabsf(dx) <= p.aDT) {
-                    wsum += s_lut[window_index(dx * p.inv)];
-                    nadd++;
+            for (int j0 = 0; j0 < cnt; j0 += kBatchDelay) {
+                float w[kBatchDelay];
+                bool in[kBatchDelay];
+#pragma unroll
+                for (int u = 0; u < kBatchDelay; u++) {
+                    const float dx = s_dx[min(j0 + u, cnt - 1)];
+                    w[u] = s_lut[window_index(dx * p.inv)];
+                    in[u] = j0 + u < cnt && fabsf(dx) <= p.aDT;
+                }
+#pragma unroll
+                for (int u = 0; u < kBatchDelay; u++) {
+                    wsum += in[u] ? w[u] : 0.0f;     // (+0 leaves the sum as it is)
+                    nadd += in[u] ? 1 : 0;
                 }
             }
         }
@@ -1217,23 +1231,25 @@ __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
                 s_off[j] = (static_cast<uint32_t>(e) % a.n_ch) * a.n_s;
             }
             __syncthreads();
-            for (int j = 0; j < cnt; j++) {
-                float sample = 0.0f;
-                const float dx = s_dx[j];
-                if (fabsf(dx) <= p.aDT) {
-                    const float w = s_lut[window_index(dx * p.inv)];
-                    float q;
-                    if (vertical) {
-                        q = s_dx2[j] + p.py2;
-                    } else {
-                        const float e = s_xe[j] - p.px;
-                        q = e * e + p.py2;
+            OutT* const row = out + static_cast<uint64_t>(base - first) * a.n_depths + t.r;
+            const auto store = [&](auto is_vertical) {
+                for (int j0 = 0; j0 < cnt; j0 += kBatchDelay) {
+                    Gather2D<RFT> g[kBatchDelay];
+#pragma unroll
+                    for (int u = 0; u < kBatchDelay; u++)
+                        g[u] = element2d_issue<RFT, false, is_vertical.value, false, false>(
+                            rsrc, last_bits, tx.t0, 0.0f, p, s_xe, s_dx, s_dx2, nullptr, s_off, s_lut, min(j0 + u, cnt - 1));
+#pragma unroll
+                    for (int u = 0; u < kBatchDelay; u++) {
+                        const float val = g[u].edge ? g[u].v0 : ((1.0f - g[u].f) * g[u].v0 + g[u].f * g[u].v1);
+                        const float sample = 0.0f + (g[u].add ? g[u].w * val : 0.0f);
+                        if (t.valid && j0 + u < cnt)
+                            row[static_cast<uint64_t>(j0 + u) * a.n_depths] = clamp_cast<OutT>(sample * scale);
                     }
-                    const float tau = tx.t0 + (sqrt_rn(q) + p.d);
-                    gather<RFT, false>(rsrc, s_off[j], a.n_s, tau, w, sample);
                 }
-                if (t.valid) out[static_cast<uint64_t>(base - first + j) * a.n_depths + t.r] = clamp_cast<OutT>(sample * scale);
-            }
+            };
+            if (vertical) store(std::true_type{});
+            else store(std::false_type{});
         }
         written = last > first ? last - first : 0;
     }
