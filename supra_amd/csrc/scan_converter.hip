@@ -317,6 +317,44 @@ __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
     }
 }
 
+// 2D, few frames: one pixel per thread, neighbours from the input, four frames'
+// gathers at once; finding and staging a tile's box (below) pays from
+// kScFewFrames frames on.  The lanes of a wave are neighbouring pixels of a row:
+// where the scanlines are parallel they read one run of samples, and the staged
+// form pays later.
+// us, this form / staged: 764 x 1601 pixels of a linear scan, 1, 4, 8, 12 frames
+// 7.6/11.2, 10.2/14.3, 15.1/21.1, 20.4/24.8, 20 frames
+// 30.7/32.1; 1601 x 1387 of a 60 degree sector,
+// 1, 2, 4 frames 8.8/14.6, 12.3/15.0, 19.3/18.0.
+constexpr uint32_t kScFewFrames = 4, kScFewFramesParallel = 20;
+template <typename InT, typename OutT>
+__global__ __launch_bounds__(256) void scan_convert_few_kernel(const ConvArgs a) {
+    constexpr uint32_t F = 4;
+    const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= a.n_pixels) return;
+    const uint64_t n = a.n_rx, q = a.idx[i];
+    // the last sample row has no successor: the reference's 3D guard, used in 2D too
+    const bool valid = q != kOutside && q + 1 + n < a.in_frame;
+    const float wx = valid ? a.wx[i] : 0.0f, wy = valid ? a.wy[i] : 0.0f;
+    const InT* in = static_cast<const InT*>(a.in);
+    OutT* out = static_cast<OutT*>(a.out) + i;
+    for (uint32_t f0 = 0; f0 < a.num_frames; f0 += F, in += F * a.in_frame, out += F * a.n_pixels) {
+        float val[F] = {};
+        if (valid) {
+#pragma unroll
+            for (uint32_t f = 0; f < F; f++)
+                if (f0 + f < a.num_frames) {
+                    const InT* p = in + f * a.in_frame;
+                    val[f] = (1 - wy) * ((1 - wx) * in_at(p, q) + wx * in_at(p, q + 1)) +
+                             wy * ((1 - wx) * in_at(p, q + n) + wx * in_at(p, q + 1 + n));
+                }
+        }
+#pragma unroll
+        for (uint32_t f = 0; f < F; f++)
+            if (f0 + f < a.num_frames) out[f * a.n_pixels] = clamp_out<OutT>(val[f]);
+    }
+}
+
 // 2D: a workgroup takes 64 x 16 output pixels, 4 consecutive ones per thread,
 // of a range of frames.  The pixels of such a tile read a small box of input
 // samples (rows of consecutive samples x neighbouring scanlines: 10 x 70 for a
@@ -511,6 +549,7 @@ unsigned host_threads() {
 struct supra_scanconv {
     int device = 0;
     bool is3d = false;
+    bool parallel = true;    // every scanline has the first one's direction
     uint32_t layout[2] = {0, 0};
     uint32_t n_samples = 0;
     uint32_t size[3] = {1, 1, 1};
@@ -571,6 +610,8 @@ extern "C" int supra_scanconv_create(const supra_scanline_rx* scanlines, const u
     if (!sc) return fail(SUPRA_ERR_INVALID_ARG, "scanconv: out of host memory");
     sc->is3d = is3d;
     sc->layout[0] = lx, sc->layout[1] = ly;
+    for (uint32_t k = 1; k < lx * ly; k++)
+        for (int d = 0; d < 3; d++) sc->parallel = sc->parallel && scanlines[k].direction[d] == scanlines[0].direction[d];
     sc->n_samples = num_samples;
     sc->resolution = res;
     std::copy(size, size + 3, sc->size);
@@ -774,9 +815,10 @@ extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanline
     a.num_frames = num_frames;
     const size_t out_size = out_dtype == SUPRA_FLOAT32 ? 4 : (out_dtype == SUPRA_INT16 ? 2 : 1);
     const bool packed = a.n_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * out_size) == 0;
-    const uint64_t threads = packed ? a.n_pixels / 4 : a.n_pixels;
+    const bool few = !sc->is3d && num_frames <= (sc->parallel ? kScFewFramesParallel : kScFewFrames);
+    const uint64_t threads = packed && !few ? a.n_pixels / 4 : a.n_pixels;
     dim3 grid(static_cast<uint32_t>((threads + 255) / 256)), block(256);
-    if (!sc->is3d) {
+    if (!sc->is3d && !few) {
         a.size_x = sc->size[0];
         a.size_y = sc->size[1] * sc->size[2];    // (rows of every plane; a 2D scan fills the first)
         const uint64_t tiles_x = (a.size_x + kScTileX - 1) / kScTileX, rows = (a.size_y + kScTileY - 1) / kScTileY;
@@ -793,7 +835,8 @@ extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanline
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define SUPRA_SC_LAUNCH(IN, OUT)                                                                                       \
     do {                                                                                                              \
-        if (!sc->is3d) hipLaunchKernelGGL((scan_convert_tile_kernel<IN, OUT>), grid, block, 0, s, a);                 \
+        if (few) hipLaunchKernelGGL((scan_convert_few_kernel<IN, OUT>), grid, block, 0, s, a);                        \
+        else if (!sc->is3d) hipLaunchKernelGGL((scan_convert_tile_kernel<IN, OUT>), grid, block, 0, s, a);            \
         else if (packed) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 4>), grid, block, 0, s, a);                 \
         else hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 1>), grid, block, 0, s, a);                             \
     } while (0)
