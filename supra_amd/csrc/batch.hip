@@ -208,6 +208,7 @@ DasArgs frame_das_args(const supra_batch* b, const FrameDesc& fd) {
     a.out = it.out;
     a.offset = static_cast<float>(it.additional_offset);
     a.far_ok = ctx->far_ok_mm ? 1 : 0;
+    a.nan_lines = ctx->nan_lines ? 1 : 0;
     return a;
 }
 
@@ -243,7 +244,7 @@ int build_das_queue(supra_batch* b, uint32_t qi) {
         fr.rf_dtype = fd.item.rf_dtype;
         fr.out_dtype = fd.item.out_dtype;
         fr.interp = fd.item.interpolate_transmits ? 1 : 0;
-        fr.map = fd.item.ctx->d_e2c ? 1 : 0;
+        fr.map = fd.item.ctx->d_e2c || fr.a.nan_lines ? 1 : 0;
         fr.n_items = fr.a.n_rx * fr.a.depth_tiles;
         if (fr.n_items >= kMaxItemsPerFrame) return fail(SUPRA_ERR_TOO_LARGE, "batch: frame %u too large", f);
         fr.frame = f;

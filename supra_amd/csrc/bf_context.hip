@@ -79,18 +79,21 @@ void build_dt_tables(supra_bf_ctx* ctx, double dt, double c) {
             t.tx_idx = s.tx[k].tx_scanline_idx;
             t.t0 = static_cast<float>(s.tx[k].initial_delay * factor_time);
             // Same single-precision operations as the kernels' aperture test.
+            // Such an element is in no aperture where its position or the
+            // scanline's is NaN: no depth is far then.
             float thr = 0.0f;
+            const auto raise = [&](float v) { thr = std::isnan(v) ? INFINITY : std::max(thr, v); };
             if (ctx->is3d) {
                 for (uint32_t ex = t.first_x; ex < t.last_x; ex++)
                     for (uint32_t ey = t.first_y; ey < t.last_y; ey++) {
                         const uint32_t e = ex + ey * ctx->el_layout[0];
                         if (!connected(e)) continue;
                         const float dx = ctx->h_ex[e] - o.x, dz = ctx->h_ey[e] - o.z;
-                        thr = std::max(thr, dx * dx + dz * dz);
+                        raise(dx * dx + dz * dz);
                     }
             } else {
                 for (uint32_t e = t.first_x; e < t.last_x; e++)
-                    if (connected(e)) thr = std::max(thr, std::fabs(ctx->h_ex[e] - o.x));
+                    if (connected(e)) raise(std::fabs(ctx->h_ex[e] - o.x));
                 thr = std::max(thr, o.max_ed_x);
             }
             t.far_thr = thr;
@@ -257,8 +260,10 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
         int32_t sel, mask;
         float w[4];
         scanline_selection(ctx->scan_mm[i], &sel, &mask, w);
+        for (double v : ctx->scan_mm[i].direction) ctx->nan_lines = ctx->nan_lines || std::isnan(v);
         for (int k = 0; k < 4; k++) {
             const supra_tx_params& t = ctx->scan_mm[i].tx[k];
+            ctx->nan_lines = ctx->nan_lines || std::isnan(t.initial_delay);
             bool bad = ctx->is3d ? (t.last_active_element[0] > ctx->el_layout[0] ||
                                     t.last_active_element[1] > ctx->el_layout[1])
                                  : (t.last_active_element[0] > ctx->n_el);
@@ -391,17 +396,18 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
     a.c = static_cast<float>(speed_of_sound_mm_per_s);
     a.offset = static_cast<float>(additional_offset);
     a.far_ok = ctx->far_ok ? 1 : 0;
-    a.grid_ok = ctx->grid_ok && ctx->max_rows <= 32 ? 1 : 0;
+    a.nan_lines = ctx->nan_lines ? 1 : 0;
+    a.grid_ok = ctx->grid_ok && ctx->max_rows <= 32 && !ctx->nan_lines ? 1 : 0;
     context_window_lut(ctx, window_type, window_parameter, a.lut);
 
     hipError_t e;
     if (sample_beamformer == SUPRA_BF_COHERENCE_FACTOR && !ctx->is3d)
-        e = launch_coherence_2d(a, rf_dtype, out_dtype, interpolate_transmits != 0, ctx->d_e2c != nullptr, hs);
+        e = launch_coherence_2d(a, rf_dtype, out_dtype, interpolate_transmits != 0, ctx->d_e2c || ctx->nan_lines, hs);
     else if (sample_beamformer == SUPRA_BF_DELAY_AND_STD_DEV || sample_beamformer == SUPRA_BF_COHERENCE_FACTOR)
         e = launch_das_variant(a, rf_dtype, out_dtype, ctx->is3d, sample_beamformer, interpolate_transmits != 0, hs);
     else
         e = launch_das(a, rf_dtype, out_dtype, ctx->is3d, sample_beamformer == SUPRA_BF_TEST_SIGNAL,
-                       interpolate_transmits != 0, ctx->d_e2c != nullptr, hs);
+                       interpolate_transmits != 0, ctx->d_e2c || ctx->nan_lines, hs);
     if (e != hipSuccess) return hip_fail(e, "das: launch");
     tables_used_on(ctx, hs);
     return SUPRA_OK;
@@ -491,6 +497,7 @@ DasArgs rawdelay_args(const supra_bf_ctx* ctx, const void* rf, uint32_t num_tx, 
     a.dt = static_cast<float>(dt);
     a.c = static_cast<float>(c);
     a.far_ok = 0;
+    a.nan_lines = ctx->nan_lines ? 1 : 0;
     build_window_lut(window_type, window_parameter, a.lut);
     return a;
 }
@@ -829,6 +836,7 @@ int das_forward_c(supra_bf_ctx* ctx, bool noalloc, uint32_t num_frames, const fl
     a.c = 0.0f;
     a.offset = static_cast<float>(additional_offset);
     a.far_ok = ctx->far_ok_mm ? 1 : 0;
+    a.nan_lines = ctx->nan_lines ? 1 : 0;
     a.scan_frame_stride = ctx->n_rx;
     a.depth_frame_stride = ctx->n_depths;
     a.el_frame_stride = ctx->n_el;
@@ -836,7 +844,7 @@ int das_forward_c(supra_bf_ctx* ctx, bool noalloc, uint32_t num_frames, const fl
     a.norm_out = norm_out;
     build_window_lut(window_type, window_parameter, a.lut);
     hipError_t e = launch_das(a, SUPRA_FLOAT32, SUPRA_FLOAT32, false, false, interpolate_transmits != 0,
-                              ctx->d_e2c != nullptr, hs);
+                              ctx->d_e2c || ctx->nan_lines, hs);
     if (e != hipSuccess) return hip_fail(e, "das forward: launch");
     return SUPRA_OK;
 }
@@ -949,6 +957,7 @@ extern "C" int supra_das_adjoint(supra_bf_ctx* ctx, uint32_t num_frames, const f
     a.offset = static_cast<float>(additional_offset);
     a.exclusive = ctx->lines_exclusive ? 1 : 0;
     a.depths_sorted = ctx->far_ok_mm ? 1 : 0;
+    a.nan_lines = ctx->nan_lines ? 1 : 0;
     a.interp_tx = interpolate_transmits ? 1 : 0;
     build_window_lut(window_type, window_parameter, a.lut);
     if ((e = launch_das_adjoint(a, num_frames, hs)) != hipSuccess) return hip_fail(e, "das adjoint: launch");

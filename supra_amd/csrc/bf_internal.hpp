@@ -62,8 +62,10 @@ struct DasArgs {
     float F, dt, c;             // fNumber, 1/fs, speed of sound [mm/s] as floats
     float offset;               // (float) additionalOffset
     int32_t max_aperture;       // unused (0)
-    int32_t grid_ok;            // 3D: element (ix, iy) is at (X[ix], Z[iy]), apertures of at most 32 rows
+    int32_t grid_ok;            // 3D: element (ix, iy) is at (X[ix], Z[iy]), apertures of at most 32 rows, no nan_lines
     int32_t far_ok;             // depth table is non-negative and non-decreasing
+    int32_t nan_lines;          // some transmit's delay or scanline's direction is NaN (nan_delays()); the
+                                // delay-and-sum kernels look at it in their MAP form
     // Per-frame geometry (one speed of sound per frame, 2D): strides between
     // the frames' tables (0: all frames share one table) and the per-frame c
     // as a float (nullptr: every frame uses c).
@@ -114,6 +116,7 @@ struct AdjointArgs {
     float F, dt, offset;
     int32_t exclusive;              // every written line has exactly one writer
     int32_t depths_sorted;          // non-negative and non-decreasing
+    int32_t nan_lines;              // as DasArgs
     int32_t interp_tx;
     float lut[kWindowEntries];
 };

@@ -132,7 +132,8 @@ __global__ __launch_bounds__(kTableThreads) void frame_tables_kernel(const Frame
         for (uint32_t e = t.first_x + part; e < t.last_x; e += kThrParts) {
             if (a.e2c && a.e2c[e] < 0) continue;
             const float v = fabsf(static_cast<float>(a.ex_mm[e] * factor) - o.x);
-            thr = (thr < v) ? v : thr;
+            // (a NaN position: no depth is far)
+            thr = (thr < v) ? v : (v != v ? INFINITY : thr);
         }
     }
     for (uint32_t m = 1; m < kThrParts; m <<= 1) {
@@ -245,7 +246,8 @@ __device__ inline void put_sample(__amdgpu_buffer_rsrc_t line, float* out, int32
     else if (v != 0.0f && u < n_s) atomicAdd(&out[u], v);
 }
 
-template <bool GRAD, bool DC, bool EXCLUSIVE>
+// NANS: the geometry has scanlines whose delays are NaN (nan_lines).
+template <bool GRAD, bool DC, bool EXCLUSIVE, bool NANS>
 __global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(const AdjointArgs a) {
     __shared__ float s_lut[kWindowEntries];
     __shared__ __align__(8) float s_rings[GRAD ? kAdjointWaves * kAdjointElements * kRingWords : 1];
@@ -322,6 +324,7 @@ __global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(co
         const float inv_med = 1.0f / med;
         const int32_t n_s = static_cast<int32_t>(a.n_s);
         const uint32_t last_bits = last_sample_bits(a.n_s);
+        const uint64_t nan = NANS && nan_delays<float, false>(1, sc, tx.t0, a.n_s) ? ~0ull : 0ull;   // (uniform)
         float w_far[kAdjointElements];
         bool empty[kAdjointElements];   // nothing was added to the ring yet
 #pragma unroll
@@ -393,7 +396,7 @@ __global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(co
                 geo[n] = sqrt_rn(ee * ee + py2) + d;
                 float tau = tx.t0 + geo[n];
                 tau = tau + a.offset;
-                act[n] = has_beta & ballot(fabsf(dx[n]) <= aDT) & ballot(__float_as_uint(tau) <= last_bits);
+                act[n] = has_beta & ballot(fabsf(dx[n]) <= aDT) & (ballot(__float_as_uint(tau) <= last_bits) | nan);
                 const int32_t i = static_cast<int32_t>(tau);   // (a delay in the RF is not negative: its floor)
                 idx[n] = i;
                 fr[n] = __builtin_amdgcn_fractf(tau);
@@ -559,13 +562,18 @@ uint32_t das_adjoint_groups(uint32_t aperture) {
 }
 uint32_t das_adjoint_waves() { return kAdjointWaves; }
 
+template <bool NANS>
+static auto adjoint_kernel(const AdjointArgs& a) {
+    if (!a.grad_rf) return das2d_adjoint_kernel<false, true, true, NANS>;
+    if (a.dc_part) return a.exclusive ? das2d_adjoint_kernel<true, true, true, NANS> : das2d_adjoint_kernel<true, true, false, NANS>;
+    return a.exclusive ? das2d_adjoint_kernel<true, false, true, NANS> : das2d_adjoint_kernel<true, false, false, NANS>;
+}
+
 hipError_t launch_das_adjoint(const AdjointArgs& a, uint32_t frames, hipStream_t stream) {
     const uint64_t blocks = static_cast<uint64_t>(frames) * a.n_rx * a.n_slots * a.egroups;
     dim3 grid(static_cast<uint32_t>(blocks)), block(kAdjointWaves * kWave);
     if (!a.grad_rf && !a.dc_part) return hipSuccess;
-    auto kernel = das2d_adjoint_kernel<false, true, true>;
-    if (a.grad_rf && a.dc_part) kernel = a.exclusive ? das2d_adjoint_kernel<true, true, true> : das2d_adjoint_kernel<true, true, false>;
-    else if (a.grad_rf) kernel = a.exclusive ? das2d_adjoint_kernel<true, false, true> : das2d_adjoint_kernel<true, false, false>;
+    const auto kernel = a.nan_lines ? adjoint_kernel<true>(a) : adjoint_kernel<false>(a);
     hipLaunchKernelGGL(kernel, grid, block, 0, stream, a);
     return hipGetLastError();
 }

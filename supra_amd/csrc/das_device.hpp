@@ -54,7 +54,8 @@ __device__ inline uint32_t last_sample_bits(uint32_t n_s) {
 // arguments at each of four exponents) on gfx950 it never differed.  Seven
 // issue slots against ten for v_sqrt_f32 and the two-sided neighbour check
 // that LLVM emits for sqrtf.  An infinite x (coordinates beyond 1e19 samples)
-// gives NaN, which every range test below treats as out of range.
+// gives NaN, which every range test below treats as out of range (delays that
+// are NaN because the geometry holds one: nan_delays()).
 __device__ inline float sqrt_rn(float x) {
     const float y = fminf(__builtin_amdgcn_rsqf(x), 0x1p60f);   // finite for x == 0
     const float g = x * y;
@@ -159,7 +160,7 @@ __device__ inline void gather(__amdgpu_buffer_rsrc_t rf, uint32_t off, uint32_t 
         // finite, so (1 - 0) v0 + 0 v1 is v0 exactly and needs no separate
         // case.  2D (int32 floor): 0 <= tau <= N-1.  3D (floor saturated at
         // 0, so a negative tau interpolates from sample 0): tau <= N-1, or
-        // tau == 0 when N == 1.  A NaN delay is out of range.
+        // tau == 0 when N == 1.  A NaN delay is out of range here.
         const float v0 = load_rf<RFT>(rf, off + ui);
         const float v1 = load_rf<RFT>(rf, off + ui + 1u);
         const float last = static_cast<float>(n_s - 1u);
@@ -177,6 +178,21 @@ __device__ inline void gather(__amdgpu_buffer_rsrc_t rf, uint32_t off, uint32_t 
     const float val = edge ? v0 : ((1.0f - f) * v0 + f * v1);
     const float contrib = w * val;
     sample = (inr | edge) ? sample + contrib : sample;
+}
+
+// (uniform) A NaN in the transmit's delay or the scanline's direction makes
+// every delay of its pixels NaN.  The reference's conversion takes such a delay
+// for sample 0 with a NaN fraction, which is in range (for N > 1; int16 RF in 2D
+// is tested on the delay itself): every element of the aperture adds NaN and the
+// pixel saturates.  The range tests leave NaN out, since it is also the root of
+// an infinite square, whose delay is out of range; so the sum of the weights
+// starts at NaN there, which gives the same pixel.  The host looks for such
+// scanlines once (nan_lines).
+template <typename RFT, bool IS3D>
+__device__ inline bool nan_delays(int32_t nan_lines, const ScanView& sc, float t0, uint32_t n_s) {
+    if (!IS3D && std::is_same_v<RFT, int16_t>) return false;
+    return nan_lines != 0 && n_s > 1u &&
+           (t0 != t0 || sc.dir_x() != sc.dir_x() || sc.dir_y() != sc.dir_y() || (IS3D && sc.dir_z() != sc.dir_z()));
 }
 
 }  // namespace

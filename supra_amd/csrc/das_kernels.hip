@@ -397,6 +397,7 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
                                __builtin_amdgcn_ballot_w64(t.valid && !(hi < static_cast<float>(a.n_s - 1u) &&
                                                                         p.py2 >= 1e-20f)) == 0;
             Sums2D<KIND> sums;
+            if (MAP && nan_delays<RFT, false>(a.nan_lines, sc, tx.t0, a.n_s)) sums.wsum = NAN;
             const int first = tx.first_x, last = tx.last_x;
             for (int base = first; base < last; base += kChunk2D) {
                 const int cnt = min(kChunk2D, last - base);
@@ -405,7 +406,7 @@ __device__ inline void das2d_tile(const DasArgs& a, const float* lut, const Tile
                     const int e = base + j;
                     uint32_t ch;
                     if (MAP) {
-                        const int32_t m = a.e2c[e];
+                        const int32_t m = a.e2c ? a.e2c[e] : static_cast<int32_t>(static_cast<uint32_t>(e) % a.n_ch);
                         ch = (m < 0) ? kNotConnected : static_cast<uint32_t>(m);
                     } else {
                         ch = static_cast<uint32_t>(e) % a.n_ch;
@@ -592,6 +593,7 @@ __global__ __launch_bounds__(kThreads) void das2d_frames_kernel(const DasArgs a)
     const int k = sc.sel();
     if (k >= 0) {                                    // uniform
         const TxDT tx = sc.tx(k);
+        if (MAP && nan_delays<RFT, false>(a.nan_lines, sc, tx.t0, a.n_s)) wsum = NAN;
         const uint64_t tx_off = static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
         __amdgpu_buffer_rsrc_t rs[FB];
 #pragma unroll
@@ -609,7 +611,7 @@ __global__ __launch_bounds__(kThreads) void das2d_frames_kernel(const DasArgs a)
                 const int e = base + j;
                 uint32_t ch;
                 if (MAP) {
-                    const int32_t m = a.e2c[e];
+                    const int32_t m = a.e2c ? a.e2c[e] : static_cast<int32_t>(static_cast<uint32_t>(e) % a.n_ch);
                     ch = (m < 0) ? kNotConnected : static_cast<uint32_t>(m);
                 } else {
                     ch = static_cast<uint32_t>(e) % a.n_ch;
@@ -868,7 +870,7 @@ __global__ __launch_bounds__(kThreads) void das3d_kernel(const DasArgs a) {
             const RFT* rf_tx = rf_frame + static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
             const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
             const bool far = a.far_ok && aDT0 >= tx.far_thr && sq0 >= sc.max_ed_x() && sq0 >= sc.max_ed_y();
-            float sample = 0.0f, wsum = 0.0f;
+            float sample = 0.0f, wsum = MAP && nan_delays<RFT, true>(a.nan_lines, sc, tx.t0, a.n_s) ? NAN : 0.0f;
             int nadd = 0;
             const int ny = (tx.last_y > tx.first_y) ? tx.last_y - tx.first_y : 0;
             const int nx = (tx.last_x > tx.first_x) ? tx.last_x - tx.first_x : 0;
@@ -884,7 +886,7 @@ __global__ __launch_bounds__(kThreads) void das3d_kernel(const DasArgs a) {
                     const uint32_t e = exi + eyi * a.layout_x;
                     uint32_t ch;
                     if (MAP) {
-                        const int32_t m = a.e2c[e];
+                        const int32_t m = a.e2c ? a.e2c[e] : static_cast<int32_t>(static_cast<uint32_t>(e) % a.n_ch);
                         ch = (m < 0) ? kNotConnected : static_cast<uint32_t>(m);
                     } else {
                         ch = e % a.n_ch;
@@ -1190,6 +1192,7 @@ __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
                            static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
         const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
         const uint32_t last_bits = last_sample_bits(a.n_s);
+        const bool nan = nan_delays<RFT, false>(a.nan_lines, sc, tx.t0, a.n_s);
         const int first = tx.first_x, last = tx.last_x;
         // pass 1: aperture weight sum and count
         float wsum = 0.0f;
@@ -1242,7 +1245,7 @@ __global__ __launch_bounds__(kThreads) void rawdelay2d_kernel(const DasArgs a) {
 #pragma unroll
                     for (int u = 0; u < kBatchDelay; u++) {
                         const float val = g[u].edge ? g[u].v0 : ((1.0f - g[u].f) * g[u].v0 + g[u].f * g[u].v1);
-                        const float sample = 0.0f + (g[u].add ? g[u].w * val : 0.0f);
+                        const float sample = 0.0f + (g[u].add || (nan && g[u].member) ? g[u].w * val : 0.0f);
                         if (t.valid && j0 + u < cnt)
                             row[static_cast<uint64_t>(j0 + u) * a.n_depths] = clamp_cast<OutT>(sample * scale);
                     }
@@ -1355,6 +1358,7 @@ __global__ __launch_bounds__(kThreads) void rawdelay3d_kernel(const DasArgs a) {
                     const float ax = s_xe[j] - px, az = s_ze[j] - pz;
                     const float tau = tx.t0 + (sqrt_rn((ax * ax + az * az) + py2) + d);
                     gather<RFT, true>(rsrc, off, a.n_s, tau, w, sample);
+                    if (nan_delays<RFT, true>(a.nan_lines, sc, tx.t0, a.n_s)) sample = NAN;
                 }
             }
             if (t.valid) out[static_cast<uint64_t>(base + j) * a.n_depths + t.r] = clamp_cast<OutT>(sample * scale);

@@ -114,7 +114,7 @@ __global__ __launch_bounds__(kThreads) void das2d_stddev_kernel(const DasArgs a)
         const TxDT tx = sc.tx(k);
         const RFT* rf_tx = rf_frame + static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
         const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
-        float sample = 0.0f, wsum = 0.0f;
+        float sample = 0.0f, wsum = nan_delays<RFT, false>(a.nan_lines, sc, tx.t0, a.n_s) ? NAN : 0.0f;
         int nadd = 0;
         for (int pass = 0; pass < 2; pass++) {
             Second<SUPRA_BF_DELAY_AND_STD_DEV> acc;
@@ -181,7 +181,7 @@ __global__ __launch_bounds__(kThreads) void das3d_variant_kernel(const DasArgs a
         const TxDT tx = sc.tx(k);
         const RFT* rf_tx = rf_frame + static_cast<uint64_t>(tx.tx_idx) * a.n_ch * a.n_s;
         const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, a.n_ch * a.n_s * sizeof(RFT));
-        float sample = 0.0f, wsum = 0.0f;
+        float sample = 0.0f, wsum = nan_delays<RFT, true>(a.nan_lines, sc, tx.t0, a.n_s) ? NAN : 0.0f;
         int nadd = 0;
         for (int pass = 0; pass < 2; pass++) {
             Second<KIND> acc;

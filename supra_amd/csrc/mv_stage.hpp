@@ -118,6 +118,7 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
     const RFT* rf_tx = static_cast<const RFT*>(g.rf) + static_cast<uint64_t>(tx.tx_idx) * g.n_ch * g.n_s;
     const __amdgpu_buffer_rsrc_t rsrc = rf_resource(rf_tx, g.n_ch * g.n_s * sizeof(RFT));
     const uint32_t last_bits = last_sample_bits(g.n_s);
+    const bool nan = nan_delays<RFT, false>(g.nan_lines, sc, tx.t0, g.n_s);
     for (int h0 = 0; h0 < H; h0 += 32) {
         const int h = h0 + hl;
         if (h >= H) continue;
@@ -142,7 +143,7 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
                 f[u] = __builtin_amdgcn_fractf(tau);
                 v0[u] = load_rf<RFT>(rsrc, off + ui);
                 v1[u] = load_rf<RFT>(rsrc, off + ui + 1u);
-                add[u] = (fabsf(dx) <= aDT) & (__float_as_uint(tau) <= last_bits);
+                add[u] = (fabsf(dx) <= aDT) & ((__float_as_uint(tau) <= last_bits) | nan);
                 edge[u] = !std::is_same_v<RFT, int16_t> && __float_as_uint(tau) == last_bits;
             }
 #pragma unroll
