@@ -281,7 +281,8 @@ __global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(co
     const uint32_t first = tx.first_x + (eg * kAdjointWaves + wave) * kAdjointElements;
 
     // The wave's elements.  One that is past the aperture or not connected has
-    // an infinite distance, so that no lane takes it, and no lines.
+    // a NaN distance, so that no lane takes it (an F-number so small that the
+    // aperture is infinite would take an infinite one), and no lines.
     float xe[kAdjointElements], dx[kAdjointElements], dc[kAdjointElements];
     int32_t base[kAdjointElements];   // samples below it are final and in out[]; the ring holds the next kRing - 1
     size_t line[kAdjointElements];
@@ -301,7 +302,7 @@ __global__ __launch_bounds__(kAdjointWaves * kWave) void das2d_adjoint_kernel(co
             ch = on[n] ? static_cast<uint32_t>(m) : 0u;
         }
         xe[n] = on[n] ? a.ex[static_cast<size_t>(f) * a.el_frame_stride + e] : 0.0f;
-        dx[n] = on[n] ? xe[n] - x : INFINITY;
+        dx[n] = on[n] ? xe[n] - x : NAN;
         near = fminf(near, fabsf(dx[n]));
         any = any || on[n];
         line[n] = a.rf_frame_stride * f + (static_cast<size_t>(tx.tx_idx) * a.n_ch + ch) * a.n_s;

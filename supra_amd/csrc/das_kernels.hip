@@ -971,7 +971,7 @@ __device__ inline void grid3d(__amdgpu_buffer_rsrc_t rf, const DasArgs& a, const
                 bool any = FAR;
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    // (a row past the aperture is staged with an infinite distance)
+                    // (a row past the aperture is staged with a NaN distance)
                     member[u] = FAR || r2s[u] <= p.aDT;
                     any |= member[u];
                 }
@@ -1125,7 +1125,7 @@ __global__ __launch_bounds__(kThreads, 4) void das3d_grid_kernel(const DasArgs a
                     const int x = j / kGridY, y = j % kGridY;
                     const uint32_t e = tx.first_x + base + x + (tx.first_y + min(y, ny - 1)) * a.layout_x;
                     const float dx = a.ex[e] - sc.x(), dz = a.ey[e] - sc.z();
-                    s_r2[j] = y < ny ? dx * dx + dz * dz : INFINITY;
+                    s_r2[j] = y < ny ? dx * dx + dz * dz : NAN;
                     s_w[j] = y < ny ? s_w2[window_index(dx * invx_far) * kWindowEntries + window_index(dz * invz_far)] : 0.0f;
                     if (y == 0) s_dx[x] = dx;
                 }
