@@ -21,6 +21,7 @@ CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libsupra_bf.so"
 SHIM_TEST = PKG / "shim_test"
+MV_PLANS_TEST = PKG / "mv_plans_test"
 TORCH_LIB = PKG / "libsupra_torch.so"
 
 ARCH = os.environ.get("SUPRA_OFFLOAD_ARCH", "gfx950")
@@ -72,9 +73,13 @@ def build(verbose: bool = False) -> Path:
     tmp = LIB.with_suffix(".so.tmp")
     _run([hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-pthread", "-o", str(tmp), *map(str, objs)], verbose)
     os.replace(tmp, LIB)
-    # the C++ engine shim's test program (include/supra_bf.hpp), next to the library
+    # the C++ test programs (the engine shim of include/supra_bf.hpp, the plans of
+    # the minimum variance), next to the library
     _run([hipcc, "-O2", "-std=c++17", f"-I{ROOT / 'include'}", str(ROOT / "tests" / "cpp" / "shim_test.cpp"),
           f"-L{PKG}", "-lsupra_bf", "-Wl,-rpath,$ORIGIN", "-o", str(SHIM_TEST)], verbose)
+    _run([hipcc, "-O2", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", f"-I{ROOT / 'include'}", f"-I{CSRC}",
+          str(ROOT / "tests" / "cpp" / "mv_plans_test.cpp"), f"-L{PKG}", "-lsupra_bf", "-Wl,-rpath,$ORIGIN", "-o",
+          str(MV_PLANS_TEST)], verbose)
     build_torch_op(hipcc, verbose)
     return LIB
 

@@ -300,10 +300,9 @@ int build_mv_queue(supra_batch* b, uint32_t qi, size_t budget) {
     return st;
 }
 
-// LDS budgets of the MV queues: the whole LDS of a CU (one workgroup) or half
-// of it (two), less room for the kernel's static LDS (16 bytes: the claimed
-// item's broadcast slot).
-constexpr size_t kMvStaticLdsReserve = 64;
+// LDS budgets of the MV queues: the whole LDS of a CU (one workgroup) or a
+// share of it, less room for the kernel's static LDS (the claimed item's
+// broadcast slot).
 size_t mv_full_budget(const supra_batch* b) {
     int dev_lds = 65536;
     (void)hipDeviceGetAttribute(&dev_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, b->device);
@@ -470,9 +469,9 @@ int autotune(supra_batch* b) {
             continue;
         }
         struct Cand { size_t budget; uint32_t wg; };
-        // one to four workgroups per CU, each planning its depth tile for
-        // its share of the LDS (a larger tile re-reads less of the temporal
-        // halo; more workgroups hide more latency)
+        // one to four workgroups per CU, as many as fit (more workgroups hide
+        // more latency); the refined kernel plans its depth tile for its share
+        // of the LDS (a larger tile re-reads less of the temporal halo)
         const Cand cands[] = {{mv_full_budget(b), 1}, {mv_share_budget(b, 2), 2}, {mv_share_budget(b, 3), 3},
                               {mv_share_budget(b, 4), 4}};
         float best = 1e30f;

@@ -771,7 +771,7 @@ __global__ __launch_bounds__(Cfg<LMAX>::kThreads) void mv_block_batch_kernel(con
     }
 }
 
-size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
+size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile, bool with_delay) {
     const uint32_t H = tile + 2 * a.T, blocks = lmax / 16;
     a.tile = tile;
     size_t off = (static_cast<size_t>(H) * a.rs * 4 + 15) & ~static_cast<size_t>(15);
@@ -787,7 +787,7 @@ size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
     // the pre-delay tables are only read before the matrices are written
     const size_t mats = static_cast<size_t>(tile) * (blocks * 160 + blocks * (blocks - 1) / 2 * 256) * 4;
     a.off_fused = static_cast<uint32_t>(off);
-    const size_t fused = a.g.rf ? delay_table_floats(a.n_ch, H) * 4 : 0;
+    const size_t fused = with_delay ? delay_table_floats(a.n_ch, H) * 4 : 0;
     return off + std::max(mats, fused);
 }
 
@@ -795,12 +795,18 @@ size_t plan_lds(MvArgs& a, uint32_t lmax, uint32_t tile) {
 
 uint32_t mv_block_lmax(uint32_t L) { return L <= 16 ? 16 : (L <= 32 ? 32 : 64); }
 
-bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds) {
+bool mv_block_plan(MvArgs& a, size_t full, size_t budget, size_t* lds) {
     const uint32_t lmax = mv_block_lmax(a.L), w = 2 * a.T + 1;
     // zero padding: the last step and the unused rows read past the aperture
     a.rs = a.n_ch + lmax + 4;
-    // Of the tiles that fit, the one with the least modelled time per output:
-    // subs (w - 1) + tile covariance evaluations on the busiest wave (9 matrix
+    // Of the tiles that fit into all of the LDS, the one with the least modelled
+    // time per output.  (Not of those that fit into the budget: the order of a
+    // window's sum and the way that a tile is solved depend on the tile, so a
+    // batch that plans for a share of the LDS would give other bits than the
+    // single call, and smaller tiles do not pay: 6 of the uneven stream's
+    // acquisitions with L = 64 take 31.8 ms with this one, 50 to 101 ms with what
+    // fits two to four times.  For the same reason the pre-delay's tables count
+    // in calls that do without.)  The time: subs (w - 1) + tile covariance evaluations on the busiest wave (9 matrix
     // instructions of 64 cycles with 32 rows, up to 51 with 64, fewer where the
     // aperture is small; with 16 rows the waves share the outputs) and one
     // round of 4 systems per wave.
@@ -810,7 +816,7 @@ bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds) {
     double best = 0;
     uint32_t pick = 0;
     for (uint32_t tile = 1; tile <= 4 * waves; tile++) {
-        if (plan_lds(a, lmax, tile) > budget) break;
+        if (plan_lds(a, lmax, tile, true) > full) break;
         const uint32_t per_wave = lmax == 16 ? (tile + waves - 1) / waves : tile;
         const uint32_t subs = (per_wave + w - 1) / w;
         const double cost = ((subs * (w - 1) + per_wave) * eval + solve) / tile;
@@ -824,9 +830,9 @@ bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds) {
         pick = a.n_d;
         a.sub = std::min(a.sub, pick);
     }
-    *lds = plan_lds(a, lmax, pick);
+    *lds = plan_lds(a, lmax, pick, a.g.rf != nullptr);
     a.n_tiles = (a.n_d + pick - 1) / pick;
-    return true;
+    return *lds <= budget;
 }
 
 template <typename InT, bool FUSED>

@@ -670,7 +670,8 @@ int mv_prepare(MvArgs& a, uint32_t num_scanlines, uint32_t num_channels, uint32_
     a.means = compute_means ? 1 : 0;
     const size_t budget = lds_budget ? std::min(lds_budget, static_cast<size_t>(max_lds_per_block()))
                                      : static_cast<size_t>(max_lds_per_block());
-    if (!pcg && mv_well_loaded(L, loading_factor) && mv_block_plan(a, budget, lds_out)) {
+    const size_t full = static_cast<size_t>(max_lds_per_block()) - kMvStaticLdsReserve;
+    if (!pcg && mv_well_loaded(L, loading_factor) && mv_block_plan(a, full, budget, lds_out)) {
         a.block = 1;
         if (static_cast<uint64_t>(a.n_tiles) * num_scanlines >= (1ull << 31))
             return fail(SUPRA_ERR_TOO_LARGE, "mv: too many workgroups");

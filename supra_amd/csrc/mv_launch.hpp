@@ -69,10 +69,13 @@ int mv_prepare(MvArgs& a, uint32_t num_scanlines, uint32_t num_channels, uint32_
                uint32_t sub_array_size, uint32_t temporal_smoothing, double sub_array_scaling_power,
                int32_t compute_means, double loading_factor, bool pcg, size_t lds_budget, size_t* lds_out);
 
-// mv_block.hip: rows the kernel is built for (16, 32 or 64), the plan for an
-// LDS budget (false: does not fit), and the launches.
+// mv_block.hip: rows the kernel is built for (16, 32 or 64), the plan (for all
+// of the LDS, `full`; false: it does not fit into `budget`), and the launches.
 uint32_t mv_block_lmax(uint32_t L);
-bool mv_block_plan(MvArgs& a, size_t budget, size_t* lds);
+bool mv_block_plan(MvArgs& a, size_t full, size_t budget, size_t* lds);
+// LDS that a launch leaves to its kernel's static LDS (a batch kernel's
+// broadcast slot, 16 bytes).
+constexpr size_t kMvStaticLdsReserve = 64;
 hipError_t launch_mv_block(const MvArgs& a, int32_t in_dtype, bool fused, size_t lds, hipStream_t stream);
 hipError_t launch_mv_block_batch(const MvBatchArgs& b, uint32_t lmax, int32_t rf_dtype, uint32_t workgroups, size_t lds,
                                  hipStream_t stream);
