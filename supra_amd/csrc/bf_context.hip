@@ -105,21 +105,33 @@ void build_dt_tables(supra_bf_ctx* ctx, double dt, double c) {
 // tables.  The wait is here, where they are replaced, and not an event behind
 // every launch: the event costs the host 1.5 us per call and the stream a
 // barrier between two kernels (one 128 x 2080 frame takes 17.4 us per call with
-// it, 14.6 without; another speed of sound uploads its tables anyway).
-static hipError_t wait_for_table_readers(supra_bf_ctx* ctx) {
+// it, 14.6 without).  It is a wait for the streams of those calls, so that other
+// work on the device goes on; the upload's own stream runs in order.  A wait for
+// the device where the streams do not tell: a captured call is replayed on any,
+// a stream that is gone may have left work behind, and past kTableStreams they
+// are not noted.
+static hipError_t wait_for_table_readers(supra_bf_ctx* ctx, hipStream_t upload) {
     if (!ctx->tables_used) return hipSuccess;
-    hipError_t e = hipDeviceSynchronize();
-    if (e != hipSuccess && !ctx->more_table_streams) {
-        // not allowed while another thread captures a graph: the launches'
-        // streams one by one (a stream that is gone has drained)
-        (void)hipGetLastError();
-        e = hipSuccess;
-        for (hipStream_t s : ctx->table_streams) {
-            const hipError_t es = hipStreamSynchronize(s);
-            if (es != hipSuccess && es != hipErrorInvalidHandle && es != hipErrorContextIsDestroyed) e = es;
+    bool device = ctx->tables_captured || ctx->more_table_streams;
+    for (size_t i = 0; i < ctx->table_streams.size() && !device; i++) {
+        const hipStream_t s = ctx->table_streams[i];
+        if (s == upload) continue;
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        hipError_t e = s ? hipStreamIsCapturing(s, &status) : hipSuccess;
+        // (a wait would end the capture without success)
+        if (e == hipSuccess && status != hipStreamCaptureStatusNone) return hipErrorStreamCaptureUnsupported;
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        if (e == hipErrorInvalidHandle || e == hipErrorContextIsDestroyed) {
+            (void)hipGetLastError();
+            device = true;
+        } else if (e != hipSuccess) {
+            return e;
         }
     }
-    if (e != hipSuccess) return e;
+    if (device) {
+        const hipError_t e = hipDeviceSynchronize();
+        if (e != hipSuccess) return e;
+    }
     ctx->tables_used = ctx->more_table_streams = false;
     ctx->table_streams.clear();
     return hipSuccess;
@@ -127,10 +139,11 @@ static hipError_t wait_for_table_readers(supra_bf_ctx* ctx) {
 
 int ensure_dt_tables(supra_bf_ctx* ctx, double dt, double c, hipStream_t stream) {
     if (ctx->cached_dt == dt && ctx->cached_c == c) return SUPRA_OK;
-    build_dt_tables(ctx, dt, c);
     hipError_t e;
-    if ((e = wait_for_table_readers(ctx)) != hipSuccess)
+    if ((e = wait_for_table_readers(ctx, stream)) != hipSuccess)
         return hip_fail(e, "geometry upload: wait for earlier kernels");
+    ctx->cached_dt = ctx->cached_c = 0;     // (until every table is there)
+    build_dt_tables(ctx, dt, c);
     if ((e = hipMemcpyAsync(ctx->d_scans, ctx->h_scans.data(), ctx->n_rx * sizeof(ScanlineDT), hipMemcpyHostToDevice,
                             stream)) != hipSuccess)
         return hip_fail(e, "upload scanlines");
@@ -153,9 +166,16 @@ int ensure_dt_tables(supra_bf_ctx* ctx, double dt, double c, hipStream_t stream)
 // Notes a launch that reads the context's dt-space tables.
 void tables_used_on(supra_bf_ctx* ctx, hipStream_t stream) {
     ctx->tables_used = true;
+    if (stream && !ctx->tables_captured) {      // (the null stream cannot be captured)
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(stream, &status) != hipSuccess || status != hipStreamCaptureStatusNone)
+            ctx->tables_captured = true;
+    }
     for (hipStream_t s : ctx->table_streams)
         if (s == stream) return;
-    if (ctx->table_streams.size() < supra_bf_ctx::kTableStreams) ctx->table_streams.push_back(stream);
+    // (hipStreamPerThread is another stream in every thread)
+    if (ctx->table_streams.size() < supra_bf_ctx::kTableStreams && stream != hipStreamPerThread)
+        ctx->table_streams.push_back(stream);
     else ctx->more_table_streams = true;
 }
 

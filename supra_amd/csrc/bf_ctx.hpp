@@ -33,9 +33,10 @@ struct supra_bf_ctx {
     double cached_dt = 0, cached_c = 0;
     // Launches have read d_scans/d_depths/d_ex/d_ey since their upload, on
     // these streams (the first kTableStreams distinct ones): an upload for
-    // another (dt, c) waits for them.
+    // another (dt, c) waits for them.  tables_captured: a launch was captured
+    // (and may be replayed at any time, on any stream).
     static constexpr size_t kTableStreams = 16;
-    bool tables_used = false, more_table_streams = false;
+    bool tables_used = false, more_table_streams = false, tables_captured = false;
     std::vector<hipStream_t> table_streams;
     // Transmits that the selected, resp. all weighted transmits of the
     // scanlines address (largest index + 1).
