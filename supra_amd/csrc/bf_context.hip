@@ -417,6 +417,7 @@ extern "C" int supra_das_run_frames(supra_bf_ctx* ctx, int32_t sample_beamformer
     a.offset = static_cast<float>(additional_offset);
     a.far_ok = ctx->far_ok ? 1 : 0;
     a.nan_lines = ctx->nan_lines ? 1 : 0;
+    a.max_aperture = static_cast<int32_t>(std::min<uint64_t>(static_cast<uint64_t>(ctx->max_aperture) * ctx->max_rows, 1u << 30));
     a.grid_ok = ctx->grid_ok && ctx->max_rows <= 32 && !ctx->nan_lines ? 1 : 0;
     context_window_lut(ctx, window_type, window_parameter, a.lut);
 

@@ -61,7 +61,7 @@ struct DasArgs {
     uint32_t depth_tiles;       // ceil(n_depths / tile)
     float F, dt, c;             // fNumber, 1/fs, speed of sound [mm/s] as floats
     float offset;               // (float) additionalOffset
-    int32_t max_aperture;       // unused (0)
+    int32_t max_aperture;       // 3D: elements of the largest aperture (bounding rows x columns)
     int32_t grid_ok;            // 3D: element (ix, iy) is at (X[ix], Z[iy]), apertures of at most 32 rows, no nan_lines
     int32_t far_ok;             // depth table is non-negative and non-decreasing
     int32_t nan_lines;          // some transmit's delay or scanline's direction is NaN (nan_delays()); the

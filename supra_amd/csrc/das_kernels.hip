@@ -940,7 +940,7 @@ __global__ __launch_bounds__(kThreads) void das3d_kernel(const DasArgs a) {
 // das3d_kernel (VALU 77 % busy, 22 to 28 instructions per element and pixel in
 // the interior).  112 registers leave four waves per SIMD; forcing five spills
 // (6.75 ms), and holding a second batch of gathers per wave was slower too
-// (7.5 ms).
+// (7.5 ms).  Where it pays: grid_pays().
 constexpr int kGridY = 32;      // aperture rows held in registers
 constexpr int kGridX = 32;      // aperture columns staged per LDS pass
 
@@ -1441,6 +1441,35 @@ static void launch_2d(const DasArgs& a, bool interp_tx, bool map, hipStream_t st
     }
 }
 
+// Where das3d_grid_kernel is the faster of the two (both give the same bits).
+// Four of its waves fit on a SIMD against eight, so it counts how the workgroups
+// fill its rounds of four per CU.  All on the card at once: it wins (us, grid /
+// general: 16 x 16 elements, 16 x 16 lines x 500 depths 48 / 70; 32 x 32, 32 x 32 x
+// 256 463 / 512; float RF with one workgroup per line is 5 % slower when they fill
+// the card).  More: with lines of four full depth tiles, which spread evenly over
+// the CUs (32 x 32, 20 x 20 x 1000 412 / 475, 64 x 64 x 1000 3434 / 3740; not where
+// the apertures are small: 12 x 12, 32 x 32 x 1000 157 / 135); two rounds that are
+// both full (28 x 28, 32 x 32 x 400 545 / 648; 24 x 24, 24 x 24 x 768, 1.7 rounds,
+// 393 / 330); many rounds of full tiles, or of the largest apertures (32 x 32,
+// 36 x 36 x 640 2 % faster).  Float RF needs a test per element for the last sample
+// and pays later (16 x 16, 32 x 32 x 1000 11 % slower, 32 x 32 2 % faster).  With an
+// offset no wave is interior: the general kernel (32 x 32, 24 x 24 x 500 688 / 456),
+// but for few waves with small apertures, which wait more than they issue
+// (12 x 12, 8 x 8 x 1000 29 / 33).
+static bool grid_pays(const DasArgs& a, bool float_rf) {
+    constexpr uint64_t kRound = 4 * 256;        // workgroups on 256 CUs
+    const uint64_t lines = static_cast<uint64_t>(a.n_rx) * a.n_frames, wgs = lines * a.depth_tiles;
+    if (a.offset != 0.0f) return lines <= 64 && a.max_aperture <= 15 * 15;
+    if (wgs <= kRound) return !float_rf || a.depth_tiles >= 2 || wgs < kRound;
+    const bool fours = a.depth_tiles % 4 == 0 && a.n_depths >= 0.95 * (static_cast<double>(a.depth_tiles) * kThreads);
+    if (fours && !float_rf) return a.max_aperture >= 15 * 15;
+    if (wgs <= 2 * kRound) return wgs >= 1900 && a.depth_tiles >= 2 && a.max_aperture >= 15 * 15;
+    const uint64_t rounds = (wgs + kRound - 1) / kRound;
+    const bool full = static_cast<double>(lines) * a.n_depths >= 0.85 * static_cast<double>(rounds * kRound * kThreads);
+    if (float_rf) return full && a.max_aperture >= 23 * 23;
+    return full ? a.max_aperture >= 15 * 15 : a.max_aperture >= 29 * 29 && a.depth_tiles >= 2;
+}
+
 template <typename RFT, typename OutT>
 static hipError_t launch_typed(const DasArgs& a, bool is3d, bool testsig, bool interp_tx, bool map,
                                hipStream_t stream) {
@@ -1460,7 +1489,7 @@ static hipError_t launch_typed(const DasArgs& a, bool is3d, bool testsig, bool i
             else hipLaunchKernelGGL((KERNEL<RFT, OutT, false, false, false>), grid, block, 0, stream, a);           \
         }                                                                                                           \
     } while (0)
-    if (is3d && a.grid_ok && !testsig && !map) {
+    if (is3d && a.grid_ok && !testsig && !map && grid_pays(a, std::is_same_v<RFT, float>)) {
         if (interp_tx) hipLaunchKernelGGL((das3d_grid_kernel<RFT, OutT, true>), grid, block, 0, stream, a);
         else hipLaunchKernelGGL((das3d_grid_kernel<RFT, OutT, false>), grid, block, 0, stream, a);
     } else if (is3d) {
