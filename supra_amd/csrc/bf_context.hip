@@ -79,23 +79,23 @@ void build_dt_tables(supra_bf_ctx* ctx, double dt, double c) {
             t.tx_idx = s.tx[k].tx_scanline_idx;
             t.t0 = static_cast<float>(s.tx[k].initial_delay * factor_time);
             // Same single-precision operations as the kernels' aperture test.
-            // Such an element is in no aperture where its position or the
-            // scanline's is NaN: no depth is far then.
             float thr = 0.0f;
-            const auto raise = [&](float v) { thr = std::isnan(v) ? INFINITY : std::max(thr, v); };
             if (ctx->is3d) {
                 for (uint32_t ex = t.first_x; ex < t.last_x; ex++)
                     for (uint32_t ey = t.first_y; ey < t.last_y; ey++) {
                         const uint32_t e = ex + ey * ctx->el_layout[0];
                         if (!connected(e)) continue;
                         const float dx = ctx->h_ex[e] - o.x, dz = ctx->h_ey[e] - o.z;
-                        raise(dx * dx + dz * dz);
+                        thr = std::max(thr, dx * dx + dz * dz);
                     }
             } else {
                 for (uint32_t e = t.first_x; e < t.last_x; e++)
-                    if (connected(e)) raise(std::fabs(ctx->h_ex[e] - o.x));
+                    if (connected(e)) thr = std::max(thr, std::fabs(ctx->h_ex[e] - o.x));
                 thr = std::max(thr, o.max_ed_x);
             }
+            // An element is in no aperture where its position or the scanline's
+            // is NaN: no depth is far then.
+            if (ctx->nan_positions) thr = INFINITY;
             t.far_thr = thr;
         }
     }
@@ -260,6 +260,8 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
     ctx->ey_mm.assign(g->element_y, g->element_y + g->num_elements);
     ctx->geom_c = g->speed_of_sound_mm_per_s;
     ctx->depth_mm = g->depth;
+    for (const auto* p : {&ctx->ex_mm, &ctx->ey_mm})
+        for (float v : *p) ctx->nan_positions = ctx->nan_positions || std::isnan(v);
     ctx->far_ok_mm = true;
     for (uint32_t i = 0; i < ctx->n_depths; i++)
         if (!(ctx->depths_mm[i] >= 0.0f) || (i > 0 && !(ctx->depths_mm[i] >= ctx->depths_mm[i - 1])))
@@ -281,6 +283,7 @@ extern "C" int supra_bf_create(const supra_rx_geometry* g, supra_bf_ctx** out_ct
         float w[4];
         scanline_selection(ctx->scan_mm[i], &sel, &mask, w);
         for (double v : ctx->scan_mm[i].direction) ctx->nan_lines = ctx->nan_lines || std::isnan(v);
+        for (double v : ctx->scan_mm[i].position) ctx->nan_positions = ctx->nan_positions || std::isnan(v);
         for (int k = 0; k < 4; k++) {
             const supra_tx_params& t = ctx->scan_mm[i].tx[k];
             ctx->nan_lines = ctx->nan_lines || std::isnan(t.initial_delay);

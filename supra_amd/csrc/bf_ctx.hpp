@@ -48,6 +48,7 @@ struct supra_bf_ctx {
     bool grid_ok = false;     // 3D: dt-space element (ix, iy) is at (X[ix], Z[iy])
     uint32_t max_rows = 0;    // 3D: largest last_y - first_y over scanlines and transmits
     bool far_ok_mm = false;   // the same for the millimetre depths (any c)
+    bool nan_positions = false;   // some scanline's or element's position is NaN
     bool nan_lines = false;   // some transmit's delay or scanline's direction is NaN
     std::mutex mu;
 
