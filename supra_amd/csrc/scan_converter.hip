@@ -20,8 +20,9 @@
 // The tables live in HBM: per pixel a uint32 sample index (0xffffffff
 // outside the scan) and two (2D) or three (3D) float weights.
 //
-// Conversion (supra_scanconv_run): 2D in tiles of 64 x 16 output pixels from
-// LDS, 3D one to four output pixels per lane, x fastest; each lane reads its
+// Conversion (supra_scanconv_run): 2D direct, in runs of 1024 or in tiles of
+// 64 x 16 output pixels from LDS (form_2d()), 3D one to four output pixels per
+// lane, x fastest; each lane reads its
 // table entries once and converts `num_frames` frames
 // (scanConvert2D :350-381, scanConvert3D :384-428), clampCast to the output
 // type.  Arithmetic is the reference's expression, in float, unfused.
@@ -317,18 +318,11 @@ __global__ __launch_bounds__(256) void scan_convert_kernel(const ConvArgs a) {
     }
 }
 
-// 2D, few frames: one pixel per thread, neighbours from the input, four frames'
-// gathers at once; finding and staging a tile's box (below) pays from
-// kScFewFrames frames on.  The lanes of a wave are neighbouring pixels of a row:
-// where the scanlines are parallel they read one run of samples, and the staged
-// form pays later.
-// us, this form / staged: 764 x 1601 pixels of a linear scan, 1, 4, 8, 12 and 20
-// frames 7.6/11.2, 10.2/14.3, 15.1/21.1, 20.4/24.8 and 30.7/32.1; 1601 x 1387 of
-// a 60 degree sector, 1, 2 and 4 frames 8.8/14.6, 12.3/15.0 and 19.3/18.0 (smaller
-// sectors of 4 frames gain: 732 x 478 pixels 8.2 -> 7.3).
-constexpr uint32_t kScFewFrames = 4, kScFewFramesParallel = 20;
+// 2D, direct: one pixel per thread, neighbours from the input, four frames'
+// gathers at once; nothing to find or stage, so the form for few frames (see
+// form_2d()).
 template <typename InT, typename OutT>
-__global__ __launch_bounds__(256) void scan_convert_few_kernel(const ConvArgs a) {
+__global__ __launch_bounds__(256) void scan_convert_direct_kernel(const ConvArgs a) {
     constexpr uint32_t F = 4;
     const uint64_t i = static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (i >= a.n_pixels) return;
@@ -352,6 +346,100 @@ __global__ __launch_bounds__(256) void scan_convert_few_kernel(const ConvArgs a)
 #pragma unroll
         for (uint32_t f = 0; f < F; f++)
             if (f0 + f < a.num_frames) out[f * a.n_pixels] = clamp_out<OutT>(val[f]);
+    }
+}
+
+// 2D, runs: 4 pixels per thread, consecutive in the output, input staged in LDS.
+// The 1024 consecutive output pixels of a workgroup read a narrow range of input
+// elements where the scanlines are parallel (a few sample rows); the workgroup
+// finds that range once and copies it per frame, converted to float as the direct
+// kernel converts each sample, into one of two LDS windows (one barrier per frame;
+// the next frame's window is loaded into registers meanwhile).  The window holds
+// floats so that neighbouring samples are read at 4-byte aligned LDS addresses.
+// The four neighbours of each pixel are the elements the direct kernel reads, so
+// the results are identical.  A workgroup whose range exceeds the window reads the
+// input directly.
+constexpr uint32_t kScRun = 1024;            // elements per window; two windows per workgroup
+constexpr int kScRunPer = kScRun / 256;      // window elements per thread
+
+template <typename InT, typename OutT>
+__global__ __launch_bounds__(256) void scan_convert_run_kernel(const ConvArgs a) {
+    constexpr int V = 4;
+    __shared__ float win[2][kScRun];
+    __shared__ uint64_t red_lo[4], red_hi[4];
+    const uint64_t i0 = (static_cast<uint64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * V;
+    const bool live = i0 < a.n_pixels;   // n_pixels is a multiple of V
+    const uint64_t n = a.n_rx;
+    uint64_t s[V];
+    bool valid[V];
+    float wx[V], wy[V];
+    uint64_t lo = ~0ull, hi = 0;
+    for (int v = 0; v < V; v++) {
+        const uint64_t i = i0 + v;
+        const uint32_t s32 = live ? a.idx[i] : kOutside;
+        s[v] = s32;
+        // the last sample row has no successor: the reference's 3D guard, used in 2D too
+        valid[v] = s32 != kOutside && s[v] + 1 + n < a.in_frame;
+        wx[v] = valid[v] ? a.wx[i] : 0.0f;
+        wy[v] = valid[v] ? a.wy[i] : 0.0f;
+        if (valid[v]) {
+            lo = min(lo, s[v]);
+            hi = max(hi, s[v] + 1 + n);
+        }
+    }
+    // block range [lo, hi] of the elements read
+    for (int o = 32; o > 0; o >>= 1) {
+        lo = min(lo, static_cast<uint64_t>(__shfl_xor(static_cast<long long>(lo), o, 64)));
+        hi = max(hi, static_cast<uint64_t>(__shfl_xor(static_cast<long long>(hi), o, 64)));
+    }
+    const uint32_t wave = threadIdx.x / 64;
+    if (threadIdx.x % 64 == 0) {
+        red_lo[wave] = lo;
+        red_hi[wave] = hi;
+    }
+    __syncthreads();
+    lo = min(min(red_lo[0], red_lo[1]), min(red_lo[2], red_lo[3]));
+    hi = max(max(red_hi[0], red_hi[1]), max(red_hi[2], red_hi[3]));
+    const bool staged = lo <= hi && hi - lo < kScRun;
+    const uint32_t extent = staged ? static_cast<uint32_t>(hi - lo + 1) : 0u;
+
+    const InT* in = static_cast<const InT*>(a.in);
+    OutT* out = static_cast<OutT*>(a.out);
+    float pre[kScRunPer];
+    auto fetch = [&](const InT* src) {
+        for (int j = 0; j < kScRunPer; j++) {
+            const uint32_t k = threadIdx.x + static_cast<uint32_t>(j) * 256u;
+            pre[j] = k < extent ? static_cast<float>(src[lo + k]) : 0.0f;
+        }
+    };
+    if (staged) fetch(in);
+    for (uint32_t f = 0; f < a.num_frames; f++, in += a.in_frame, out += a.n_pixels) {
+        const uint32_t b = f & 1u;
+        if (staged) {
+            for (int j = 0; j < kScRunPer; j++) {
+                const uint32_t k = threadIdx.x + static_cast<uint32_t>(j) * 256u;
+                if (k < extent) win[b][k] = pre[j];
+            }
+            __syncthreads();
+            if (f + 1 < a.num_frames) fetch(in + a.in_frame);
+        }
+        OutPack<OutT, V> o;
+        for (int v = 0; v < V; v++) {
+            float val = 0.0f;
+            if (valid[v]) {
+                if (staged) {
+                    const uint32_t q = static_cast<uint32_t>(s[v] - lo);
+                    val = (1 - wy[v]) * ((1 - wx[v]) * win[b][q] + wx[v] * win[b][q + 1]) +
+                          wy[v] * ((1 - wx[v]) * win[b][q + n] + wx[v] * win[b][q + 1 + n]);
+                } else {
+                    const uint64_t q = s[v];
+                    val = (1 - wy[v]) * ((1 - wx[v]) * in_at(in, q) + wx[v] * in_at(in, q + 1)) +
+                          wy[v] * ((1 - wx[v]) * in_at(in, q + n) + wx[v] * in_at(in, q + 1 + n));
+                }
+            }
+            o.v[v] = clamp_out<OutT>(val);
+        }
+        if (live) *reinterpret_cast<OutPack<OutT, V>*>(out + i0) = o;
     }
 }
 
@@ -550,6 +638,7 @@ struct supra_scanconv {
     int device = 0;
     bool is3d = false;
     bool parallel = true;    // every scanline has the first one's direction
+    double row_step = 1.0;   // sample rows per pixel row
     uint32_t layout[2] = {0, 0};
     uint32_t n_samples = 0;
     uint32_t size[3] = {1, 1, 1};
@@ -614,6 +703,7 @@ extern "C" int supra_scanconv_create(const supra_scanline_rx* scanlines, const u
         for (int d = 0; d < 3; d++) sc->parallel = sc->parallel && scanlines[k].direction[d] == scanlines[0].direction[d];
     sc->n_samples = num_samples;
     sc->resolution = res;
+    sc->row_step = res / sample_distance;
     std::copy(size, size + 3, sc->size);
     sc->bb_min[0] = lo.x, sc->bb_min[1] = lo.y, sc->bb_min[2] = lo.z;
     sc->bb_max[0] = hi.x, sc->bb_max[1] = hi.y, sc->bb_max[2] = hi.z;
@@ -789,6 +879,51 @@ extern "C" int supra_scanconv_mask(const supra_scanconv* sc, uint8_t* mask_devic
     return SUPRA_OK;
 }
 
+namespace {
+
+// The form of a 2D conversion; all three give the same bits.  Times in us,
+// direct / runs / tiles.
+//  * Scanlines that are not parallel: runs would read hundreds of sample rows.
+//    Direct while the box of a tile is not worth finding: 489 x 319 pixels, 12 and
+//    16 frames 7.8/-/7.9 (float 7.5/-/8.6) and 9.6/-/8.2; 801 x 694, 6, 7
+//    and 8 frames 9.9/-/11.6, 11.2/-/11.8 and 12.9/-/11.9; 1306 x 852, 7 frames
+//    13.6/-/16.1; 1601 x 1387, 3 and 4 frames 15.1/-/16.4 and 18.5/-/16.7.
+//  * Parallel scanlines, a large image whose pixels go out in fours and whose
+//    runs fit the window: runs, from the frames on at which their window is
+//    worth loading (the fewer samples it holds the sooner): 1982 x 2080 from 128
+//    lines, 3 and 6 frames 21.1/21.6/27.4 and 30.8/29.1/34.5, 20 frames
+//    82/60/67 (float 164/100/145); 2868 x 1500 from 256 lines, 8 frames 39.9/41.5/39.3
+//    (float 45/43/45), 20 frames 88/78/69 (float 183/125/148).  Tiles write one
+//    byte per pixel and rows that begin at a multiple of four as well, and where a
+//    run holds many samples they read fewer: 2868 x 1500, 32 frames 137/115/98 (but
+//    1976 x 2074 from 128 lines -/84/94; images beyond the last cache: 64 frames
+//    -/241/249).
+//  * Else: direct until the lines of the input that a row of pixels reads leave
+//    the caches: 115 k pixels, 32 frames 7.9/-/13.6; 700 k, 32 frames 28/-/36, 64
+//    frames 52/-/60; 4.1 M, 8 and 20 frames 37/-/39 and 82/-/67.  One thread takes
+//    every frame of a pixel, so an image of a few workgroups takes long: 14 k
+//    pixels, 24 and 32 frames 5.9/-/6.2 and 7.2/-/6.3.
+enum class Form2D { kDirect, kRuns, kTiles };
+Form2D form_2d(const supra_scanconv* sc, bool packed, bool float_in, size_t out_size, uint32_t frames) {
+    const uint64_t pixels = sc->pixels();
+    const auto direct_up_to = [&](uint32_t most) { return frames <= most ? Form2D::kDirect : Form2D::kTiles; };
+    if (!sc->parallel) return direct_up_to(pixels < 200000 ? 12 : (pixels <= 1250000 ? 7 : (float_in ? 4 : 3)));
+    // samples that the 1024 pixels of a run read
+    const double rows = (1023.0 / sc->size[0] + 1.0) * sc->row_step + 2.0;
+    const double samples = rows * sc->layout[0] * sc->layout[1];
+    if (packed && pixels >= 800000 && samples <= kScRun) {
+        const bool short_runs = samples <= 500.0;
+        const uint32_t most = pixels < 1500000 ? (float_in ? 9u : 20u) : (short_runs ? 3u : (float_in ? 4u : 9u));
+        if (frames <= most) return Form2D::kDirect;
+        const bool tiles = !short_runs && !float_in && out_size == 1 && sc->size[0] % 4 == 0 && frames >= 24 &&
+                           pixels * frames <= 225000000;
+        return tiles ? Form2D::kTiles : Form2D::kRuns;
+    }
+    return direct_up_to(pixels < 40000 ? 24 : (pixels < 500000 ? 96 : (pixels < 1500000 ? 36 : (pixels < 3000000 ? 16 : 8))));
+}
+
+}  // namespace
+
 extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanlines_in, int32_t in_dtype,
                                   uint32_t num_frames, void* out, int32_t out_dtype, void* stream) {
     clear_error();
@@ -815,10 +950,11 @@ extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanline
     a.num_frames = num_frames;
     const size_t out_size = out_dtype == SUPRA_FLOAT32 ? 4 : (out_dtype == SUPRA_INT16 ? 2 : 1);
     const bool packed = a.n_pixels % 4 == 0 && reinterpret_cast<uintptr_t>(out) % (4 * out_size) == 0;
-    const bool few = !sc->is3d && num_frames <= (sc->parallel ? kScFewFramesParallel : kScFewFrames);
-    const uint64_t threads = packed && !few ? a.n_pixels / 4 : a.n_pixels;
+    const Form2D form = form_2d(sc, packed, in_dtype == SUPRA_FLOAT32, out_size, num_frames);   // (of 2D)
+    const bool fours = packed && (sc->is3d || form == Form2D::kRuns);     // 4 pixels per thread
+    const uint64_t threads = fours ? a.n_pixels / 4 : a.n_pixels;
     dim3 grid(static_cast<uint32_t>((threads + 255) / 256)), block(256);
-    if (!sc->is3d && !few) {
+    if (!sc->is3d && form == Form2D::kTiles) {
         a.size_x = sc->size[0];
         a.size_y = sc->size[1] * sc->size[2];    // (rows of every plane; a 2D scan fills the first)
         const uint64_t tiles_x = (a.size_x + kScTileX - 1) / kScTileX, rows = (a.size_y + kScTileY - 1) / kScTileY;
@@ -835,10 +971,16 @@ extern "C" int supra_scanconv_run(const supra_scanconv* sc, const void* scanline
     hipStream_t s = static_cast<hipStream_t>(stream);
 #define SUPRA_SC_LAUNCH(IN, OUT)                                                                                       \
     do {                                                                                                              \
-        if (few) hipLaunchKernelGGL((scan_convert_few_kernel<IN, OUT>), grid, block, 0, s, a);                        \
-        else if (!sc->is3d) hipLaunchKernelGGL((scan_convert_tile_kernel<IN, OUT>), grid, block, 0, s, a);            \
-        else if (packed) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 4>), grid, block, 0, s, a);                 \
-        else hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 1>), grid, block, 0, s, a);                             \
+        if (sc->is3d) {                                                                                               \
+            if (fours) hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 4>), grid, block, 0, s, a);                   \
+            else hipLaunchKernelGGL((scan_convert_kernel<IN, OUT, 1>), grid, block, 0, s, a);                         \
+        } else if (form == Form2D::kDirect) {                                                                         \
+            hipLaunchKernelGGL((scan_convert_direct_kernel<IN, OUT>), grid, block, 0, s, a);                          \
+        } else if (form == Form2D::kRuns) {                                                                           \
+            hipLaunchKernelGGL((scan_convert_run_kernel<IN, OUT>), grid, block, 0, s, a);                             \
+        } else {                                                                                                      \
+            hipLaunchKernelGGL((scan_convert_tile_kernel<IN, OUT>), grid, block, 0, s, a);                            \
+        }                                                                                                             \
     } while (0)
 #define SUPRA_SC_OUT(IN)                                                                                              \
     do {                                                                                                              \
