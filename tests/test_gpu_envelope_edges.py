@@ -48,3 +48,14 @@ def test_extreme_samples(device, value):
     img[130:, 40] = value
     img[:, 60] = 0.0
     check(img, 65)
+
+
+@pytest.mark.parametrize("n_taps", [1, 2, 3])
+@pytest.mark.parametrize("shape", [(520, 3, 2), (256, 65, 65)])
+def test_short_filters_of_many_frames(device, n_taps, shape):
+    """Filters that sum every tap keep short tiles without padding rows, also
+    where the other filters take the tall ones."""
+    rng = np.random.default_rng(n_taps)
+    img = (rng.normal(size=shape) * 1000).astype(np.float32)
+    img[1, -1, 0], img[-1, 0, -1] = np.nan, np.inf
+    check(img, n_taps)
