@@ -808,18 +808,30 @@ bool mv_block_plan(MvArgs& a, size_t full, size_t budget, size_t* lds) {
     // fits two to four times.  For the same reason the pre-delay's tables count
     // in calls that do without.)  The time: subs (w - 1) + tile covariance evaluations on the busiest wave (9 matrix
     // instructions of 64 cycles with 32 rows, up to 51 with 64, fewer where the
-    // aperture is small; with 16 rows the waves share the outputs) and one
-    // round of 4 systems per wave.
+    // aperture is small; with 16 rows the waves share the outputs) and rounds of
+    // 4 systems per wave (one, but for tall tiles).
+    // Tall tiles: with 16 rows a wave would sum w - 1 + 4 covariances for 4 outputs, so long
+    // windows take 8, 12 or 16 outputs per wave, as far as the frame still makes
+    // 384 workgroups (128 lines x 1024 depths, 128 channels, L = 4: T = 24 0.90 ms
+    // with 64, 1.82 with 16, 1.08 in mv_kernels.hip; T = 8 474 us with 32, 713
+    // with 16, 631 there; T = 3 410 and 403; 16 lines x 600 depths,
+    // 32 channels, T = 5: 24.4 us with 32 and 23.3 with 16).
     const uint32_t waves = lmax == 32 ? 3 : 4;
     const double eval = lmax == 64 ? 1400.0 : (lmax == 32 ? 580.0 : 320.0);
     const double solve = lmax == 64 ? 23000.0 : (lmax == 32 ? 6000.0 : 2000.0);
+    uint32_t longest = 4 * waves;
+    if (lmax == 16 && a.T >= 4) {
+        const uint32_t tall = a.T < 10 ? 32 : (a.n_ch < 160 && a.T < 20 ? 48 : 64);
+        if (static_cast<uint64_t>(a.n_rx) * ((a.n_d + tall - 1) / tall) >= 384) longest = tall;
+    }
     double best = 0;
     uint32_t pick = 0;
-    for (uint32_t tile = 1; tile <= 4 * waves; tile++) {
+    for (uint32_t tile = 1; tile <= longest; tile++) {
         if (plan_lds(a, lmax, tile, true) > full) break;
         const uint32_t per_wave = lmax == 16 ? (tile + waves - 1) / waves : tile;
         const uint32_t subs = (per_wave + w - 1) / w;
-        const double cost = ((subs * (w - 1) + per_wave) * eval + solve) / tile;
+        const uint32_t rounds = (tile + 4 * waves - 1) / (4 * waves);
+        const double cost = ((subs * (w - 1) + per_wave) * eval + rounds * solve) / tile;
         if (pick && cost >= best) continue;
         best = cost;
         pick = tile;

@@ -99,5 +99,8 @@ int main() {
     failures += run(200, 7, 64, 4, false);
     failures += run(256, 75, 16, 12, true);
     failures += run(128, 40, 8, 0, false);
+    failures += run(48, 4200, 16, 4, false);     // tall tiles
+    failures += run(40, 6200, 8, 18, true);
+    failures += run(170, 8200, 5, 10, false);
     return failures;
 }
