@@ -32,6 +32,17 @@ struct SampleMeta {
 // (it decides the sizes that fit at all; stage_delayed uses 3 n_ch and 2 H).
 __host__ __device__ inline size_t delay_table_floats(size_t n_ch, size_t H) { return kWindowEntries + 4 * n_ch + 6 * H; }
 
+// The thread's index, as a value that the compiler does not know: what is
+// derived from it is computed where it is used, not once before the work loop of
+// a batch kernel.  Kept over the solve it cost mv_batch_kernel with 64 rows 8
+// registers, 258 in all, and with them the second workgroup of a CU (8 frames of
+// 140 x 900, 96 channels, L = 40, weakly loaded: 29.9 ms, 20.6 with 248).
+__device__ inline int opaque_tid() {
+    int t = static_cast<int>(threadIdx.x);
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
 // Fused mode: the pre-delayed samples of scanline s, depths [h_lo, h_lo+H),
 // computed from the RF exactly as the pre-delay kernel writes them
 // (rawdelay2d_kernel in das_kernels.hip; RawDelay.cu:221-312, 404-468):
@@ -48,6 +59,7 @@ __host__ __device__ inline size_t delay_table_floats(size_t n_ch, size_t H) { re
 template <typename RFT, int NT>
 __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t s, uint32_t h_lo, int H,
                                      float* xs, unsigned char* lds) {
+    const int tid = opaque_tid();
     constexpr int kRows = NT / 32, kBatch = 8;
     const DasArgs& g = a.g;
     const int n_ch = static_cast<int>(a.n_ch), rs = static_cast<int>(a.rs);
@@ -59,7 +71,7 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
     int* s_count = reinterpret_cast<int*>(s_off + n_ch);
     float* s_scale = reinterpret_cast<float*>(s_count + hstride);
 
-    const int hl = static_cast<int>(threadIdx.x % 32), cl = static_cast<int>(threadIdx.x / 32);
+    const int hl = tid % 32, cl = tid / 32;
     // the first 32 depths stay in registers over the passes (all of them, mostly)
     const float d_first = g.depths[h_lo + min(hl, H - 1)];
     const auto aperture = [&](float d) { return (((d * g.dt) * g.c) / (2.0f * g.F)) / g.c / g.dt; };
@@ -72,9 +84,9 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
         tx = sc.tx(k);
         cnt = tx.last_x > tx.first_x ? static_cast<int>(tx.last_x - tx.first_x) : 0;
     }
-    for (int i = threadIdx.x; i < kWindowEntries; i += NT) s_lut[i] = lut[i];
-    for (int i = threadIdx.x; i < H; i += NT) s_count[i] = 0;
-    for (int j = threadIdx.x; j < cnt; j += NT) {
+    for (int i = tid; i < kWindowEntries; i += NT) s_lut[i] = lut[i];
+    for (int i = tid; i < H; i += NT) s_count[i] = 0;
+    for (int j = tid; j < cnt; j += NT) {
         const int e = static_cast<int>(tx.first_x) + j;
         const float xe = g.ex[e];
         s_xe[j] = xe;
@@ -98,7 +110,7 @@ __device__ inline void stage_delayed(const MvArgs& a, const float* lut, uint32_t
         if (h < H && n != 0) atomicAdd(&s_count[h], n);
     }
     __syncthreads();
-    for (int h = threadIdx.x; h < H; h += NT) {
+    for (int h = tid; h < H; h += NT) {
         const float* w = xs + h * rs;
         const int nadd = s_count[h];
         float wsum = 0.0f;
