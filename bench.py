@@ -615,11 +615,11 @@ def main() -> int:
     algo_gbs = res["bytes"] / (res["ev_ms"] * 1e-3) / 1e9
     roofline = {"bound": "hbm", "achieved": round(algo_gbs, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": round(algo_gbs / HBM_PEAK_GBS, 4), "traffic": None,
-                "kernel": "das3d_kernel", "avg_launch_ms": round(res["ev_ms"], 4),
+                "kernel": "das3d_grid_kernel", "avg_launch_ms": round(res["ev_ms"], 4),
                 "algorithmic_bytes_per_launch": res["bytes"]}
     traffic_file = ROOT / "profiles" / "traffic.json"
     if traffic_file.exists():
-        t = json.loads(traffic_file.read_text()).get("das3d_kernel/matrix_3d")
+        t = json.loads(traffic_file.read_text()).get("das3d_grid_kernel/matrix_3d")
         if t:
             roofline["traffic"] = t["hbm_bytes_per_launch"]
     extra = {}

@@ -16,15 +16,16 @@
 // launch — reset of the queue counters, the kernels — is captured once in a
 // hipGraph; supra_batch_launch replays it.
 //
-// Footprints differ by an order of magnitude (DAS: 70 VGPRs, 10 KB LDS; MV:
-// 256 VGPRs and up to the whole LDS), so one kernel for all items would run
+// Footprints differ by an order of magnitude (DAS: 74 VGPRs, 10 KB LDS; MV:
+// 248 VGPRs and up to the whole LDS), so one kernel for all items would run
 // the delay-and-sum items at the minimum-variance occupancy; the queues keep
 // each class at its own.
 //
 // The autotuner times each queue alone on the real batch for a few
 // candidates (DAS: 2, 4, 7 or 8 persistent workgroups per CU; MV: one to
-// four workgroups per CU, each with the depth tile that fits its share of
-// the LDS) and keeps the fastest; then it
+// four workgroups per CU, as many as fit; the refined kernel's depth tile
+// then fits its share of the LDS, the block kernel's depends on the frame
+// alone, so that a batch gives the single calls' bits) and keeps the fastest; then it
 // times the whole launch with the queues concurrent and with the queues one
 // after another (shortest time per frame first) and keeps the second unless
 // the first is more than 5 % faster.  Without the autotuner the queues run

@@ -44,7 +44,7 @@
 // What bounds it: 16 frames of 128 lines x 2080 depths x 64 elements take
 // 0.56 ms (0.75 ms with one element per wave, a share handed from lane to
 // lane and an 8 + 4 byte depth entry): the address unit is busy 90 % and the
-// VALU 85 % of that time, HBM (0.45 GB read, 1.07 GB written) a third.  Two
+// VALU 85 % of that time, HBM (0.86 GB read, 1.07 GB written) 43 %.  Two
 // elements per wave share a depth's position, aperture and beta; 3 and 4 cost
 // waves (their rings) and time the same and 7 % more.  Loads and stores
 // complete in one order, so the depth loop keeps a fixed number of stores per

@@ -27,8 +27,8 @@
 // root and the logarithm.  32 frames of 2080 x 128 to uint8: 28.3 us, 48.1 us with
 // every tap and one sum per row.  ROWS is 64 where that leaves at least two
 // workgroups per CU (fewer halo rows staged per output) and taps are left out,
-// else 32.  The fused variant applies the log compression to the float envelope in registers (the
-// same operations as the two-step path with a float intermediate).
+// else 32.  The fused variant applies the log compression to the float envelope in
+// registers (the same operations as the two-step path with a float intermediate).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

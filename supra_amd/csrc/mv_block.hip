@@ -34,7 +34,7 @@
 // and the vector instructions (49 %) of the waves of a SIMD add up.  At L = 64
 // the matrices fill the LDS and one wave per SIMD waits for itself.
 // 128 x 2080 samples, L = 32, T = 5: 0.66 ms against 2.01 ms of
-// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 0.92 ms against
+// mv_kernels.hip; pre-delay + 128 x 1750 samples, L = 64: 0.90 ms against
 // 9.51 ms (in both, windows of few terms take the short way below);
 // relative error of the image against FP64 1.3e-6 against 2.1e-6.
 // Summing the blocks off the first column by differences along the block
